@@ -419,3 +419,35 @@ def test_all_scalars_equal(libs, stream, value):
     pb = gpu_bases(libs, stream, ks)
     for window in (16, 13):
         assert list(run_device(libs, stream, pb, ss, window)) == list(closed_form(ks, ss)), window
+
+
+@pytest.mark.parametrize("n,window,heavy", [
+    # chunks of 4 entries: runs of RUN_MAX - 1 .. RUN_MAX + 2 chunks, off the chunk edges too
+    (900, 12, [60, 64, 67, 68, 69, 72, 75, 1]),
+    # long runs next to each other, one over several tiles of the piece tree
+    (60000, 12, [20000, 3, 9000, 70, 71, 72, 15000, 5, 5, 1200]),
+    # chunks of 32 entries (thread-wide closing pass) and runs of every kind
+    (1 << 19, 16, [100000, 511, 512, 513, 543, 544, 545, 576, 577, 2, 70000, 64, 33, 32, 31]),
+    # every entry in one run, and in two
+    (5000, 13, [5000]),
+    (5000, 13, [2500, 2500]),
+])
+def test_runs_over_chunk_edges(libs, stream, n, window, heavy):
+    """Small scalars 1, 2, ... with the given multiplicities (the rest uniform):
+    bucket v of window 0 is a run of exactly that many sorted entries, plus what
+    the uniform scalars add to it."""
+    ks = random_elements(n, 91)
+    ss = random_elements(n, 92)
+    at = 0
+    for v, count in enumerate(heavy, start=1):
+        ss[at:at + count] = mont_limbs(v)
+        at += count
+    perm = np.random.Generator(np.random.PCG64(93)).permutation(n)
+    ss = np.ascontiguousarray(ss[perm])
+    if at < n:  # the runs' lengths stay exact: the uniform scalars keep out of window 0's small buckets
+        small = [i for i, x in enumerate(array_to_ints(ss)) if 0 < from_mont(x) % (1 << window) <= len(heavy) + 1]
+        for i in small:
+            if from_mont(array_to_ints(ss[i:i + 1])[0]) > len(heavy):
+                ss[i] = mont_limbs(1 << (window - 2))
+    got = run_device(libs, stream, gpu_bases(libs, stream, ks), ss, window)
+    assert list(got) == list(closed_form(ks, ss))

@@ -4,15 +4,22 @@
 // Same formulas as G1XYZZ in g1.hpp (EFD "xyzz", a = 0: madd-2008-s,
 // add-2008-s, dbl-2008-s-1, with the equal and opposite point cases handled
 // exactly), with Fq29's lazy reduction.  Invariant of every point passed
-// between operations: X < 8p, Y < 4p, ZZ < 2p, ZZZ < 2p, limbs normalised; the
+// between operations: X < 8p, Y < 4p, ZZ, ZZZ < 2p, limbs normalised; the
 // identity has every limb zero (ZZ = 0 is the test).  Each formula below keeps
-// it, with these bounds (A B <= 168 for every product):
+// it, with these bounds (A B <= 168 for every product, A B + C D for a pair
+// that shares one reduction):
 //  madd:  U2 = x ZZ (32 x 2), S2 = y ZZZ; P = U2 + 8p - X < 10p,
 //         R = S2 + 4p - Y < 6p; PP = P^2 (100), PPP = P PP, Q = X PP, R^2 (36);
-//         X3 = R^2 + 6p - PPP - 2Q < 8p; Y3 = R (Q + 8p - X3) (60) + 2p - Y PPP < 4p
-//  add:   U1, U2, S1, S2 < 2p; P, R < 4p; X3 < 8p; Q - X3 < 10p (40); Y3 < 4p
+//         X3 = R^2 + 6p - PPP - 2Q < 8p; Y3 = R (Q + 8p - X3) + (4p - Y) PPP (60 + 8) < 2p
+//  add:   U1, U2, S1, S2 < 2p; P, R < 4p; X3 < 8p; Q - X3 < 10p; Y3 = R (Q + 8p - X3) + (4p - S1) PPP
 //  dbl:   U = 2Y < 8p; V = U^2 (64), X^2 (64); M = 3 X^2 < 6p; X3 = M^2 + 4p - 2S < 6p;
-//         Y3 = M (S + 8p - X3) (60) + 2p - W Y < 4p
+//         Y3 = M (S + 8p - X3) + (4p - Y) W (60 + 8) < 2p
+// Y3's two products share a reduction: 90 limb products fewer of about 1 700.
+// Equal operands double through the addition's own steps: with P = 2Y, R = 3 X^2,
+// Q = X P^2 and no P^3 in X3 they are dbl-2008-s-1's, so the case costs one more
+// product in its branch and no second formula in the code.  The instruction
+// cache (64 KB per two CUs) holds a loop over one addition but not the 80 to
+// 313 KB that kernels with a doubling inlined in every addition took.
 // Affine inputs come from HBM in the form of bn254.hpp and are read as
 // x 2^261 below 32p (Fq29::load_mont256); they meet only ZZ and ZZZ in
 // products (32 x 2), and are brought below 2p (Fq29::reduce_2p) where they
@@ -94,9 +101,7 @@ struct G1X29 {
     G1X29 r;
     r.zz = v * zz;
     r.x = m2.sub<4>(s + s);
-    const Fq29 a = m * s.sub<8>(r.x);
-    const Fq29 b = w * y;
-    r.y = a.sub<2>(b);
+    r.y = Fq29::mul_add(m, s.sub<8>(r.x), y.neg<4>(), w);
     r.zzz = w * zzz;
     return r;
   }
@@ -107,52 +112,60 @@ struct G1X29 {
     if (is_identity()) return from_affine(a);
     const Fq29 u2 = a.x * zz;
     const Fq29 s2 = a.y * zzz;
-    const Fq29 p = u2.sub<8>(x);
-    const Fq29 rr = s2.sub<4>(y);
+    Fq29 p = u2.sub<8>(x);
+    Fq29 rr = s2.sub<4>(y);
+    bool same = false;
     if (p.is_zero_modp()) {
-      if (rr.is_zero_modp()) return from_affine(a).dbl();
-      return identity();
+      if (!rr.is_zero_modp()) return identity();
+      doubling_steps(p, rr);
+      same = true;
     }
-    const Fq29 pp = p * p;
-    const Fq29 r2 = rr * rr;
-    const Fq29 ppp = p * pp;
-    const Fq29 q = x * pp;
-    G1X29 r;
-    r.zz = zz * pp;
-    r.x = r2.sub<6>(ppp + q + q);
-    const Fq29 t = rr * q.sub<8>(r.x);
-    const Fq29 b = y * ppp;
-    r.y = t.sub<2>(b);
-    r.zzz = zzz * ppp;
-    return r;
+    return finish(p, rr, x, y, zz, zzz, same);
   }
 
   // add-2008-s: this + o
   ZKP_HD G1X29 add(const G1X29& o) const {
     if (o.is_identity()) return *this;
     if (is_identity()) return o;
-    const Fq29 u1 = x * o.zz;
+    Fq29 u1 = x * o.zz;
     const Fq29 u2 = o.x * zz;
-    const Fq29 s1 = y * o.zzz;
+    Fq29 s1 = y * o.zzz;
     const Fq29 s2 = o.y * zzz;
-    const Fq29 p = u2.sub<2>(u1);
-    const Fq29 rr = s2.sub<2>(s1);
+    Fq29 p = u2.sub<2>(u1);
+    Fq29 rr = s2.sub<2>(s1);
+    Fq29 zz12 = zz * o.zz;
+    Fq29 zzz12 = zzz * o.zzz;
+    bool same = false;
     if (p.is_zero_modp()) {
-      if (rr.is_zero_modp()) return dbl();
-      return identity();
+      if (!rr.is_zero_modp()) return identity();
+      doubling_steps(p, rr);
+      u1 = x;
+      s1 = y;
+      zz12 = zz;
+      zzz12 = zzz;
+      same = true;
     }
+    return finish(p, rr, u1, s1, zz12, zzz12, same);
+  }
+
+ private:
+  // P and R of the addition's last steps when they double this point.
+  ZKP_HD void doubling_steps(Fq29& p, Fq29& rr) const {
+    const Fq29 x2 = x * x;
+    p = (y + y).norm();
+    rr = (x2 + x2 + x2).norm();
+  }
+  // X3, Y3, ZZ3, ZZZ3 from P, R, U1, S1, ZZ1 ZZ2 and ZZZ1 ZZZ2.
+  ZKP_HD static G1X29 finish(const Fq29& p, const Fq29& rr, const Fq29& u1, const Fq29& s1, const Fq29& zz12,
+                             const Fq29& zzz12, bool same) {
     const Fq29 pp = p * p;
     const Fq29 r2 = rr * rr;
-    const Fq29 zz12 = zz * o.zz;
-    const Fq29 zzz12 = zzz * o.zzz;
     const Fq29 ppp = p * pp;
     const Fq29 q = u1 * pp;
     G1X29 r;
     r.zz = zz12 * pp;
-    r.x = r2.sub<6>(ppp + q + q);
-    const Fq29 t = rr * q.sub<8>(r.x);
-    const Fq29 b = s1 * ppp;
-    r.y = t.sub<2>(b);
+    r.x = r2.sub<6>((same ? Fq29::zero() : ppp) + q + q);
+    r.y = Fq29::mul_add(rr, q.sub<8>(r.x), s1.neg<4>(), ppp);
     r.zzz = zzz12 * ppp;
     return r;
   }
@@ -161,98 +174,108 @@ struct G1X29 {
 // ---- quad-cooperative XYZZ arithmetic (device) ----
 //
 // Where few point operations are left (the last levels of the bucket
-// reduction) each one would run on a single lane with its products one after
-// another.  Here the four lanes of a quad (q = lane & 3) hold the same
-// operands and split every phase of independent products among themselves:
-// lane q computes product q and DPP quad permutes hand every product to all
-// four lanes, so add-2008-s takes four product latencies (4, 4, 3, 3
-// products) instead of 14 and dbl-2008-s-1 three (2, 4, 3) instead of 9.
-// Every branch depends only on the shared operands, so the four lanes of a
-// quad always run together.
-template <int SRC>
-__device__ __forceinline__ Fq29 quad29_from(const Fq29& x) {
+// reduction, the accumulation of a small MSM) each one would run on a single
+// lane with its products one after another.  Here a point lies across the four
+// lanes of a quad (q = lane & 3), lane 0 holding X, 1 Y, 2 ZZ and 3 ZZZ, and a
+// phase of independent products is one product on every lane: add-2008-s takes
+// four product latencies instead of 14 (4, 4, 3 and 3 products), madd-2008-s
+// four instead of 10, doubling (equal operands) one more.  DPP quad permutes
+// move factors between the lanes, nine moves each; a first form in which all
+// four lanes held all four coordinates spent twice as many moves and selects
+// and four times the registers.  Every branch depends only on values that the
+// whole quad shares, so its lanes always run together.
+template <int L0, int L1, int L2, int L3>
+__device__ __forceinline__ u32 quad_perm(u32 x) {
+  return (u32)__builtin_amdgcn_mov_dpp((int)x, L0 | L1 << 2 | L2 << 4 | L3 << 6, 0xf, 0xf, false);
+}
+template <int L0, int L1, int L2, int L3>
+__device__ __forceinline__ Fq29 quad_perm(const Fq29& x) {
   Fq29 r;
 #pragma unroll
-  for (int i = 0; i < 9; i++) r.l[i] = (u32)__builtin_amdgcn_mov_dpp((int)x.l[i], SRC * 0x55, 0xf, 0xf, false);
+  for (int i = 0; i < 9; i++) r.l[i] = quad_perm<L0, L1, L2, L3>(x.l[i]);
   return r;
 }
-
-// lane q of the quad takes operand q.  The choice is a bit-select on masks of
-// q's two bits (v_bfi_b32), kept opaque: written as a select over the operands
-// the optimiser folds it into a load of operand[q] from a stack copy.
-__device__ __forceinline__ u32 quad29_bfi(u32 m, u32 x1, u32 x0) {
-  u32 r;
-  asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(m), "v"(x1), "v"(x0));
-  return r;
+template <int L>
+__device__ __forceinline__ Fq29 quad_lane(const Fq29& x) {
+  return quad_perm<L, L, L, L>(x);
 }
-
-__device__ __forceinline__ Fq29 quad29_pick(u32 q, const Fq29& a, const Fq29& b, const Fq29& c, const Fq29& d) {
-  const u32 m1 = 0u - (q & 1u), m2 = 0u - ((q >> 1) & 1u);
+// lane by lane: c ? a : b
+__device__ __forceinline__ Fq29 lane_pick(bool c, const Fq29& a, const Fq29& b) {
   Fq29 r;
 #pragma unroll
-  for (int i = 0; i < 9; i++)
-    r.l[i] = quad29_bfi(m2, quad29_bfi(m1, d.l[i], c.l[i]), quad29_bfi(m1, b.l[i], a.l[i]));
+  for (int i = 0; i < 9; i++) r.l[i] = c ? a.l[i] : b.l[i];
   return r;
 }
 
-// out[k] = l[k] * r[k] for k < N (N <= 4) on every lane of the quad
-template <int N>
-__device__ __forceinline__ void quad29_mul(u32 q, const Fq29 (&l)[N], const Fq29 (&r)[N], Fq29 (&out)[N]) {
-  const Fq29 a = quad29_pick(q, l[0], l[N > 1 ? 1 : 0], l[N > 2 ? 2 : 0], l[N > 3 ? 3 : 0]);
-  const Fq29 b = quad29_pick(q, r[0], r[N > 1 ? 1 : 0], r[N > 2 ? 2 : 0], r[N > 3 ? 3 : 0]);
-  const Fq29 m = a * b;
-  out[0] = quad29_from<0>(m);
-  if (N > 1) out[N > 1 ? 1 : 0] = quad29_from<1>(m);
-  if (N > 2) out[N > 2 ? 2 : 0] = quad29_from<2>(m);
-  if (N > 3) out[N > 3 ? 3 : 0] = quad29_from<3>(m);
-}
+struct Quad29 {
+  Fq29 c;  // this lane's coordinate
 
-__device__ __forceinline__ G1X29 quad29_dbl(const G1X29& a, u32 q) {
-  if (a.is_identity()) return a;
-  const Fq29 u = a.y + a.y;
-  Fq29 p1[2];
-  quad29_mul<2>(q, {u, a.x}, {u, a.x}, p1);  // V, X^2
-  const Fq29 v = p1[0];
-  const Fq29 m = (p1[1] + p1[1] + p1[1]).norm();
-  Fq29 p2[4];
-  quad29_mul<4>(q, {u, a.x, m, v}, {v, v, m, a.zz}, p2);  // W, S, M^2, ZZ3
-  const Fq29 w = p2[0], s = p2[1];
-  G1X29 r;
-  r.x = p2[2].sub<4>(s + s);
-  r.zz = p2[3];
-  Fq29 p3[3];
-  quad29_mul<3>(q, {m, w, w}, {s.sub<8>(r.x), a.y, a.zzz}, p3);
-  r.y = p3[0].sub<2>(p3[1]);
-  r.zzz = p3[2];
-  return r;
-}
-
-__device__ __forceinline__ G1X29 quad29_add(const G1X29& a, const G1X29& o, u32 q) {
-  if (o.is_identity()) return a;
-  if (a.is_identity()) return o;
-  Fq29 p1[4];
-  quad29_mul<4>(q, {a.x, o.x, a.y, o.y}, {o.zz, a.zz, o.zzz, a.zzz}, p1);  // U1, U2, S1, S2
-  const Fq29 u1 = p1[0], s1 = p1[2];
-  const Fq29 p = p1[1].sub<2>(u1);
-  const Fq29 rr = p1[3].sub<2>(s1);
-  if (p.is_zero_modp()) {
-    if (rr.is_zero_modp()) return quad29_dbl(a, q);
-    return G1X29::identity();
+  __device__ __forceinline__ static Quad29 identity() { return Quad29{Fq29::zero()}; }
+  __device__ __forceinline__ static Quad29 load(const u32* p, u32 q) { return Quad29{Fq29::load(p + 8 * q)}; }
+  __device__ __forceinline__ void store(u32* p, u32 q) const { c.reduce_2p().store(p + 8 * q); }
+  __device__ __forceinline__ bool is_identity() const {
+    u32 any = 0;
+#pragma unroll
+    for (int i = 0; i < 9; i++) any |= c.l[i];
+    return quad_perm<2, 2, 2, 2>(any) == 0;
   }
-  Fq29 p2[4];
-  quad29_mul<4>(q, {p, rr, a.zz, a.zzz}, {p, rr, o.zz, o.zzz}, p2);  // PP, R^2, ZZ1 ZZ2, ZZZ1 ZZZ2
-  const Fq29 pp = p2[0];
-  Fq29 p3[3];
-  quad29_mul<3>(q, {p, u1, p2[2]}, {pp, pp, pp}, p3);  // PPP, Q, ZZ3
-  const Fq29 ppp = p3[0], qq = p3[1];
-  G1X29 r;
-  r.x = p2[1].sub<6>(ppp + qq + qq);
-  r.zz = p3[2];
-  Fq29 p4[3];
-  quad29_mul<3>(q, {rr, s1, p2[3]}, {qq.sub<8>(r.x), ppp, ppp}, p4);
-  r.y = p4[0].sub<2>(p4[1]);
-  r.zzz = p4[2];
-  return r;
-}
+  // lane 0's coordinate x and lane 1's y of an affine point (lanes 2 and 3 hold them too)
+  __device__ __forceinline__ static Quad29 from_affine(const Fq29& xy, u32 q) {
+    return Quad29{lane_pick(q < 2, xy.reduce_2p(), Fq29::one())};
+  }
+
+  // P (lane 0) and R (lane 1) in d; r1: U1 (lane 0) and S1 (lane 1); zz: ZZ1
+  // ZZ2 (lane 2) and ZZZ1 ZZZ2 (lane 3); r2: P^2 (lane 0) and R^2 (lane 1).
+  __device__ __forceinline__ static Quad29 finish(const Fq29& d, const Fq29& r1, const Fq29& zz, const Fq29& r2,
+                                                  bool same, u32 q) {
+    const Fq29 g = lane_pick(q == 0, d, lane_pick(q == 1, quad_lane<0>(r1), zz));
+    const Fq29 r3 = g * quad_lane<0>(r2);  // PPP, Q, ZZ3
+    const Fq29 ppp = quad_lane<0>(r3), qq = quad_lane<1>(r3);
+    const Fq29 x3 = quad_lane<1>(r2).sub<6>((same ? Fq29::zero() : ppp) + qq + qq);
+    const Fq29 h1 = lane_pick(q == 0, quad_lane<1>(d), lane_pick(q == 1, r1.neg<4>(), zz));
+    const Fq29 r4 = h1 * lane_pick(q == 0, qq.sub<8>(x3), ppp);  // R (Q - X3), -S1 PPP, , ZZZ3
+    const Fq29 y3 = (r4 + quad_lane<0>(r4)).norm();
+    return Quad29{lane_pick(q < 2, lane_pick(q == 0, x3, y3), lane_pick(q == 2, r3, r4))};
+  }
+  // d for doubling this point: 2Y on lane 0, 3 X^2 on the others
+  __device__ __forceinline__ Fq29 doubling_steps(u32 q) const {
+    const Fq29 x2 = quad_lane<0>(c * c), y = quad_lane<1>(c);
+    return lane_pick(q == 0, y + y, x2 + x2 + x2).norm();
+  }
+
+  __device__ __forceinline__ Quad29 add(const Quad29& o, u32 q) const {
+    if (o.is_identity()) return *this;
+    if (is_identity()) return o;
+    Fq29 r1 = c * quad_perm<2, 3, 0, 1>(o.c);        // U1, S1, U2, S2
+    Fq29 d = quad_perm<2, 3, 0, 1>(r1).sub<2>(r1);  // P, R
+    Fq29 f = o.c;
+    bool same = false;
+    const u32 zero = d.is_zero_modp() ? 1u : 0u;
+    if (quad_perm<0, 0, 0, 0>(zero)) {
+      if (!quad_perm<1, 1, 1, 1>(zero)) return identity();
+      d = doubling_steps(q);
+      r1 = c;
+      f = Fq29::one();  // ZZ 1 and ZZZ 1: the doubled point's own
+      same = true;
+    }
+    const Fq29 r2 = lane_pick(q < 2, d, c) * lane_pick(q < 2, d, f);  // PP, R^2, ZZ1 ZZ2, ZZZ1 ZZZ2
+    return finish(d, r1, r2, r2, same, q);
+  }
+
+  // this + an affine point, xy as in from_affine (below 32p)
+  __device__ __forceinline__ Quad29 add_affine(const Fq29& xy, bool inf, u32 q) const {
+    if (inf) return *this;
+    if (is_identity()) return from_affine(xy, q);
+    Fq29 d = (xy * quad_perm<2, 3, 2, 3>(c)).sub<8>(c);  // U2 - X, S2 - Y (below 10p)
+    bool same = false;
+    const u32 zero = d.is_zero_modp() ? 1u : 0u;
+    if (quad_perm<0, 0, 0, 0>(zero)) {
+      if (!quad_perm<1, 1, 1, 1>(zero)) return identity();
+      d = doubling_steps(q);
+      same = true;
+    }
+    return finish(d, c, c, d * d, same, q);
+  }
+};
 
 }  // namespace zkp

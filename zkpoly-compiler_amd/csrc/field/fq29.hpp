@@ -168,6 +168,41 @@ struct F29 {
     return r;
   }
 
+  // (a b + c d) 2^-261 with one reduction: below 2p for A B + C D <= 168.  Limbs
+  // below 2^29: 18 2^58 + 9 2^58 + carry < 2^64.
+  ZKP_HD static F29 mul_add(const F29& a, const F29& b, const F29& c, const F29& d) {
+    u32 m[9];
+    F29 r;
+    u64 acc = 0;
+#pragma unroll
+    for (int k = 0; k < 17; k++) {
+#pragma unroll
+      for (int i = 0; i < 9; i++) {
+        const int j = k - i;
+        if (j >= 0 && j <= 8) acc += (u64)a.l[i] * b.l[j];
+      }
+#pragma unroll
+      for (int i = 0; i < 9; i++) {
+        const int j = k - i;
+        if (j >= 0 && j <= 8) acc += (u64)c.l[i] * d.l[j];
+      }
+#pragma unroll
+      for (int i = 0; i < 9; i++) {
+        const int j = k - i;
+        if (i < k && j >= 1 && j <= 8) acc += (u64)m[i] * Params::P[j];
+      }
+      if (k < 9) {
+        m[k] = ((u32)acc * INV) & MASK;
+        acc += (u64)m[k] * Params::P[0];
+      } else {
+        r.l[k - 9] = (u32)acc & MASK;
+      }
+      acc >>= 29;
+    }
+    r.l[8] = (u32)acc;
+    return r;
+  }
+
   ZKP_HD F29 operator+(const F29& b) const {
     F29 r;
 #pragma unroll
@@ -214,6 +249,16 @@ struct F29 {
     F29 r;
 #pragma unroll
     for (int i = 0; i < 9; i++) r.l[i] = l[i] + kp.l[i] - b.l[i];
+    return r.norm();
+  }
+
+  // K p - this, normalised (this < K p).
+  template <int K>
+  ZKP_HD F29 neg() const {
+    constexpr Lifted<K> kp{};
+    F29 r;
+#pragma unroll
+    for (int i = 0; i < 9; i++) r.l[i] = kp.l[i] - l[i];
     return r.norm();
   }
 

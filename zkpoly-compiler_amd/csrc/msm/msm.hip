@@ -16,11 +16,12 @@
 //     a two-level partition sort in LDS (coarse bins, then the low bucket
 //     bits), no device atomics; windows above 20 bits use a device-atomic
 //     counting sort instead.
-//  3. bucket accumulation, load balanced: every thread owns 32 consecutive
-//     sorted entries and adds each run of equal keys into an XYZZ sum (mixed
-//     additions); runs that cross a chunk edge become (key, partial) pairs
-//     that the next level reduces the same way, so a bucket holding any share
-//     of the points (e.g. the scalar-1 bucket) costs log levels, not a serial walk.
+//  3. bucket accumulation, load balanced: every thread owns a chunk of
+//     consecutive sorted entries and adds each run of equal keys into an XYZZ
+//     sum (mixed additions); a run cut by chunk edges leaves pieces that one
+//     thread (or quad of lanes) per run adds up, and a run of many pieces (a
+//     bucket holding a large share of the points, e.g. the scalar-1 bucket) goes
+//     to a tree over all pieces instead, so it costs log steps, not a serial walk.
 //     Buckets and partials are G1X29 (xyzz29.hpp): Fq in nine 29-bit limbs,
 //     radix 2^261, lazily reduced -- one instruction per limb product.
 //  4. bucket reduction per window, S_w = sum_b b * B_b, by halving levels
@@ -40,6 +41,7 @@
 #include <chrono>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "../curve/g1.hpp"
@@ -49,11 +51,40 @@ namespace zkp {
 namespace msm {
 
 constexpr int THREADS = 256;
-constexpr uint32_t CHUNK = 32;   // sorted entries per thread at accumulation level 0
-constexpr uint32_t CHUNK_L = 8;  // (key, partial) entries per thread at the later levels
 constexpr uint32_t RED_TAIL = 128;  // items per window finished inside one workgroup
 constexpr uint32_t SCALAR_BITS = 254;
 constexpr int MAX_LEVELS = 24;
+
+// How up to `entries` sorted entries are shared out for the accumulation: `ch`
+// consecutive entries (a multiple of 4, read as 16-byte words) per thread, or
+// per quad of lanes.  65 536 lanes are one wave on each of the 1 024 SIMDs.  An
+// addition takes 4.5 us of a lone wave, 2.3 us of a quad; every chunk edge leaves
+// a piece of a run that costs a general addition (1.4 times the products) later.
+//  * Up to 800 K entries the chain of one chunk's additions sets the time, so
+//    quads take it, sixteen entries each, fewer where a bucket holds only a few.
+//  * Up to 4 M: two waves per SIMD, which fill the VALU nearly, in chunks of 16
+//    to 32, so that a bucket of the usual 32 entries has few pieces.
+//  * Above: all threads resident at once, four waves per SIMD, so that no last
+//    round of workgroups runs nearly empty; up to 128 entries.
+struct Share {
+  uint32_t ch;
+  bool quads;
+};
+static inline Share share_for(uint64_t entries) {
+  const bool quads = entries <= 800000;
+  uint64_t c;
+  if (quads) {
+    c = entries / 8192;
+    if (c > 16) c = 16;
+    if (c < 4) c = 4;
+  } else {
+    const uint64_t all = (entries + 262143) / 262144, two = (entries + 131071) / 131072;
+    c = two < 16 ? 16 : two < 32 ? two : 32;
+    if (all > c) c = all;
+    if (c > 128) c = 128;
+  }
+  return Share{(uint32_t)((c + 3) & ~3ull), quads};
+}
 
 #define ZKP_CHECK(x)                          \
   do {                                        \
@@ -67,6 +98,8 @@ struct Config {
   uint32_t n_windows;       // physical windows per table
   uint32_t n_precompute;    // point tables
   uint32_t buckets;         // 2^(s-1)
+  uint32_t top_log;         // the top window's buckets come in 2^top_log copies each
+  uint32_t bias[8];         // sum of 2^(s-1) 2^(s w) over the windows below the top one
 };
 
 static inline uint32_t div_ceil32(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
@@ -100,26 +133,60 @@ static bool make_config(uint32_t s, uint32_t target, Config* c) {
   c->n_precompute = div_ceil32(c->actual_windows, c->n_windows);
   if (c->n_precompute != ref_precompute) return false;  // would need a table the caller does not have
   c->buckets = 1u << (s - 1);
+  // The top window has 254 - s (windows - 1) bits, one to seven for most s, so
+  // its digits would put n points into a handful of buckets.  Where no other
+  // window shares its buckets (one table) digit d goes to bucket
+  // (d - 1) 2^top_log + (point index mod 2^top_log) instead, and the bucket
+  // reduction folds the copies in its first top_log levels: the same number of
+  // additions, and no run of thousands of pieces (2^14 points, s = 10, 4 bits:
+  // the long-run kernels took 125 us and now return at once).
+  c->top_log = 0;
+  if (c->n_precompute == 1 && c->n_windows == c->actual_windows) {
+    const uint32_t top = top_window_of_r_minus_1((c->actual_windows - 1) * s, s) + 1;  // largest digit
+    while ((top << (c->top_log + 1)) <= c->buckets) c->top_log++;
+  }
+  for (int i = 0; i < 8; i++) c->bias[i] = 0;
+  for (uint32_t w = 0; w + 1 < c->actual_windows; w++) {
+    const uint32_t bit = s * w + s - 1;
+    c->bias[bit >> 5] |= 1u << (bit & 31);
+  }
   return true;
 }
 
 // ---------------------------------------------------------------- digits
 
-// Signed s-bit digit of window w; `carry` flows from lower windows.
-__device__ __forceinline__ int next_digit(const Fr& c, uint32_t w, uint32_t s, int& carry) {
-  const uint32_t bit = w * s;
-  const uint32_t limb = bit >> 5, off = bit & 31;
-  uint64_t two = 0;
-  if (limb < 8) two = c.v[limb];
-  if (limb + 1 < 8) two |= (uint64_t)c.v[limb + 1] << 32;
-  int d = (int)((two >> off) & ((1ull << s) - 1)) + carry;
-  if (d >= (1 << (s - 1))) {
-    d -= 1 << s;
-    carry = 1;
-  } else {
-    carry = 0;
+// The signed s-bit digits of a scalar, lowest window first.  With 2^(s-1) added
+// at every window but the top one, window w's digit is its s bits minus
+// 2^(s-1): no carry runs from digit to digit, and the value moves down s bits
+// per window in registers (an index by bit position would put it in scratch).
+struct Digits {
+  uint32_t v[8];
+
+  __device__ __forceinline__ Digits(const uint32_t* scalar, const Config& cfg) {
+    const Fr c = Fr::load(scalar).to_canonical();
+    uint32_t carry = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = adc(c.v[i], cfg.bias[i], carry);  // below 2^255
   }
-  return d;
+  // an entry of no digits but zeros: all windows give 0
+  __device__ __forceinline__ explicit Digits(const Config& cfg) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = cfg.bias[i];
+  }
+  __device__ __forceinline__ int next(const Config& cfg, uint32_t w) {
+    const uint32_t d = v[0] & ((1u << cfg.s) - 1);
+#pragma unroll
+    for (int i = 0; i < 7; i++) v[i] = __builtin_amdgcn_alignbit(v[i + 1], v[i], cfg.s);
+    v[7] >>= cfg.s;
+    return w + 1 < cfg.actual_windows ? (int)d - (int)(1u << (cfg.s - 1)) : (int)d;
+  }
+};
+
+// Key of a nonzero digit d of window w: its bucket over all physical windows.
+__device__ __forceinline__ uint32_t bucket_key(const Config& cfg, uint32_t w, int d, uint64_t i) {
+  uint32_t b = (uint32_t)(d < 0 ? -d : d) - 1;
+  if (w + 1 == cfg.actual_windows) b = (b << cfg.top_log) | ((uint32_t)i & ((1u << cfg.top_log) - 1));
+  return (w % cfg.n_windows) * cfg.buckets + b;
 }
 
 // Wave-aggregated atomic increment of counter[bin] for the active lanes;
@@ -161,13 +228,10 @@ __global__ void __launch_bounds__(THREADS)
   for (uint64_t r = 0; r < rounds; r++) {
     const uint64_t i = r * stride + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = i < n;
-    const Fr c = valid ? Fr::load(scalars + i * 8).to_canonical() : Fr::zero();
-    int carry = 0;
+    Digits digits = valid ? Digits(scalars + i * 8, cfg) : Digits(cfg);
     for (uint32_t w = 0; w < cfg.actual_windows; w++) {
-      const int d = next_digit(c, w, cfg.s, carry);
-      const uint32_t pw = w % cfg.n_windows;
-      const uint32_t bin = pw * cfg.buckets + (uint32_t)(d < 0 ? -d : d) - 1;
-      aggregated_increment(hist, bin, valid && d != 0);
+      const int d = digits.next(cfg, w);
+      aggregated_increment(hist, bucket_key(cfg, w, d, i), d != 0);
     }
   }
 }
@@ -180,14 +244,12 @@ __global__ void __launch_bounds__(THREADS)
   for (uint64_t r = 0; r < rounds; r++) {
     const uint64_t i = r * stride + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = i < n;
-    const Fr c = valid ? Fr::load(scalars + i * 8).to_canonical() : Fr::zero();
-    int carry = 0;
+    Digits digits = valid ? Digits(scalars + i * 8, cfg) : Digits(cfg);
     for (uint32_t w = 0; w < cfg.actual_windows; w++) {
-      const int d = next_digit(c, w, cfg.s, carry);
-      const uint32_t pw = w % cfg.n_windows;
+      const int d = digits.next(cfg, w);
       const uint32_t table = w / cfg.n_windows;
-      const uint32_t key = pw * cfg.buckets + (uint32_t)(d < 0 ? -d : d) - 1;
-      const bool active = valid && d != 0;
+      const uint32_t key = bucket_key(cfg, w, d, i);
+      const bool active = d != 0;
       const uint32_t pos = aggregated_increment(cursor, key, active);
       if (active) {
         keys[pos] = key;
@@ -201,6 +263,7 @@ __global__ void __launch_bounds__(THREADS)
 
 constexpr int SCAN_BLOCK = 1024;  // elements per block: 256 threads x 4
 
+template <int NT = THREADS>
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* sh, uint32_t* total) {
   // inclusive scan inside each wave by shuffles, then the waves' totals through LDS
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -214,7 +277,7 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
   __syncthreads();
   uint32_t before = 0, all = 0;
 #pragma unroll
-  for (uint32_t w = 0; w < THREADS / 64; w++) {
+  for (uint32_t w = 0; w < NT / 64; w++) {
     const uint32_t t = sh[w];
     before += w < wave ? t : 0u;
     all += t;
@@ -297,20 +360,19 @@ __device__ __forceinline__ void part_count_tile(const uint32_t* __restrict__ sca
   for (uint32_t p = threadIdx.x; p < tp; p += THREADS) {
     const uint64_t i = first + p;
     if (i >= n) break;
-    const Fr c = Fr::load(scalars + i * 8).to_canonical();
-    int carry = 0;
+    Digits digits(scalars + i * 8, cfg);
     for (uint32_t w = 0; w < cfg.actual_windows; w++) {
-      const int d = next_digit(c, w, cfg.s, carry);
-      if (d == 0) continue;
-      const uint32_t key = (w % cfg.n_windows) * cfg.buckets + (uint32_t)(d < 0 ? -d : d) - 1;
-      atomicAdd(&cnt[key >> low_bits], 1u);
+      const int d = digits.next(cfg, w);
+      if (d != 0) atomicAdd(&cnt[bucket_key(cfg, w, d, i) >> low_bits], 1u);
     }
   }
 }
 
+// Also clears what the later kernels add into: the matrix's last entry and the
+// H bucket counts of k_seg_hist.
 __global__ void __launch_bounds__(THREADS)
     k_part_count(const uint32_t* __restrict__ scalars, uint64_t n, Config cfg, SortPlan sp,
-                 uint32_t* __restrict__ matrix) {
+                 uint32_t* __restrict__ matrix, uint32_t* __restrict__ ghist) {
   extern __shared__ uint32_t dyn[];
   uint32_t* cnt = dyn;  // nc
   for (uint32_t b = threadIdx.x; b < sp.nc; b += THREADS) cnt[b] = 0;
@@ -318,17 +380,21 @@ __global__ void __launch_bounds__(THREADS)
   part_count_tile(scalars, n, cfg, sp.low_bits, (uint64_t)blockIdx.x * sp.tp, sp.tp, cnt);
   __syncthreads();
   for (uint32_t b = threadIdx.x; b < sp.nc; b += THREADS) matrix[(uint64_t)b * sp.tiles + blockIdx.x] = cnt[b];
+  if (blockIdx.x == 0 && threadIdx.x == 0) matrix[(uint64_t)sp.nc * sp.tiles] = 0;
+  const uint32_t H = cfg.n_windows * cfg.buckets;
+  for (uint32_t b = blockIdx.x * THREADS + threadIdx.x; b < H; b += gridDim.x * THREADS) ghist[b] = 0;
 }
 
-// Exclusive scan of a[0..m) in LDS by the whole block; sh is THREADS words of scratch.
+// Exclusive scan of a[0..m) in LDS by the whole block; sh is NT / 64 words of scratch.
+template <int NT = THREADS>
 __device__ __forceinline__ void lds_exclusive_scan(uint32_t* a, uint32_t m, uint32_t* sh) {
-  const uint32_t per = (m + THREADS - 1) / THREADS;
+  const uint32_t per = (m + NT - 1) / NT;
   const uint32_t base = threadIdx.x * per;
   uint32_t local = 0;
   for (uint32_t k = 0; k < per; k++)
     if (base + k < m) local += a[base + k];
   uint32_t total;
-  uint32_t pre = block_exclusive_scan(local, sh, &total);
+  uint32_t pre = block_exclusive_scan<NT>(local, sh, &total);
   for (uint32_t k = 0; k < per; k++) {
     if (base + k < m) {
       const uint32_t x = a[base + k];
@@ -365,16 +431,15 @@ __global__ void __launch_bounds__(THREADS)
     for (uint32_t p = 0; p < PART_PPT; p++) {
       const uint64_t i = first + p * THREADS + threadIdx.x;
       const bool valid = i < n;
-      const Fr c = valid ? Fr::load(scalars + i * 8).to_canonical() : Fr::zero();
-      int carry = 0;
+      Digits digits = valid ? Digits(scalars + i * 8, cfg) : Digits(cfg);
 #pragma unroll
       for (uint32_t w = 0; w < PART_WMAX; w++) {
         ek[p][w] = ~0u;
         er[p][w] = 0;
         if (w < cfg.actual_windows) {
-          const int d = next_digit(c, w, cfg.s, carry);
-          if (valid && d != 0) {
-            const uint32_t key = (w % cfg.n_windows) * cfg.buckets + (uint32_t)(d < 0 ? -d : d) - 1;
+          const int d = digits.next(cfg, w);
+          if (d != 0) {
+            const uint32_t key = bucket_key(cfg, w, d, i);
             ek[p][w] = key | (d < 0 ? 0x80000000u : 0u);
             er[p][w] = atomicAdd(&base[key >> sp.low_bits], 1u);
           }
@@ -408,12 +473,11 @@ __global__ void __launch_bounds__(THREADS)
     for (uint32_t p = threadIdx.x; p < sp.tp; p += THREADS) {
       const uint64_t i = first + p;
       if (i >= n) break;
-      const Fr c = Fr::load(scalars + i * 8).to_canonical();
-      int carry = 0;
+      Digits digits(scalars + i * 8, cfg);
       for (uint32_t w = 0; w < cfg.actual_windows; w++) {
-        const int d = next_digit(c, w, cfg.s, carry);
+        const int d = digits.next(cfg, w);
         if (d == 0) continue;
-        const uint32_t key = (w % cfg.n_windows) * cfg.buckets + (uint32_t)(d < 0 ? -d : d) - 1;
+        const uint32_t key = bucket_key(cfg, w, d, i);
         const uint32_t slot = atomicAdd(&cur[key >> sp.low_bits], 1u);
         skey[slot] = key;
         sval[slot] = (uint32_t)((w / cfg.n_windows) * n + i) | (d < 0 ? 0x80000000u : 0u);
@@ -435,8 +499,9 @@ __global__ void __launch_bounds__(THREADS)
 // Second level: every coarse bin's segment is sorted by the low bits in slices
 // of at most SEG_SLICE entries, so a segment holding most entries of a narrow
 // window (s = 12, 13, 14, 18 and the small windows) is spread over many
-// workgroups.  Bucket counts of a one-slice segment are stored, those of a
-// longer one added up with one device atomic per nonzero bucket per slice.
+// workgroups.  A segment of one slice is counted and placed by that slice's
+// workgroup alone; the bucket counts of a longer one are added up first, with
+// one device atomic per nonzero bucket per slice (k_seg_hist, k_seg_scan).
 constexpr uint32_t SEG_SLICE = 8192;  // entries per workgroup, staged in LDS at once (64 KB)
 constexpr uint32_t SEG_PER_THREAD = SEG_SLICE / THREADS;
 
@@ -457,12 +522,12 @@ __device__ __forceinline__ uint32_t seg_begin(const uint32_t* offsets, const Sor
   return offsets[(uint64_t)cb * sp.tiles];
 }
 
-// slice_prefix[cb] = slices of the segments before cb (nc + 1 entries); one workgroup.
-__global__ void __launch_bounds__(THREADS)
-    k_seg_plan(const uint32_t* __restrict__ offsets, SortPlan sp, uint32_t* __restrict__ slice_prefix) {
-  __shared__ uint32_t sh[THREADS];
-  extern __shared__ uint32_t cnt[];  // nc + 1
-  for (uint32_t cb = threadIdx.x; cb <= sp.nc; cb += THREADS) {
+// slice_prefix[cb] = slices of the segments before cb (nc + 1 entries, cnt: LDS
+// of as many words), and the entry count; one workgroup of NT threads.
+template <int NT>
+__device__ __forceinline__ void seg_plan(const uint32_t* offsets, const SortPlan& sp, uint32_t* slice_prefix,
+                                         uint32_t* counts, uint32_t* cnt, uint32_t* sh) {
+  for (uint32_t cb = threadIdx.x; cb <= sp.nc; cb += NT) {
     uint32_t k = 0;
     if (cb < sp.nc) {
       const uint32_t size = seg_begin(offsets, sp, cb + 1) - seg_begin(offsets, sp, cb);
@@ -470,9 +535,48 @@ __global__ void __launch_bounds__(THREADS)
     }
     cnt[cb] = k;
   }
+  if (threadIdx.x == 0) counts[0] = seg_begin(offsets, sp, sp.nc);
   __syncthreads();
-  lds_exclusive_scan(cnt, sp.nc + 1, sh);
-  for (uint32_t cb = threadIdx.x; cb <= sp.nc; cb += THREADS) slice_prefix[cb] = cnt[cb];
+  lds_exclusive_scan<NT>(cnt, sp.nc + 1, sh);
+  for (uint32_t cb = threadIdx.x; cb <= sp.nc; cb += NT) slice_prefix[cb] = cnt[cb];
+}
+
+__global__ void __launch_bounds__(THREADS)
+    k_seg_plan(const uint32_t* __restrict__ offsets, SortPlan sp, uint32_t* __restrict__ slice_prefix,
+               uint32_t* __restrict__ counts) {
+  __shared__ uint32_t sh[THREADS];
+  extern __shared__ uint32_t cnt[];  // nc + 1
+  seg_plan<THREADS>(offsets, sp, slice_prefix, counts, cnt, sh);
+}
+
+// The scan of a small matrix (m entries) and the slice plan in one launch of
+// one workgroup: 1 024 threads take 4 096 entries a step.  Up to
+// SCAN_SMALL_MAX entries its steps (1 us each) take less than the four launches
+// of the tiled scan and k_seg_plan (18 us).
+constexpr int SCAN_SMALL_THREADS = 1024;
+constexpr uint32_t SCAN_SMALL_MAX = 32768;
+__global__ void __launch_bounds__(SCAN_SMALL_THREADS)
+    k_scan_small(uint32_t* matrix, uint32_t m, SortPlan sp, uint32_t* __restrict__ slice_prefix,
+                 uint32_t* __restrict__ counts) {
+  __shared__ uint32_t sh[SCAN_SMALL_THREADS / 64];
+  extern __shared__ uint32_t cnt[];  // nc + 1
+  uint32_t carry = 0;
+  for (uint32_t at = 0; at < m; at += 4 * SCAN_SMALL_THREADS) {
+    const uint32_t base = at + threadIdx.x * 4;
+    uint32_t v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = base + k < m ? matrix[base + k] : 0;
+    uint32_t total;
+    uint32_t pre = carry + block_exclusive_scan<SCAN_SMALL_THREADS>(v[0] + v[1] + v[2] + v[3], sh, &total);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (base + k < m) matrix[base + k] = pre;
+      pre += v[k];
+    }
+    carry += total;
+  }
+  __syncthreads();
+  seg_plan<SCAN_SMALL_THREADS>(matrix, sp, slice_prefix, counts, cnt, sh);
 }
 
 struct SegSlice {
@@ -494,13 +598,14 @@ __device__ __forceinline__ bool seg_slice(const uint32_t* offsets, const uint32_
   return true;
 }
 
-// ghist[cb * nb + bin] (zeroed beforehand) = entries of the segment in each bucket.
+// ghist[cb * nb + bin] (zeroed beforehand) = entries of the segment in each
+// bucket, for the segments of several slices.
 __global__ void __launch_bounds__(THREADS)
     k_seg_hist(const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ offsets,
                const uint32_t* __restrict__ slice_prefix, SortPlan sp, uint32_t* __restrict__ ghist) {
   extern __shared__ uint32_t h[];  // nb
   SegSlice sl;
-  if (!seg_slice(offsets, slice_prefix, sp, &sl)) return;  // uniform per block
+  if (!seg_slice(offsets, slice_prefix, sp, &sl) || sl.single) return;  // uniform per block
   const uint32_t nb = 1u << sp.low_bits, mask = nb - 1;
   for (uint32_t b = threadIdx.x; b < nb; b += THREADS) h[b] = 0;
   __syncthreads();
@@ -509,20 +614,20 @@ __global__ void __launch_bounds__(THREADS)
   uint32_t* g = ghist + (uint64_t)sl.cb * nb;
   for (uint32_t b = threadIdx.x; b < nb; b += THREADS) {
     const uint32_t c = h[b];
-    if (sl.single)
-      g[b] = c;
-    else if (c)
-      atomicAdd(&g[b], c);
+    if (c) atomicAdd(&g[b], c);
   }
 }
 
-// Per segment: ghist becomes the scatter cursor, the first entry of each bucket.
+// Per segment of several slices: ghist becomes the scatter cursor, the first
+// entry of each bucket.
 __global__ void __launch_bounds__(THREADS)
-    k_seg_scan(const uint32_t* __restrict__ offsets, SortPlan sp, uint32_t* __restrict__ ghist) {
+    k_seg_scan(const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ slice_prefix, SortPlan sp,
+               uint32_t* __restrict__ ghist) {
   extern __shared__ uint32_t h[];  // nb
   __shared__ uint32_t sh[THREADS];
   const uint32_t nb = 1u << sp.low_bits;
   const uint32_t cb = blockIdx.x;
+  if (slice_prefix[cb + 1] - slice_prefix[cb] <= 1) return;  // uniform per block
   const uint32_t start = seg_begin(offsets, sp, cb);
   uint32_t* g = ghist + (uint64_t)cb * nb;
   for (uint32_t b = threadIdx.x; b < nb; b += THREADS) h[b] = g[b];
@@ -568,11 +673,13 @@ __global__ void __launch_bounds__(THREADS)
   uint32_t* cur = cursor + (uint64_t)sl.cb * nb;
   for (uint32_t b = threadIdx.x; b < nb; b += THREADS) {
     const uint32_t c = cnt[b];
-    gcur[b] = sl.single ? cur[b] : (c ? atomicAdd(&cur[b], c) : 0u);
+    if (!sl.single) gcur[b] = c ? atomicAdd(&cur[b], c) : 0u;
     lbase[b] = c;
   }
   __syncthreads();
   lds_exclusive_scan(lbase, nb, sh);
+  if (sl.single)
+    for (uint32_t b = threadIdx.x; b < nb; b += THREADS) gcur[b] = sl.lo + lbase[b];
 #pragma unroll
   for (uint32_t k = 0; k < SEG_PER_THREAD; k++) {
     const uint32_t e = sl.lo + k * THREADS + threadIdx.x;
@@ -598,131 +705,334 @@ static inline uint32_t seg_scatter_lds(uint32_t low_bits) { return (3u * (1u << 
 
 // ---------------------------------------------------------------- accumulation
 
-// Closes a bucket.  Every bucket is completed at exactly one level (its whole
-// run, or all its partials, inside one chunk), so in the first part of an MSM
-// (fresh buckets hold the identity) the sum is stored, in later parts added.
-// Identity sums are skipped: slots without a partial carry a key too.
-__device__ __forceinline__ void bucket_close(u32* buckets, uint32_t key, const G1X29& sum, bool fresh) {
-  if (sum.is_identity()) return;
-  u32* p = buckets + (size_t)key * 32;
-  if (fresh) {
-    sum.store(p);
-    return;
-  }
-  const G1X29 cur = G1X29::load(p);
-  (cur.is_identity() ? sum : cur.add(sum)).store(p);
+// Closes a bucket: every bucket is completed exactly once (by one chunk, by
+// its run's thread or by the piece tree), and the set it goes to was filled
+// with the identity, so the sum is stored; an identity sum needs no store.
+__device__ __forceinline__ void quad_close(u32* buckets, uint32_t key, const Quad29& sum, uint32_t q) {
+  if (!sum.is_identity()) sum.store(buckets + (size_t)key * 32, q);
 }
 
 __device__ __forceinline__ Affine29 fetch_point(const u32* __restrict__ points, uint32_t v) {
   return Affine29::load(points + (size_t)(v & 0x7fffffffu) * 16, (v & 0x80000000u) != 0);
 }
 
-// One accumulation level.  Thread t owns sorted entries [t*CH, ...) and sums
-// each run of equal keys, one entry per loop step in every lane (a wave takes
-// CH steps whatever the run lengths).  A run closed on both sides goes to its bucket;
-// the chunk's first run (if it continues from the previous chunk) and last run
-// (if it continues into the next) are emitted as (key, partial) at slots 2t and
-// 2t + 1 of the next level, identity where there is nothing to carry, so every
-// key's pieces stay contiguous.
-template <bool FROM_POINTS, uint32_t CH>
-__device__ __forceinline__ void accumulate_chunk(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
-                                                 const u32* __restrict__ src, uint32_t* counts, uint32_t level, bool fresh,
-                                                 u32* buckets, uint32_t* __restrict__ next_keys,
-                                                 u32* __restrict__ next_pts) {
-  const uint32_t N = counts[level];
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t nchunks = (N + CH - 1) / CH;
-  if (t == 0) counts[level + 1] = 2 * nchunks;
-  if (t >= nchunks) return;
-  const uint32_t start = t * CH;
-  const uint32_t end = start + CH < N ? start + CH : N;
-  const uint32_t key_first = keys[start], key_last = keys[end - 1];
-  const bool open_left = start > 0 && keys[start - 1] == key_first;
-  const bool open_right = end < N && keys[end] == key_last;
-  bool a_done = false, b_done = false;
-  G1X29 acc = G1X29::identity();
-  uint32_t run_start = start;
-  for (uint32_t i = start; i < end; i++) {
-    const uint32_t key = keys[i];
-    if (FROM_POINTS)
-      acc = acc.add_affine(fetch_point(src, vals[i]));
+__device__ __forceinline__ uint32_t chunks_of(uint32_t entries, uint32_t ch) {
+  return entries / ch + (entries % ch != 0);
+}
+
+// Thread t owns sorted entries [t * ch, ...) (key, point index | sign << 31) and
+// sums each run of equal keys, one entry per loop step in every lane (a wave
+// takes ch steps whatever the run lengths).  A run closed on both sides goes to
+// its bucket; a run that continues from the previous chunk leaves its sum in
+// piece slot 2t, another one that continues into the next chunk in slot 2t + 1.
+// Nothing else is written: which slots hold a piece follows from the keys at
+// the chunk edges.
+// 109 VGPRs let four waves share a SIMD, which covers the dependent loads of an
+// entry (key, point index, point): 2^20 points at window 16 take 1.32 ms, 83 %
+// of the VALU's issue; 1.43 ms with the doubling inlined a second time (three waves).
+template <bool QUAD>
+__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3)))
+    k_accumulate(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
+                 const u32* __restrict__ points, uint32_t* counts, uint32_t ch, u32* buckets,
+                 u32* __restrict__ pieces) {
+  const uint32_t N = counts[0];
+  const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t t = QUAD ? gid >> 2 : gid, q = gid & 3;
+  if (gid == 0) counts[1] = 0;  // k_close_runs raises it
+  if (t >= chunks_of(N, ch)) return;
+  const uint32_t start = t * ch;
+  const uint32_t end = N - start > ch ? start + ch : N;
+  const bool open_left = start > 0 && keys[start - 1] == keys[start];
+  const bool open_right = end < N && keys[end] == keys[end - 1];
+  typename std::conditional<QUAD, Quad29, G1X29>::type acc;
+  acc = acc.identity();
+  auto put = [&](u32* p) {
+    if constexpr (QUAD)
+      acc.store(p, q);
     else
-      acc = acc.add(G1X29::load(src + (size_t)i * 32));
-    const bool run_end = (i + 1 == end) || keys[i + 1] != key;
-    if (run_end) {
-      const bool first = run_start == start, last = i + 1 == end;
-      if (first && open_left) {
-        if (next_pts) acc.store(next_pts + (size_t)(2 * t) * 32);
-        a_done = true;
-      } else if (last && open_right) {
-        if (next_pts) acc.store(next_pts + (size_t)(2 * t + 1) * 32);
-        b_done = true;
-      } else {
-        bucket_close(buckets, key, acc, fresh);
-      }
-      acc = G1X29::identity();
-      run_start = i + 1;
+      acc.store(p);
+  };
+  bool first = true;  // still in the chunk's first run
+  uint4 k4, v4;  // the next entries: a 16-byte load of each array per four steps
+  uint32_t next_key = keys[start];
+  for (uint32_t i = start; i < end; i++) {
+    if (((i - start) & 3) == 0) {  // the arrays end on a 16-byte word
+      k4 = *reinterpret_cast<const uint4*>(keys + i);
+      v4 = *reinterpret_cast<const uint4*>(vals + i);
+    }
+    const uint32_t key = next_key, val = v4.x;
+    v4 = make_uint4(v4.y, v4.z, v4.w, 0);
+    k4 = make_uint4(k4.y, k4.z, k4.w, 0);
+    const bool last = i + 1 == end;
+    next_key = last ? ~key : ((i - start) & 3) == 3 ? keys[i + 1] : k4.x;
+    if constexpr (QUAD) {
+      u32 w[8];
+      Fq29::load_words(points + (size_t)(val & 0x7fffffffu) * 16 + 8 * (q & 1), w);
+      u32 any = 0;
+#pragma unroll
+      for (int j = 0; j < 8; j++) any |= w[j];
+      any |= quad_perm<1, 0, 3, 2>(any);  // (0, 0) is the identity
+      Fq29 xy = Fq29::from_words<5>(w);
+      xy = lane_pick((q & 1) != 0 && (val & 0x80000000u) != 0, Fq29::zero().sub<32>(xy), xy);
+      acc = acc.add_affine(xy, any == 0, q);
+    } else {
+      acc = acc.add_affine(fetch_point(points, val));
+    }
+    if (next_key != key) {
+      if (first && open_left)
+        put(pieces + (size_t)(2 * t) * 32);
+      else if (last && open_right)
+        put(pieces + (size_t)(2 * t + 1) * 32);
+      else if (!acc.is_identity())
+        put(buckets + (size_t)key * 32);
+      acc = acc.identity();
+      first = false;
     }
   }
-  if (next_keys) {
-    next_keys[2 * t] = key_first;
-    next_keys[2 * t + 1] = key_last;
-    if (!a_done) G1X29::identity().store(next_pts + (size_t)(2 * t) * 32);
-    if (!b_done) G1X29::identity().store(next_pts + (size_t)(2 * t + 1) * 32);
-  }
 }
 
-// Level 0: entries are (key, point index | sign << 31).  Three waves per SIMD
-// (168 VGPRs, a few values spilled) run it faster than two without spills: the
-// dependent loads of an entry (key, point index, point) wait less.
-__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3)))
-    k_accumulate0(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
-                  const u32* __restrict__ points, uint32_t* counts, bool fresh, u32* buckets,
-                  uint32_t* __restrict__ next_keys, u32* __restrict__ next_pts) {
-  accumulate_chunk<true, CHUNK>(keys, vals, points, counts, 0, fresh, buckets, next_keys, next_pts);
-}
-
-// Level >= 1: entries are (key, XYZZ partial).  With run_flag given, the
-// level runs only when *run_flag is set (k_close_runs found a long run).
-__global__ void __launch_bounds__(THREADS)
-    k_accumulate(const uint32_t* __restrict__ keys, const u32* __restrict__ pts, uint32_t* counts, uint32_t level,
-                 bool fresh, u32* buckets, uint32_t* __restrict__ next_keys, u32* __restrict__ next_pts,
-                 const uint32_t* __restrict__ run_flag) {
-  if (run_flag && *run_flag == 0u) return;
-  accumulate_chunk<false, CHUNK_L>(keys, nullptr, pts, counts, level, fresh, buckets, next_keys, next_pts);
-}
-
-// After the first chunked level the open pieces of a bucket form short runs
-// of equal keys (for scalars spread over the buckets, a bucket that crosses
-// chunk edges leaves two to four slots), which fixed chunk edges would keep
-// deferring level after level.  Here the thread at the first slot of every
-// run of at most RUN_MAX slots adds the run, closes the bucket and marks the
-// slots consumed (ZZ = 0, the identity), so the bucket is completed once.  A
-// longer run (a bucket holding a large share of the points) raises *run_flag
-// and stays for the chunked levels, which see the consumed slots as identity.
+// A run cut by chunk edges has pieces 2t + 1 (it starts in chunk t), 2(t + 1),
+// 2(t + 2), ...  One thread (QUAD: one quad of lanes) per chunk edge
+// adds the pieces of the run that starts left of it and closes the bucket.
+// With scalars spread over the buckets nearly every edge starts a run of two
+// to a few pieces, so the lanes of a wave stay busy.  A run of more than
+// RUN_MAX pieces after its first is left to k_long_tiles, and counts[1] says so.
 constexpr uint32_t RUN_MAX = 16;
 
+template <bool QUAD>
 __global__ void __launch_bounds__(THREADS)
-    k_close_runs(const uint32_t* __restrict__ keys, u32* __restrict__ pts, const uint32_t* __restrict__ counts,
-                 uint32_t level, bool fresh, u32* buckets, uint32_t* __restrict__ run_flag) {
-  const uint32_t N = counts[level];
-  const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= N) return;
-  const uint32_t key = keys[s];
-  if (s > 0 && keys[s - 1] == key) return;  // not the first slot of its run
-  uint32_t e = s + 1;
-  while (e < N && e - s <= RUN_MAX && keys[e] == key) e++;
-  if (e - s > RUN_MAX) {
-    *run_flag = 1u;
+    k_close_runs(const uint32_t* __restrict__ keys, const u32* __restrict__ pieces, uint32_t* counts, uint32_t ch,
+                 u32* buckets) {
+  const uint32_t N = counts[0];
+  const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t t = QUAD ? gid >> 2 : gid, q = gid & 3;
+  const uint32_t nchunks = chunks_of(N, ch);
+  if (t + 1 >= nchunks) return;
+  const uint32_t key = keys[t * ch + ch - 1];
+  if (keys[(t + 1) * ch] != key) return;                                   // no run crosses this edge
+  if (t > 0 && keys[t * ch] == key && keys[t * ch - 1] == key) return;  // it started further left
+  if (t + 1 + RUN_MAX < nchunks && keys[(t + 1 + RUN_MAX) * ch] == key) {
+    counts[1] = 1;
     return;
   }
-  G1X29 acc = G1X29::identity();
-  for (uint32_t i = s; i < e; i++) {
-    u32* p = pts + (size_t)i * 32;
-    acc = acc.add(G1X29::load(p));
-    Fq::zero().store(p + 16);
+  // pieces after the first: 1 .. RUN_MAX, the chunks from t + 1 on that start with the key
+  uint32_t n = 1, above = RUN_MAX + 1;
+  if (t + 2 >= nchunks || keys[(t + 2) * ch] != key) above = 2;
+  while (above - n > 1) {
+    const uint32_t mid = (n + above) >> 1;
+    if (t + mid < nchunks && keys[(t + mid) * ch] == key)
+      n = mid;
+    else
+      above = mid;
   }
-  bucket_close(buckets, key, acc, fresh);
+  const u32* base = pieces + (size_t)(2 * t + 1) * 32;  // piece k > 0 is k * 64 - 32 words on
+  if constexpr (QUAD) {
+    Quad29 acc = Quad29::load(base, q), p = Quad29::load(base + 32, q);
+    for (uint32_t k = 1;; k++) {
+      // the next piece crosses from memory during this addition
+      const Quad29 next = k < n ? Quad29::load(base + 32 + (size_t)k * 64, q) : p;
+      acc = acc.add(p, q);
+      if (k >= n) break;
+      p = next;
+    }
+    quad_close(buckets, key, acc, q);
+  } else {
+    G1X29 acc = G1X29::load(base), p = G1X29::load(base + 32);
+    for (uint32_t k = 1;; k++) {
+      const G1X29 next = k < n ? G1X29::load(base + 32 + (size_t)k * 64) : p;
+      acc = acc.add(p);
+      if (k >= n) break;
+      p = next;
+    }
+    if (!acc.is_identity()) acc.store(buckets + (size_t)key * 32);
+  }
+}
+
+// ---- the pieces of long runs: a segmented sum over all pieces in order ----
+//
+// A segment of the piece sequence is its first run's key and sum, and, when it
+// holds several runs, its last run's key and sum; the runs between are complete
+// and closed.  Every quad of lanes walks a share of the pieces, the 64 quads of
+// a workgroup join their segments in LDS as a tree, k_long_tiles leaves one
+// segment per workgroup and k_long_join joins those.  So a run of any length
+// costs (its pieces / 64 / LONG_TILES) + about 30 additions in sequence.
+constexpr uint32_t LONG_QUADS = THREADS / 4;
+constexpr uint32_t LONG_TILES = 512;
+
+enum : uint32_t { SEG_EMPTY = 0, SEG_ONE = 1, SEG_SEVERAL = 2 };  // runs in a segment: none, one, more
+
+struct SegmentLds {
+  Quad29 first[LONG_QUADS][4], last[LONG_QUADS][4];  // [quad][lane]
+  uint32_t key_first[LONG_QUADS], key_last[LONG_QUADS], runs[LONG_QUADS];
+};
+
+// The walk of one quad: pieces in order, each joined to the run before it.
+struct SegmentWalk {
+  uint32_t key_first = 0, key = 0, runs = SEG_EMPTY;
+  Quad29 sum;
+
+  __device__ __forceinline__ void piece(SegmentLds& S, uint32_t quad, uint32_t q, u32* buckets, uint32_t k,
+                                        const Quad29& p) {
+    if (runs != SEG_EMPTY && k == key) {
+      sum = sum.add(p, q);
+      return;
+    }
+    if (runs == SEG_EMPTY) {
+      key_first = k;
+      runs = SEG_ONE;
+    } else {
+      if (runs == SEG_ONE)
+        S.first[quad][q] = sum;
+      else
+        quad_close(buckets, key, sum, q);
+      runs = SEG_SEVERAL;
+    }
+    key = k;
+    sum = p;
+  }
+  __device__ __forceinline__ void finish(SegmentLds& S, uint32_t quad, uint32_t q) const {
+    if (runs == SEG_ONE) S.first[quad][q] = sum;
+    if (runs == SEG_SEVERAL) S.last[quad][q] = sum;
+    if (q != 0) return;
+    S.runs[quad] = runs;
+    S.key_first[quad] = key_first;
+    S.key_last[quad] = key;
+  }
+};
+
+// Joins the quads' segments into quad 0's (whole workgroup).  Every value a
+// quad reads before it writes is its own or that of the quad it takes in.
+__device__ __forceinline__ void join_segments(SegmentLds& S, uint32_t quad, uint32_t q, u32* buckets) {
+  for (uint32_t step = 1; step < LONG_QUADS; step <<= 1) {
+    __syncthreads();
+    if (quad & (2 * step - 1)) continue;
+    const uint32_t r = quad + step;
+    const uint32_t lruns = S.runs[quad], rruns = S.runs[r];
+    if (rruns == SEG_EMPTY) continue;
+    const uint32_t lkey = S.key_last[quad], rkey = S.key_first[r];
+    const Quad29 f = S.first[r][q];
+    uint32_t runs = SEG_SEVERAL;
+    if (lruns == SEG_EMPTY) {
+      S.first[quad][q] = f;
+      runs = rruns;
+      if (q == 0) S.key_first[quad] = rkey;
+    } else {
+      const Quad29 l = lruns == SEG_ONE ? S.first[quad][q] : S.last[quad][q];
+      if (lkey == rkey) {
+        const Quad29 s = l.add(f, q);
+        if (lruns == SEG_ONE)
+          S.first[quad][q] = s;
+        else if (rruns == SEG_ONE)
+          S.last[quad][q] = s;
+        else
+          quad_close(buckets, lkey, s, q);
+        if (lruns == SEG_ONE && rruns == SEG_ONE) runs = SEG_ONE;
+      } else {
+        if (lruns == SEG_SEVERAL) quad_close(buckets, lkey, l, q);
+        if (rruns == SEG_SEVERAL)
+          quad_close(buckets, rkey, f, q);
+        else
+          S.last[quad][q] = f;
+      }
+    }
+    if (rruns == SEG_SEVERAL) S.last[quad][q] = S.last[r][q];
+    if (q == 0) {
+      S.runs[quad] = runs;
+      S.key_last[quad] = S.key_last[r];
+    }
+  }
+  __syncthreads();
+}
+
+// One workgroup's share of the chunks; its segment goes to seg_pts[2b], [2b + 1]
+// and seg_meta[3b ..] (runs, first key, last key).  Only the pieces of long
+// runs count: the others were closed by k_close_runs.
+__global__ void __launch_bounds__(THREADS)
+    k_long_tiles(const uint32_t* __restrict__ keys, const u32* __restrict__ pieces,
+                 const uint32_t* __restrict__ counts, uint32_t ch, u32* buckets, uint32_t* __restrict__ seg_meta,
+                 u32* __restrict__ seg_pts) {
+  if (counts[1] == 0) return;
+  __shared__ SegmentLds S;
+  const uint32_t N = counts[0];
+  const uint32_t nchunks = chunks_of(N, ch);
+  const uint32_t quad = threadIdx.x >> 2, q = threadIdx.x & 3;
+  const uint32_t per = (nchunks + LONG_TILES * LONG_QUADS - 1) / (LONG_TILES * LONG_QUADS);
+  const uint32_t lo = (blockIdx.x * LONG_QUADS + quad) * per;
+  const uint32_t hi = lo + per < nchunks ? lo + per : nchunks;
+  SegmentWalk w;
+  for (uint32_t base = lo; base < hi; base += 4) {
+    // four chunks at a time, their keys looked at by one lane each: bit 0, slot
+    // 2u holds a piece of a long run; bit 1, slot 2u + 1 does
+    const uint32_t u0 = base + q;
+    uint32_t mine = 0, kf = 0, kl = 0;
+    if (u0 < hi) {
+      kf = keys[u0 * ch];
+      kl = keys[u0 + 1 < nchunks ? u0 * ch + ch - 1 : N - 1];
+      const bool open_left = u0 > 0 && keys[u0 * ch - 1] == kf;
+      if (open_left) {
+        // c: the first chunk, within RUN_MAX + 1 before u0, that starts with the
+        // run's key; the run starts there or in the chunk before, and is long
+        // when the chunk RUN_MAX + 1 after its start still holds it
+        uint32_t below = u0 > RUN_MAX + 1 ? u0 - RUN_MAX - 2 : ~0u, c = u0;  // chunk `below` is not looked at
+        while (c - below > 1) {
+          const uint32_t mid = below + ((c - below) >> 1);
+          if (keys[mid * ch] == kf)
+            c = mid;
+          else
+            below = mid;
+        }
+        const uint32_t t = c > 0 && keys[c * ch - 1] == kf ? c - 1 : c;
+        if (u0 - t > RUN_MAX || (t + 1 + RUN_MAX < nchunks && keys[(t + 1 + RUN_MAX) * ch] == kf)) mine = 1;
+      }
+      // (a chunk that is all the run of slot 2u has nothing in slot 2u + 1)
+      if (!(open_left && kl == kf) && u0 + 1 + RUN_MAX < nchunks && keys[(u0 + 1) * ch] == kl &&
+          keys[(u0 + 1 + RUN_MAX) * ch] == kl)
+        mine |= 2;
+    }
+    const uint32_t lane0 = __lane_id() & ~3u;
+    for (uint32_t j = 0; j < 8; j++) {
+      const int from = (int)(lane0 + (j >> 1));
+      const uint32_t bits = __shfl(mine, from);
+      const uint32_t key_f = __shfl(kf, from), key_l = __shfl(kl, from);
+      if ((bits >> (j & 1)) & 1)
+        w.piece(S, quad, q, buckets, (j & 1) ? key_l : key_f,
+                Quad29::load(pieces + (size_t)(2 * (base + (j >> 1)) + (j & 1)) * 32, q));
+    }
+  }
+  w.finish(S, quad, q);
+  join_segments(S, quad, q, buckets);
+  if (quad == 0) {
+    uint32_t* m = seg_meta + 3 * blockIdx.x;
+    if (q == 0) {
+      m[0] = S.runs[0];
+      m[1] = S.key_first[0];
+      m[2] = S.key_last[0];
+    }
+    if (S.runs[0] != SEG_EMPTY) S.first[0][q].store(seg_pts + (size_t)(2 * blockIdx.x) * 32, q);
+    if (S.runs[0] == SEG_SEVERAL) S.last[0][q].store(seg_pts + (size_t)(2 * blockIdx.x + 1) * 32, q);
+  }
+}
+
+// The tiles' segments joined (one workgroup); the last runs are closed.
+__global__ void __launch_bounds__(THREADS)
+    k_long_join(const uint32_t* __restrict__ counts, const uint32_t* __restrict__ seg_meta,
+                const u32* __restrict__ seg_pts, u32* buckets) {
+  if (counts[1] == 0) return;
+  __shared__ SegmentLds S;
+  const uint32_t quad = threadIdx.x >> 2, q = threadIdx.x & 3;
+  SegmentWalk w;
+  const uint32_t per = 2 * LONG_TILES / LONG_QUADS;
+  for (uint32_t v = quad * per; v < (quad + 1) * per; v++) {
+    const uint32_t b = v >> 1;
+    if (seg_meta[3 * b] > (v & 1))
+      w.piece(S, quad, q, buckets, seg_meta[3 * b + 1 + (v & 1)], Quad29::load(seg_pts + (size_t)v * 32, q));
+  }
+  w.finish(S, quad, q);
+  join_segments(S, quad, q, buckets);
+  if (quad == 0) {
+    if (S.runs[0] != SEG_EMPTY) quad_close(buckets, S.key_first[0], S.first[0][q], q);
+    if (S.runs[0] == SEG_SEVERAL) quad_close(buckets, S.key_last[0], S.last[0][q], q);
+  }
 }
 
 __global__ void __launch_bounds__(THREADS) k_zero_u32(uint32_t* p, uint64_t n) {
@@ -794,6 +1104,9 @@ __global__ void k_set_count(uint32_t* counts, const uint32_t* offsets, uint32_t 
 // S = Y_0.  Level 0 has X = Y = buckets, bucket b at j = b - 1, which makes
 // S = sum_b b B_b.  X' and Y' are computed by different threads (different
 // waves), so a level is two point operations deep.
+// The top window's first top_log levels only fold its buckets' copies,
+// X'_i = X_2i + X_2i+1 and Y'_i = Y_2i + Y_2i+1, which leaves
+// S = sum_i i X'_i + sum_i Y'_i with one item per digit.
 
 // The first two levels at once, one thread per block of four buckets
 // B_0..B_3 (items 4i..4i+3 of a window): X'' = 4T with T = B_0 + .. + B_3, and
@@ -802,26 +1115,45 @@ __global__ void k_set_count(uint32_t* counts, const uint32_t* offsets, uint32_t 
 // items.  Six additions and two doublings (102 products) per four buckets,
 // where two halving levels take 51 products per pair, 153 per four buckets.
 __global__ void __launch_bounds__(THREADS)
-    k_reduce_block4(const u32* __restrict__ B, uint32_t M, uint32_t n_windows, u32* __restrict__ Xo,
+    k_reduce_block4(const u32* __restrict__ B, uint32_t M, uint32_t n_windows, uint32_t fold_top, u32* __restrict__ Xo,
                     u32* __restrict__ Yo) {
   const uint32_t blocks = (M >> 2) * n_windows;
   const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
   if (gid >= blocks) return;
+  // folding levels of this window: both, X'' = Y'' = T; the first, X'' = 2T and Y'' = T + s_2
+  const uint32_t fold = gid / (M >> 2) == n_windows - 1 ? fold_top : 0;
   const size_t j0 = (size_t)gid * 4;  // windows are consecutive runs of M items: block gid covers 4 gid..4 gid+3
-  const G1X29 b3 = G1X29::load(B + (j0 + 3) * 32);
-  const G1X29 s2 = G1X29::load(B + (j0 + 2) * 32).add(b3);
-  const G1X29 u = s2.add(b3);  // s_2 + s_3
-  const G1X29 s1 = G1X29::load(B + (j0 + 1) * 32).add(s2);
-  const G1X29 t = G1X29::load(B + j0 * 32).add(s1);
-  t.add(s1).add(u).store(Yo + (size_t)gid * 32);
-  t.dbl().dbl().store(Xo + (size_t)gid * 32);
+  // s = s_3, s_2, s_1, s_0 = T and y their sum, one addition per loop step so
+  // that one copy of its code serves them all; then two doublings of T.
+  G1X29 s = G1X29::load(B + (j0 + 3) * 32);
+  G1X29 y = s;
+#pragma unroll 1
+  for (int step = 0; step < 8; step++) {
+    const bool to_s = !(step & 1);
+    if (fold >= 2 && (!to_s || step >= 6)) continue;
+    if (fold == 1) {
+      if (step == 1) y = s;
+      if (step == 1 || step == 3 || step == 7) continue;
+    }
+    const G1X29 a = to_s ? s : y;
+    G1X29 b = s;
+    if (to_s && step < 6) b = G1X29::load(B + (j0 + 2 - (step >> 1)) * 32);
+    const G1X29 r = step < 6 ? a.add(b) : s.dbl();
+    if (to_s || step >= 6)
+      s = r;
+    else
+      y = r;
+    if (step == 5) y.store(Yo + (size_t)gid * 32);
+  }
+  if (fold >= 2) s.store(Yo + (size_t)gid * 32);
+  s.store(Xo + (size_t)gid * 32);
 }
 
 // One level over all windows: threads [0, Mo * n_windows) write X', the next
 // Mo * n_windows threads write Y' (Mo = M / 2).
 __global__ void __launch_bounds__(THREADS)
     k_reduce_level(const u32* __restrict__ X, const u32* __restrict__ Y, uint32_t M, uint32_t n_windows,
-                   bool first, u32* __restrict__ Xo, u32* __restrict__ Yo) {
+                   bool first, bool fold_top, u32* __restrict__ Xo, u32* __restrict__ Yo) {
   const uint32_t Mo = M >> 1;
   const uint32_t items = Mo * n_windows;
   const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -829,22 +1161,24 @@ __global__ void __launch_bounds__(THREADS)
   const bool yside = gid >= items;
   const uint32_t it = yside ? gid - items : gid;
   const size_t j0 = (size_t)(it / Mo) * M + 2 * (it % Mo);
+  const u32* src = yside && !first ? Y : X;
   const G1X29 x1 = G1X29::load(X + (j0 + 1) * 32);
-  if (!yside) {
-    G1X29::load(X + j0 * 32).add(x1).dbl().store(Xo + (size_t)it * 32);
-  } else {
-    const u32* src = first ? X : Y;
-    const G1X29 y1 = first ? x1 : G1X29::load(Y + (j0 + 1) * 32);
-    G1X29::load(src + j0 * 32).add(y1).add(x1).store(Yo + (size_t)it * 32);
+  G1X29 r = G1X29::load(src + j0 * 32);
+  G1X29 o = G1X29::load(src + (j0 + 1) * 32);
+  const int steps = fold_top && it / Mo == n_windows - 1 ? 1 : 2;
+#pragma unroll 1
+  for (int step = 0; step < steps; step++) {  // one copy of the addition; X' doubles through it
+    r = r.add(o);
+    o = yside ? x1 : r;
   }
+  r.store((yside ? Yo : Xo) + (size_t)it * 32);
 }
 
-// The same level with a quad of lanes per point operation (quad29_add /
-// quad29_dbl): for the narrow levels, where the operations are few and each
+// The same level with a quad of lanes per point operation (Quad29): for the narrow levels, where the operations are few and each
 // one's latency, not the throughput, sets the time.
 __global__ void __launch_bounds__(THREADS)
     k_reduce_level_quad(const u32* __restrict__ X, const u32* __restrict__ Y, uint32_t M, uint32_t n_windows,
-                        bool first, u32* __restrict__ Xo, u32* __restrict__ Yo) {
+                        bool first, bool fold_top, u32* __restrict__ Xo, u32* __restrict__ Yo) {
   const uint32_t Mo = M >> 1;
   const uint32_t items = Mo * n_windows;
   const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -853,55 +1187,67 @@ __global__ void __launch_bounds__(THREADS)
   const bool yside = op >= items;
   const uint32_t it = yside ? op - items : op;
   const size_t j0 = (size_t)(it / Mo) * M + 2 * (it % Mo);
-  const G1X29 x1 = G1X29::load(X + (j0 + 1) * 32);
-  G1X29 r;
-  if (!yside) {
-    r = quad29_dbl(quad29_add(G1X29::load(X + j0 * 32), x1, q), q);
-  } else {
-    const u32* src = first ? X : Y;
-    const G1X29 y1 = first ? x1 : G1X29::load(Y + (j0 + 1) * 32);
-    r = quad29_add(quad29_add(G1X29::load(src + j0 * 32), y1, q), x1, q);
+  const u32* src = yside && !first ? Y : X;
+  const Quad29 x1 = Quad29::load(X + (j0 + 1) * 32, q);
+  Quad29 r = Quad29::load(src + j0 * 32, q);
+  Quad29 o = Quad29::load(src + (j0 + 1) * 32, q);
+  const int steps = fold_top && it / Mo == n_windows - 1 ? 1 : 2;
+#pragma unroll 1
+  for (int step = 0; step < steps; step++) {
+    r = r.add(o, q);
+    o = yside ? x1 : r;
   }
-  if (q == 0) r.store((yside ? Yo : Xo) + (size_t)it * 32);
+  r.store((yside ? Yo : Xo) + (size_t)it * 32, q);
 }
 
 // The last levels of window blockIdx.x (M <= RED_TAIL items) in LDS, all in
-// one launch, a quad of lanes per point operation: QUAD_TAIL_THREADS threads,
-// the operations writing X' on the lower half of them; out[w] = S_w.  At
-// 512 threads the kernel may keep 256 VGPRs, which the quad's operand copies
-// need (at 1024 it spilled).
+// one launch, a quad of lanes per point operation; out[w] = S_w.  fold_top: how
+// many of the levels fold the top window's copies.  The X' quads of a level of
+// P items come first and the Y' quads from the next wave on, so that the two
+// waves of the narrow levels run on two SIMDs (waves 0 and 4 of a workgroup
+// would share one).
 constexpr uint32_t QUAD_TAIL_THREADS = 4 * RED_TAIL;
 __global__ void __launch_bounds__(QUAD_TAIL_THREADS)
     k_reduce_tail_quad(const u32* __restrict__ X, const u32* __restrict__ Y, uint32_t M, bool first,
-                       u32* __restrict__ out) {
-  __shared__ G1X29 sx[RED_TAIL], sy[RED_TAIL];
+                       uint32_t fold_top, u32* __restrict__ out) {
+  __shared__ Quad29 sh[2][RED_TAIL][4];  // X, Y; [item][lane]
   const size_t base = (size_t)blockIdx.x * M;
-  for (uint32_t j = threadIdx.x; j < M; j += QUAD_TAIL_THREADS) {
-    sx[j] = G1X29::load(X + (base + j) * 32);
-    sy[j] = first ? sx[j] : G1X29::load(Y + (base + j) * 32);
+  const uint32_t op = threadIdx.x >> 2, q = threadIdx.x & 3;
+  if (op < M) {
+    sh[0][op][q] = Quad29::load(X + (base + op) * 32, q);
+    sh[1][op][q] = Quad29::load((first ? X : Y) + (base + op) * 32, q);
   }
   __syncthreads();
-  const uint32_t op = threadIdx.x >> 2, q = threadIdx.x & 3;
-  const bool yside = op >= RED_TAIL / 2;
-  const uint32_t i = yside ? op - RED_TAIL / 2 : op;
+  uint32_t fold = blockIdx.x + 1 == gridDim.x ? fold_top : 0;
   for (uint32_t P = M >> 1; P >= 1; P >>= 1) {
+    const uint32_t y0 = P < 16 ? 16 : P;  // first Y' quad
+    const uint32_t side = op >= y0 ? 1 : 0;
+    const uint32_t i = op - (side ? y0 : 0);
     const bool act = i < P;  // the same for the four lanes of a quad
-    G1X29 r;
+    const int steps = fold > 0 ? 1 : 2;
+    if (fold > 0) fold--;
+    Quad29 r, o;
     if (act) {
-      const G1X29 x1 = sx[2 * i + 1];
-      r = yside ? quad29_add(quad29_add(sy[2 * i], sy[2 * i + 1], q), x1, q)
-                : quad29_dbl(quad29_add(sx[2 * i], x1, q), q);
+      r = sh[side][2 * i][q];
+      o = sh[side][2 * i + 1][q];
+#pragma unroll 1
+      for (int step = 0; step < steps; step++) {  // X' doubles through the addition
+        r = r.add(o, q);
+        o = r;
+        if (side) o = sh[0][2 * i + 1][q];
+      }
     }
     __syncthreads();
-    if (act && q == 0) {
-      if (yside)
-        sy[i] = r;
-      else
-        sx[i] = r;
-    }
+    if (act) sh[side][i][q] = r;
     __syncthreads();
   }
-  if (threadIdx.x == 0) sy[0].store_mont256(out + (size_t)blockIdx.x * 32);  // the host reads G1XYZZ
+  // The host reads G1XYZZ: a coordinate per lane (were the value uniform the
+  // compiler would take its products to the scalar unit, 12 us of them).
+  if (threadIdx.x < 4) {
+    u32 w[8];
+    sh[1][0][q].c.to_mont256(w);
+    Fq::from_raw(w).store(out + (size_t)blockIdx.x * 32 + 8 * q);
+  }
 }
 
 // ---------------------------------------------------------------- precompute
@@ -941,7 +1287,7 @@ static inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Device workspace for one MSM of `len` points (per table) and config cfg.
 struct Layout {
-  size_t hist, block_sums, cursor, keys0, vals0, counts, lvl_keys[2], lvl_pts[2], buckets, red[4], sums, total;
+  size_t hist, block_sums, cursor, keys0, vals0, counts, pieces, seg_meta, seg_pts, buckets, red[4], sums, total;
   size_t matrix, keys_tmp, vals_tmp, slices;  // partition sort (when `part`)
   uint32_t max_slices;
   bool part;
@@ -950,8 +1296,8 @@ struct Layout {
   uint32_t nb_matrix;
   uint32_t H, nb_scan;
   uint64_t n_entries_max;
-  uint32_t level_max[MAX_LEVELS];
-  int levels;  // accumulation levels after level 0
+  Share share;          // how the accumulation is shared out
+  uint32_t chunks_max;  // accumulating threads or quads
   uint32_t red_m[MAX_LEVELS];
   int red_levels;  // one-level launches before the in-workgroup tail
   size_t bucket_bytes;  // one bucket set (n_windows * 2^(s-1) XYZZ points)
@@ -997,23 +1343,8 @@ static bool make_layout(const Config& cfg, uint64_t len, Layout* L, uint32_t set
   }
   L->n_entries_max = len * cfg.actual_windows;
   if (len * cfg.n_precompute >= 0x80000000ull || L->n_entries_max >= 0xffffffffull) return false;
-  // accumulation level sizes (upper bounds)
-  uint64_t m = L->n_entries_max;
-  int lv = 0;
-  uint64_t max_even = 0, max_odd = 0;
-  uint32_t chunk = CHUNK;  // level 0, then CHUNK_L
-  while (m > chunk) {
-    m = 2 * ((m + chunk - 1) / chunk);
-    chunk = CHUNK_L;
-    if (lv >= MAX_LEVELS - 1) return false;
-    L->level_max[lv] = (uint32_t)m;
-    if (lv % 2 == 0) max_even = m > max_even ? m : max_even;
-    else max_odd = m > max_odd ? m : max_odd;
-    lv++;
-  }
-  L->levels = lv;
-  if (max_even < 2) max_even = 2;
-  if (max_odd < 2) max_odd = 2;
+  L->share = share_for(L->n_entries_max);
+  L->chunks_max = (uint32_t)((L->n_entries_max + L->share.ch - 1) / L->share.ch);
   // reduction level sizes (halving down to RED_TAIL items per window)
   uint32_t M = cfg.buckets;
   int rl = 0;
@@ -1038,13 +1369,12 @@ static bool make_layout(const Config& cfg, uint64_t len, Layout* L, uint32_t set
     L->slices = off; off = align256(off + ((size_t)L->sp.nc + 1) * 4);
     L->max_slices = (uint32_t)((L->n_entries_max + SEG_SLICE - 1) / SEG_SLICE) + L->sp.nc;
   }
-  L->counts = off; off = align256(off + MAX_LEVELS * 4 * 2);
+  L->counts = off; off = align256(off + 2 * 4);
   L->keys0 = off; off = align256(off + L->n_entries_max * 4);
   L->vals0 = off; off = align256(off + L->n_entries_max * 4);
-  L->lvl_keys[0] = off; off = align256(off + max_even * 4);
-  L->lvl_pts[0] = off; off = align256(off + max_even * 128);
-  L->lvl_keys[1] = off; off = align256(off + max_odd * 4);
-  L->lvl_pts[1] = off; off = align256(off + max_odd * 128);
+  L->pieces = off; off = align256(off + (size_t)L->chunks_max * 2 * 128);
+  L->seg_meta = off; off = align256(off + (size_t)LONG_TILES * 3 * 4);
+  L->seg_pts = off; off = align256(off + (size_t)LONG_TILES * 2 * 128);
   L->bucket_bytes = align256((size_t)L->H * 128);
   L->buckets = off; off += L->bucket_bytes * sets;
   // reduction ping-pong: X and Y for even / odd levels
@@ -1142,29 +1472,32 @@ static hipError_t sort_part(const Config& cfg, const Layout& L, char* ws, const 
     uint32_t* matrix = reinterpret_cast<uint32_t*>(ws + L.matrix);
     uint32_t* ktmp = reinterpret_cast<uint32_t*>(ws + L.keys_tmp);
     uint32_t* vtmp = reinterpret_cast<uint32_t*>(ws + L.vals_tmp);
+    const uint32_t nbk = 1u << sp.low_bits;
+    uint32_t* slices = reinterpret_cast<uint32_t*>(ws + L.slices);
     pt.mark("start");
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(THREADS), 0, stream, matrix + (mn - 1), (uint64_t)1);
-    hipLaunchKernelGGL(k_part_count, dim3(sp.tiles), dim3(THREADS), sp.nc * 4, stream, d_scalars, len, cfg, sp, matrix);
+    hipLaunchKernelGGL(k_part_count, dim3(sp.tiles), dim3(THREADS), sp.nc * 4, stream, d_scalars, len, cfg, sp, matrix,
+                       cursor);
     ZKP_CHECK(hipGetLastError());
     pt.mark("count");
-    const uint32_t nbm = div_ceil32(mn, SCAN_BLOCK);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(nbm), dim3(THREADS), 0, stream, matrix, (uint32_t)mn, bsums);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(THREADS), 0, stream, bsums, nbm);
-    hipLaunchKernelGGL(k_scan_add, dim3(div_ceil32(mn, THREADS)), dim3(THREADS), 0, stream, matrix, (uint32_t)mn, bsums,
-                       nullptr);
-    hipLaunchKernelGGL(k_set_count, dim3(1), dim3(64), 0, stream, counts, matrix, (uint32_t)(mn - 1));
+    if (mn <= SCAN_SMALL_MAX) {
+      hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(SCAN_SMALL_THREADS), (sp.nc + 1) * 4, stream, matrix,
+                         (uint32_t)mn, sp, slices, counts);
+    } else {
+      const uint32_t nbm = div_ceil32(mn, SCAN_BLOCK);
+      hipLaunchKernelGGL(k_scan_blocks, dim3(nbm), dim3(THREADS), 0, stream, matrix, (uint32_t)mn, bsums);
+      hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(THREADS), 0, stream, bsums, nbm);
+      hipLaunchKernelGGL(k_scan_add, dim3(div_ceil32(mn, THREADS)), dim3(THREADS), 0, stream, matrix, (uint32_t)mn,
+                         bsums, nullptr);
+      hipLaunchKernelGGL(k_seg_plan, dim3(1), dim3(THREADS), (sp.nc + 1) * 4, stream, matrix, sp, slices, counts);
+    }
     ZKP_CHECK(hipGetLastError());
     pt.mark("scan");
     hipLaunchKernelGGL(k_part_scatter, dim3(sp.tiles), dim3(THREADS), sp.lds_part, stream, d_scalars, len, cfg, sp,
                        matrix, ktmp, vtmp);
     ZKP_CHECK(hipGetLastError());
     pt.mark("partition");
-    const uint32_t nbk = 1u << sp.low_bits;
-    uint32_t* slices = reinterpret_cast<uint32_t*>(ws + L.slices);
-    hipLaunchKernelGGL(k_seg_plan, dim3(1), dim3(THREADS), (sp.nc + 1) * 4, stream, matrix, sp, slices);
-    hipLaunchKernelGGL(k_zero_u32, dim3(grid_for(L.H, 4096)), dim3(THREADS), 0, stream, cursor, (uint64_t)L.H);
     hipLaunchKernelGGL(k_seg_hist, dim3(L.max_slices), dim3(THREADS), nbk * 4, stream, ktmp, matrix, slices, sp, cursor);
-    hipLaunchKernelGGL(k_seg_scan, dim3(sp.nc), dim3(THREADS), nbk * 4, stream, matrix, sp, cursor);
+    hipLaunchKernelGGL(k_seg_scan, dim3(sp.nc), dim3(THREADS), nbk * 4, stream, matrix, slices, sp, cursor);
     const uint32_t lds_seg = seg_scatter_lds(sp.low_bits);
     hipLaunchKernelGGL(k_seg_scatter, dim3(L.max_slices), dim3(THREADS), lds_seg, stream, ktmp, vtmp, matrix, slices,
                        sp, cursor, keys0, vals0);
@@ -1192,63 +1525,58 @@ static hipError_t sort_part(const Config& cfg, const Layout& L, char* ws, const 
   return hipSuccess;
 }
 
+// Launches with at most this many point operations run a quad of lanes per
+// operation (their time is the operations' latency, not their count): a quad
+// adds in 2.5 us where a lone lane takes 5.6 us, but 65 536 quads already put
+// four waves on every SIMD.
+constexpr uint64_t QUAD_OPS = 65536;
+
 // Second half: adds the sorted entries' points (n_precompute tables laid out
 // table-major at d_points) into bucket set `set`.
-static hipError_t accumulate_sorted(const Config& cfg, const Layout& L, char* ws, uint32_t set, const u32* d_points,
-                                    bool fresh, hipStream_t stream, PhaseTimer& pt) {
+static hipError_t accumulate_sorted(const Layout& L, char* ws, uint32_t set, const u32* d_points,
+                                    hipStream_t stream, PhaseTimer& pt) {
   uint32_t* counts = reinterpret_cast<uint32_t*>(ws + L.counts);
   uint32_t* keys0 = reinterpret_cast<uint32_t*>(ws + L.keys0);
   uint32_t* vals0 = reinterpret_cast<uint32_t*>(ws + L.vals0);
+  u32* pieces = reinterpret_cast<u32*>(ws + L.pieces);
+  uint32_t* seg_meta = reinterpret_cast<uint32_t*>(ws + L.seg_meta);
+  u32* seg_pts = reinterpret_cast<u32*>(ws + L.seg_pts);
   u32* buckets = bucket_set(L, ws, set);
-  const uint64_t nchunks0 = (L.n_entries_max + CHUNK - 1) / CHUNK;
-  // with a single chunk every run is closed: no next level
-  uint32_t* nk = L.levels > 0 ? reinterpret_cast<uint32_t*>(ws + L.lvl_keys[0]) : nullptr;
-  u32* np = L.levels > 0 ? reinterpret_cast<u32*>(ws + L.lvl_pts[0]) : nullptr;
-  hipLaunchKernelGGL(k_accumulate0, dim3(grid_for(nchunks0, 1u << 30)), dim3(THREADS), 0, stream, keys0, vals0,
-                     d_points, counts, fresh, buckets, nk, np);
+  const uint32_t ch = L.share.ch;
+  if (L.share.quads)
+    hipLaunchKernelGGL(k_accumulate<true>, dim3(div_ceil32(4ull * L.chunks_max, THREADS)), dim3(THREADS), 0, stream,
+                       keys0, vals0, d_points, counts, ch, buckets, pieces);
+  else
+    hipLaunchKernelGGL(k_accumulate<false>, dim3(div_ceil32(L.chunks_max, THREADS)), dim3(THREADS), 0, stream, keys0,
+                       vals0, d_points, counts, ch, buckets, pieces);
   ZKP_CHECK(hipGetLastError());
-  pt.mark("accumulate0");
-  // level 1 chunked, then the short runs of level 2 closed directly; the later
-  // chunked levels only run when a long run remains.  A top window of few
-  // bits puts its digits in a handful of buckets (runs far above RUN_MAX), so
-  // then every level runs and the run pass is left out.
-  uint32_t* run_flag = counts + MAX_LEVELS;
-  const uint32_t top_bits = SCALAR_BITS - (cfg.actual_windows - 1) * cfg.s;
-  const bool close_runs = top_bits >= 10;
-  for (int lv = 0; lv < L.levels; lv++) {
-    const int cur = lv % 2, nxt = 1 - cur;
-    const bool last = lv == L.levels - 1;
-    const uint64_t nch = (L.level_max[lv] + CHUNK_L - 1) / CHUNK_L;
-    hipLaunchKernelGGL(k_accumulate, dim3(grid_for(nch, 1u << 30)), dim3(THREADS), 0, stream,
-                       reinterpret_cast<const uint32_t*>(ws + L.lvl_keys[cur]),
-                       reinterpret_cast<const u32*>(ws + L.lvl_pts[cur]), counts, (uint32_t)(lv + 1), fresh, buckets,
-                       last ? nullptr : reinterpret_cast<uint32_t*>(ws + L.lvl_keys[nxt]),
-                       last ? nullptr : reinterpret_cast<u32*>(ws + L.lvl_pts[nxt]),
-                       lv == 0 || !close_runs ? nullptr : run_flag);
+  pt.mark("accumulate");
+  if (L.chunks_max > 1) {
+    if (L.share.quads)
+      hipLaunchKernelGGL(k_close_runs<true>, dim3(div_ceil32(4ull * L.chunks_max, THREADS)), dim3(THREADS), 0, stream,
+                         keys0, pieces, counts, ch, buckets);
+    else
+      hipLaunchKernelGGL(k_close_runs<false>, dim3(div_ceil32(L.chunks_max, THREADS)), dim3(THREADS), 0, stream, keys0,
+                         pieces, counts, ch, buckets);
     ZKP_CHECK(hipGetLastError());
-    if (lv == 0 && !last && close_runs) {
-      hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(THREADS), 0, stream, run_flag, (uint64_t)1);
-      hipLaunchKernelGGL(k_close_runs, dim3(grid_for(L.level_max[1], 1u << 30)), dim3(THREADS), 0, stream,
-                         reinterpret_cast<const uint32_t*>(ws + L.lvl_keys[nxt]),
-                         reinterpret_cast<u32*>(ws + L.lvl_pts[nxt]), counts, 2u, fresh, buckets, run_flag);
-      ZKP_CHECK(hipGetLastError());
-    }
   }
-  pt.mark("levels");
+  if (L.chunks_max > RUN_MAX + 1) {
+    hipLaunchKernelGGL(k_long_tiles, dim3(LONG_TILES), dim3(THREADS), 0, stream, keys0, pieces, counts, ch, buckets,
+                       seg_meta, seg_pts);
+    hipLaunchKernelGGL(k_long_join, dim3(1), dim3(THREADS), 0, stream, counts, seg_meta, seg_pts, buckets);
+    ZKP_CHECK(hipGetLastError());
+  }
+  pt.mark("runs");
   return hipSuccess;
 }
 
 // Adds sum_i k_i P_i for one part (len points, n_precompute tables laid out
 // table-major at d_points) into bucket set `set`.
 static hipError_t accumulate_part(const Config& cfg, const Layout& L, char* ws, uint32_t set, const u32* d_points,
-                                  const u32* d_scalars, uint64_t len, bool fresh, hipStream_t stream, PhaseTimer& pt) {
+                                  const u32* d_scalars, uint64_t len, hipStream_t stream, PhaseTimer& pt) {
   ZKP_CHECK(sort_part(cfg, L, ws, d_scalars, len, stream, pt));
-  return accumulate_sorted(cfg, L, ws, set, d_points, fresh, stream, pt);
+  return accumulate_sorted(L, ws, set, d_points, stream, pt);
 }
-
-// Levels with at most this many point operations run a quad of lanes per
-// operation (their time is the operations' latency, not their count).
-constexpr uint64_t QUAD_LEVEL_OPS = 65536;
 
 // Reduction of bucket set `set`; the n_windows window sums end at *out_dev (XYZZ).
 static hipError_t reduce_buckets(const Config& cfg, const Layout& L, char* ws, uint32_t set, hipStream_t stream,
@@ -1258,38 +1586,44 @@ static hipError_t reduce_buckets(const Config& cfg, const Layout& L, char* ws, u
   uint32_t M = cfg.buckets;
   if (M < 2 || (M & (M - 1))) return hipErrorInvalidValue;  // 2^(s-1) buckets, s >= 2
   int rl0 = 0;
-  if (L.red_levels >= 2) {
-    // levels 0 and 1 in one pass, into level 1's buffers
+  uint32_t fold = cfg.top_log;  // levels that fold the top window's copies
+  // Levels 0 and 1 in one pass, into level 1's buffers, where its blocks are
+  // enough to occupy the chip: the pass is a chain of eight point operations
+  // (63 us however few blocks), the two levels by quads take 20-30 us up to
+  // 32 768 blocks.
+  if (L.red_levels >= 2 && (uint64_t)(M >> 2) * cfg.n_windows > QUAD_OPS / 2) {
     u32* Xo = reinterpret_cast<u32*>(ws + L.red[2]);
     u32* Yo = reinterpret_cast<u32*>(ws + L.red[3]);
     const uint32_t blocks = (M >> 2) * cfg.n_windows;
     hipLaunchKernelGGL(k_reduce_block4, dim3(div_ceil32(blocks, THREADS)), dim3(THREADS), 0, stream, X, M,
-                       cfg.n_windows, Xo, Yo);
+                       cfg.n_windows, fold, Xo, Yo);
     ZKP_CHECK(hipGetLastError());
     X = Xo;
     Y = Yo;
     M >>= 2;
     rl0 = 2;
+    fold -= fold < 2 ? fold : 2;
   }
   for (int rl = rl0; rl < L.red_levels; rl++) {
     u32* Xo = reinterpret_cast<u32*>(ws + L.red[(rl % 2) * 2]);
     u32* Yo = reinterpret_cast<u32*>(ws + L.red[(rl % 2) * 2 + 1]);
     const uint32_t Mo = L.red_m[rl];
     const uint64_t ops = 2ull * Mo * cfg.n_windows;
-    if (ops <= QUAD_LEVEL_OPS)
+    if (ops <= QUAD_OPS || rl0 == 0)
       hipLaunchKernelGGL(k_reduce_level_quad, dim3(div_ceil32(4 * ops, THREADS)), dim3(THREADS), 0, stream, X, Y, M,
-                         cfg.n_windows, rl == 0, Xo, Yo);
+                         cfg.n_windows, rl == 0, fold > 0, Xo, Yo);
     else
       hipLaunchKernelGGL(k_reduce_level, dim3(div_ceil32(ops, THREADS)), dim3(THREADS), 0, stream, X, Y, M,
-                         cfg.n_windows, rl == 0, Xo, Yo);
+                         cfg.n_windows, rl == 0, fold > 0, Xo, Yo);
     ZKP_CHECK(hipGetLastError());
     X = Xo;
     Y = Yo;
     M = Mo;
+    fold -= fold > 0 ? 1 : 0;
   }
   u32* sums = reinterpret_cast<u32*>(ws + L.sums);
   hipLaunchKernelGGL(k_reduce_tail_quad, dim3(cfg.n_windows), dim3(QUAD_TAIL_THREADS), 0, stream, X, Y, M,
-                     L.red_levels == 0, sums);
+                     L.red_levels == 0, fold, sums);
   ZKP_CHECK(hipGetLastError());
   *out_dev = sums;
   pt.mark("reduce");
@@ -1319,7 +1653,7 @@ static hipError_t msm_device(const Config& cfg, const u32* d_points, const u32* 
                              const Layout& L, hipStream_t stream, G1XYZZ* result, bool debug) {
   PhaseTimer pt{debug, stream, {}, {}};
   ZKP_CHECK(reset_buckets(cfg, L, ws, 0, stream));
-  if (len > 0) ZKP_CHECK(accumulate_part(cfg, L, ws, 0, d_points, d_scalars, len, true, stream, pt));
+  if (len > 0) ZKP_CHECK(accumulate_part(cfg, L, ws, 0, d_points, d_scalars, len, stream, pt));
   const u32* d_sums = nullptr;
   ZKP_CHECK(reduce_buckets(cfg, L, ws, 0, stream, &d_sums, pt));
   std::vector<G1XYZZ> sums;
@@ -1558,10 +1892,10 @@ static hipError_t msm_card(const Config& cfg, const HostPlan& P, unsigned card, 
         ZKP_CHECK(hipEventRecord(R.sc_free[ss], R.s));
         if (j == 0) ZKP_CHECK(hipStreamWaitEvent(R.s, R.pt_ready[st], 0));
         if (idx == 0 || P.scratch_set == UINT32_MAX) {
-          ZKP_CHECK(accumulate_sorted(cfg, L, ws, j, pts((uint32_t)st), idx == 0, R.s, pt));
+          ZKP_CHECK(accumulate_sorted(L, ws, j, pts((uint32_t)st), R.s, pt));
         } else {
           ZKP_CHECK(reset_buckets(cfg, L, ws, P.scratch_set, R.s));
-          ZKP_CHECK(accumulate_sorted(cfg, L, ws, P.scratch_set, pts((uint32_t)st), true, R.s, pt));
+          ZKP_CHECK(accumulate_sorted(L, ws, P.scratch_set, pts((uint32_t)st), R.s, pt));
           hipLaunchKernelGGL(k_merge_buckets, dim3(div_ceil32(L.H, THREADS)), dim3(THREADS), 0, R.s,
                              bucket_set(L, ws, j), bucket_set(L, ws, P.scratch_set), L.H);
           ZKP_CHECK(hipGetLastError());
@@ -1749,7 +2083,7 @@ hipError_t zkp_msm_device_enqueue(const unsigned int* d_points, const unsigned i
   char* ws = reinterpret_cast<char*>(d_workspace);
   PhaseTimer pt{false, stream, {}, {}};
   ZKP_CHECK(reset_buckets(cfg, L, ws, 0, stream));
-  if (len > 0) ZKP_CHECK(accumulate_part(cfg, L, ws, 0, d_points, d_scalars, len, true, stream, pt));
+  if (len > 0) ZKP_CHECK(accumulate_part(cfg, L, ws, 0, d_points, d_scalars, len, stream, pt));
   const u32* d_sums = nullptr;
   ZKP_CHECK(reduce_buckets(cfg, L, ws, 0, stream, &d_sums, pt));
   if (h_sums != nullptr)
