@@ -1,7 +1,7 @@
 // BN254 Fq in nine 29-bit limbs with Montgomery radix R' = 2^261: the
 // arithmetic of the MSM's buckets (host + device).  The limb layout and the
-// bounds are written for any modulus below 2^254 (F29<Params>); the NTT keeps
-// the 8 x 32-bit product of bn254.hpp (see the note on F29 below).
+// bounds are written for any modulus below 2^254 (F29<Params>).  The
+// transforms have their own signed form (fr29.hpp).
 //
 // Why 29 bits: a 29 x 29-bit limb product is below 2^58, so one column of the
 // product-scanning multiplication (at most nine a_i b_j and nine m_i p_j
@@ -45,10 +45,6 @@ struct Fq29Params {
                                   0x11b7bc3cu, 0x1cbd99bau, 0x183340fbu, 0x000e0a77u};  // 2^256 mod p
 };
 
-// The NTT's twiddle product was tried through this form too (x read as is, the
-// twiddle 5 bits up, the result packed back): 267 instructions against 295, but
-// 171 v_mad_u64_u32 against 136, and the 2^24 transform ran 2.21 ms against
-// 2.14 ms -- the multiply-adds, not the instruction count, set its pace.
 template <class Params>
 struct F29 {
   u32 l[9];

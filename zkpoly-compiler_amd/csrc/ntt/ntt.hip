@@ -25,11 +25,10 @@
 //    pairs with the next pair's loads in flight during the current stages.
 //  * dit_pass_r4: a workgroup loads a tile of 2^TILE_LOG elements -- 2^d
 //    butterfly-connected rows times 2^c adjacent columns, so every global
-//    access is a run of >= 2^c consecutive 32-byte elements -- into LDS (two
-//    16-byte planes), runs d consecutive stages there two at a time (radix-4
-//    register blocks), and writes it back.
-//    Between stages and passes values stay in [0, 4p) (lazy reduction); the
-//    last pass stores canonical values.
+//    access is a run of >= 2^c consecutive 32-byte elements -- and runs d
+//    consecutive stages on it two at a time (radix-4 register blocks) in
+//    signed 29-bit limbs (Fr29), through LDS between them.
+//    Passes hand on values below 1.0002 r; the last one stores canonical values.
 //    A transform of 2^24 is the head + 3 passes (7 + 6 + 6 stages), or
 //    + 2 passes (10 + 9) with min_col_log = 1.
 // The first version (bitrev_kernel + radix-2 dit_pass, 11 + 9 + 4 stages) is
@@ -43,6 +42,7 @@
 
 #include "../common/poly_ptr.hpp"
 #include "../field/bn254.hpp"
+#include "../field/fr29.hpp"
 
 namespace zkp {
 namespace ntt {
@@ -181,6 +181,17 @@ struct BatchInstance {
   uint32_t head_t;  // stages fused into the bit reversal (0: none)
   uint32_t head_g;  // the head's 2^head_g workgroups walk the tile pairs
 };
+
+// A pointer read out of a work list carries no address space, and loads
+// through it would be flat ones, which wait on the LDS counter too: it is made
+// anew from a kernel argument's pointer and the distance, kept opaque so that
+// the sum is not folded back.
+template <class P>
+__device__ __forceinline__ P* in_global(P* p, const BatchInstance* anchor) {
+  uint64_t d = (uint64_t)p - (uint64_t)anchor;
+  asm("" : "+v"(d));
+  return (P*)((char*)const_cast<BatchInstance*>(anchor) + d);
+}
 
 // Pass parameters of one instance in one round (d == 0: no pass this round);
 // pad != 0 marks the instance's last pass (canonical output).
@@ -650,8 +661,9 @@ __global__ void __launch_bounds__(HEAD_THREADS)
   const uint64_t b = blockIdx.x;
   if (b >= head_prefix[count]) return;
   const uint32_t k = find_instance(head_prefix, count, b);
-  const BatchInstance I = inst[k];
-  head_twiddles_from_table(L, I.tw, I.log_n, I.head_t);
+  BatchInstance I = inst[k];
+  I.v.ptr = in_global(I.v.ptr, inst);
+  head_twiddles_from_table(L, in_global(I.tw, inst), I.log_n, I.head_t);
   head_walk(L, I.v, I.log_n, I.head_t, I.head_g, b - head_prefix[k]);
 }
 
@@ -678,181 +690,179 @@ __device__ __forceinline__ TileGeom tile_geom(uint32_t s0, uint32_t d, uint32_t 
   return TileGeom{lo_block << c_log | (hi << (s0 + d)), 1, 1ull << s0};
 }
 
-// Element e of a tile: its LDS position (row k, column c -> k * C + c) and its
-// global index.  Consecutive e walk the contiguous direction in memory.
-__device__ __forceinline__ uint64_t tile_elem(const TileGeom& g, uint32_t d, uint32_t c_log, uint32_t e,
-                                              uint32_t& pos) {
-  uint32_t c, k;
-  if (g.cstride == 1) {
-    c = e & ((1u << c_log) - 1);
-    k = e >> c_log;
-  } else {
-    k = e & ((1u << d) - 1);
-    c = e >> d;
-  }
-  pos = (k << c_log) | c;
-  return tile_index(g.base, g.cstride, g.kstride, c, k);
+// A tile in LDS: limbs 0-3, 4-7 and 8 of its elements (Fr29), 72 KB.
+struct PassLds {
+  uint4 p0[1 << TILE_LOG], p1[1 << TILE_LOG];
+  int32_t p2[1 << TILE_LOG];
+};
+
+__device__ __forceinline__ Fr29 lds_get29(const PassLds& L, uint32_t p) {
+  const uint4 a = L.p0[p], b = L.p1[p];
+  return Fr29{{(int32_t)a.x, (int32_t)a.y, (int32_t)a.z, (int32_t)a.w, (int32_t)b.x, (int32_t)b.y, (int32_t)b.z,
+               (int32_t)b.w, L.p2[p]}};
+}
+__device__ __forceinline__ void lds_put29(PassLds& L, uint32_t p, const Fr29& x) {
+  L.p0[p] = make_uint4((u32)x.l[0], (u32)x.l[1], (u32)x.l[2], (u32)x.l[3]);
+  L.p1[p] = make_uint4((u32)x.l[4], (u32)x.l[5], (u32)x.l[6], (u32)x.l[7]);
+  L.p2[p] = x.l[8];
 }
 
-// Stages [s0, s0 + d) on the tile in LDS; ends with a barrier.  Butterflies are
-// lazy (Harvey): values stay in [0, 4p).  Stages go two at a time: a thread
-// owns quads of rows {k0, k0+h, k0+2h, k0+3h} (h = 2^m, bits m and m+1 of k0
-// clear), which stages m and m+1 connect only among themselves; stage m uses
-// one twiddle for both of its butterflies (k0 and k0+2h agree modulo 2^(s0+m)),
-// stage m+1 two.  Per LDS round trip a thread does 2 quads = 8 butterflies with
-// 4 independent products per stage; an odd last stage runs radix-2.
-template <int NT, int U>
-__device__ __forceinline__ void pass_stages(uint4* __restrict__ lds0, uint4* __restrict__ lds1,
-                                            const uint32_t* __restrict__ tw, uint32_t log_n, uint32_t s0, uint32_t d,
-                                            uint32_t c_log, const TileGeom& geo) {
+// Word offsets of N elements of the view, `step` apart from position `at`
+// (before the wrap) on; a view that does not wrap (uniform) only adds.
+template <int N>
+__device__ __forceinline__ void pass_rows(const PolyView& v, bool wraps, uint64_t at, uint64_t step,
+                                          uint64_t (&row)[N]) {
+  if (wraps) {
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+      uint64_t p = at + r * step;
+      if (p >= v.whole_len) p -= v.whole_len;
+      row[r] = p * 8;
+    }
+  } else {
+    row[0] = at * 8;
+#pragma unroll
+    for (int r = 1; r < N; r++) row[r] = row[r - 1] + step * 8;
+  }
+}
+// Reduced below 1.0002 r; the transform's last pass (final) stores canonical values.
+__device__ __forceinline__ void pass_store(uint32_t* dst, const Fr29& x, bool final_pass) {
+  Fr y;
+  x.reduce().to_words(y.v);
+  if (final_pass) y = Fr::reduce_once(y);
+  y.store(dst);
+}
+
+// One tile per workgroup: stages [s0, s0 + d) over 2^d rows x 2^c_log columns.
+// Stages go two at a time: thread g owns the quad of rows {k0, k0+h, k0+2h,
+// k0+3h} (h = 2^m, bits m and m+1 of k0 clear) of a column, which stages m and
+// m+1 connect only among themselves; stage m uses one twiddle for both of its
+// butterflies (k0 and k0+2h agree modulo 2^(s0+m)), stage m+1 two: with the
+// first at table entry e they are e / 2 and e / 2 + n / 4.  An odd last stage
+// runs radix-2.  The first round takes its rows from memory and the last one
+// writes them there, so a tile goes through LDS between rounds only; the next
+// round's first twiddle is on its way during a round's products.
+// Values are Fr29, carried only where a bound asks for it: the two operands of
+// a quad that are not factors of its first stage are normalised as they are
+// read, the other two go into their products as the last round left them.
+// A pass is bound by VALU issue.  At 2^24 it takes 5 600 instructions per wave
+// (ten stages) where 32-bit limbs took 7 000, 0.72 against 0.81 ms.
+constexpr int PASS_THREADS = 512;
+static_assert(4 * PASS_THREADS >= 1 << TILE_LOG, "a quad per thread");
+
+__device__ __forceinline__ void dit_tile_r4(PassLds& L, const PolyView& v, const uint32_t* __restrict__ tw,
+                                            uint32_t log_n, uint32_t s0, uint32_t d, uint32_t c_log, uint64_t tile,
+                                            bool final_pass) {
   const uint32_t C = 1u << c_log;
   const uint32_t T = (1u << d) << c_log;
+  const TileGeom geo = tile_geom(s0, d, c_log, tile);
+  const bool wraps = v.offset + v.len > v.whole_len;
+  const uint32_t c = threadIdx.x & (C - 1);
+  const uint32_t qr = threadIdx.x >> c_log;
+  const bool live = threadIdx.x < (T >> 2);
+  // this thread's column modulo 2^s0, the part of a twiddle's exponent that no row adds to
+  const uint64_t lo = (geo.base & ((1ull << s0) - 1)) + (s0 ? c : 0);
+  // words before the table entry of stage s0 + m for rows that are kk modulo 2^m
+  auto entry = [&](uint32_t m, uint32_t kk) -> uint64_t {
+    return (lo + ((uint64_t)kk << s0)) << (log_n - 1 - (s0 + m)) << 3;
+  };
   uint32_t m = 0;
+  Fr w1;
+  if (d > 1 && live) w1 = Fr::load(tw + entry(0, 0));
   for (; m + 1 < d; m += 2) {
-    const uint32_t s = s0 + m;
     const uint32_t h = 1u << m;
-    const uint64_t mask1 = (1ull << s) - 1, mask2 = (1ull << (s + 1)) - 1;
-    const uint32_t sh1 = log_n - 1 - s, sh2 = log_n - 2 - s;
-    const uint32_t quads = T >> 2;
-    for (uint32_t g0 = threadIdx.x; g0 < quads; g0 += U * NT) {
-      Fr x[U][4], w1[U], w2[U], w3[U];
-      uint32_t pos[U][4];
-      bool live[U];
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const uint32_t g = g0 + u * NT;
-        live[u] = g < quads;
-        const uint32_t gg = live[u] ? g : g0;
-        const uint32_t c = gg & (C - 1);
-        const uint32_t qr = gg >> c_log;
-        const uint32_t k0 = ((qr >> m) << (m + 2)) | (qr & (h - 1));
-        const uint64_t i0 = tile_index(geo.base, geo.cstride, geo.kstride, c, k0);
-        const uint64_t i1 = tile_index(geo.base, geo.cstride, geo.kstride, c, k0 + h);
-        w1[u] = Fr::load(tw + (((i0 & mask1) << sh1) << 3));
-        w2[u] = Fr::load(tw + (((i0 & mask2) << sh2) << 3));
-        w3[u] = Fr::load(tw + (((i1 & mask2) << sh2) << 3));
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          pos[u][r] = ((k0 + r * h) << c_log) | c;
-          x[u][r] = lds_get(lds0, lds1, pos[u][r]);
-        }
+    const bool from_memory = m == 0, to_memory = m + 2 == d;
+    if (live) {
+      const uint32_t kk = qr & (h - 1);
+      const uint32_t k0 = ((qr >> m) << (m + 2)) | kk;
+      const uint32_t* tw2 = tw + (entry(m, kk) >> 1);
+      const Fr w2 = Fr::load(tw2), w3 = Fr::load(tw2 + (2ull << log_n));
+      const Fr29 v1 = Fr29::from_words<5>(w1.v);
+      if (m + 3 < d) w1 = Fr::load(tw + entry(m + 2, qr & (4 * h - 1)));
+      const uint64_t at = v.offset + tile_index(geo.base, geo.cstride, geo.kstride, c, k0);
+      const uint32_t pos = (k0 << c_log) | c;
+      Fr29 x0, x1, x2, x3;
+      if (from_memory) {
+        uint64_t row[4];
+        pass_rows(v, wraps, at, geo.kstride << m, row);
+        const Fr y0 = Fr::load(v.ptr + row[0]), y1 = Fr::load(v.ptr + row[1]), y2 = Fr::load(v.ptr + row[2]), y3 = Fr::load(v.ptr + row[3]);
+        x0 = Fr29::from_words<0>(y0.v);
+        x1 = Fr29::from_words<0>(y1.v);
+        x2 = Fr29::from_words<0>(y2.v);
+        x3 = Fr29::from_words<0>(y3.v);
+      } else {
+        x0 = lds_get29(L, pos).norm();
+        x1 = lds_get29(L, pos + (h << c_log));
+        x2 = lds_get29(L, pos + (2 * h << c_log)).norm();
+        x3 = lds_get29(L, pos + (3 * h << c_log));
       }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        Fr t1, t3, t2, t4;
-        Fr::mul_lazy2(x[u][1], w1[u], x[u][3], w1[u], t1, t3);
-        const Fr x0 = Fr::reduce_2p(x[u][0]), x2 = Fr::reduce_2p(x[u][2]);
-        const Fr a0 = Fr::add_raw(x0, t1), a1 = Fr::sub_2p(x0, t1);
-        const Fr a2 = Fr::add_raw(x2, t3), a3 = Fr::sub_2p(x2, t3);
-        Fr::mul_lazy2(a2, w2[u], a3, w3[u], t2, t4);
-        const Fr a0n = Fr::reduce_2p(a0), a1n = Fr::reduce_2p(a1);
-        x[u][0] = Fr::add_raw(a0n, t2);
-        x[u][2] = Fr::sub_2p(a0n, t2);
-        x[u][1] = Fr::add_raw(a1n, t4);
-        x[u][3] = Fr::sub_2p(a1n, t4);
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        if (!live[u]) continue;
-#pragma unroll
-        for (int r = 0; r < 4; r++) lds_put(lds0, lds1, pos[u][r], x[u][r]);
+      const Fr29 t1 = Fr29::mul(x1, v1), t3 = Fr29::mul(x3, v1);
+      const Fr29 t2 = Fr29::mul(x2 + t3, Fr29::from_words<5>(w2.v));
+      const Fr29 t4 = Fr29::mul(x2 - t3, Fr29::from_words<5>(w3.v));
+      const Fr29 a0 = x0 + t1, a1 = x0 - t1;
+      if (to_memory) {
+        uint64_t row[4];
+        pass_rows(v, wraps, at, geo.kstride << m, row);
+        pass_store(v.ptr + row[0], a0 + t2, final_pass);
+        pass_store(v.ptr + row[1], a1 + t4, final_pass);
+        pass_store(v.ptr + row[2], a0 - t2, final_pass);
+        pass_store(v.ptr + row[3], a1 - t4, final_pass);
+      } else {
+        lds_put29(L, pos, a0 + t2);
+        lds_put29(L, pos + (h << c_log), a1 + t4);
+        lds_put29(L, pos + (2 * h << c_log), a0 - t2);
+        lds_put29(L, pos + (3 * h << c_log), a1 - t4);
       }
     }
-    __syncthreads();
+    if (!to_memory) __syncthreads();
   }
   if (m < d) {  // odd last stage, radix-2
-    const uint32_t s = s0 + m;
     const uint32_t half = 1u << m;
-    const uint64_t jmask = (1ull << s) - 1;
-    const uint32_t tw_shift = log_n - 1 - s;
-    for (uint32_t b = threadIdx.x; b < (T >> 1); b += NT) {
-      const uint32_t c = b & (C - 1);
-      const uint32_t q = b >> c_log;
-      const uint32_t ka = ((q >> m) << (m + 1)) | (q & (half - 1));
-      const uint32_t pa = (ka << c_log) | c;
-      const uint32_t pb = ((ka + half) << c_log) | c;
-      const Fr w = Fr::load(tw + (((tile_index(geo.base, geo.cstride, geo.kstride, c, ka) & jmask) << tw_shift) << 3));
-      const Fr x = Fr::reduce_2p(lds_get(lds0, lds1, pa));
-      const Fr t = Fr::mul_lazy(lds_get(lds0, lds1, pb), w);
-      lds_put(lds0, lds1, pa, Fr::add_raw(x, t));
-      lds_put(lds0, lds1, pb, Fr::sub_2p(x, t));
-    }
-    __syncthreads();
-  }
-}
-
-// The tile back to memory; the transform's last pass (final) stores
-// canonical values.
-template <int NT>
-__device__ __forceinline__ void pass_store(const uint4* __restrict__ lds0, const uint4* __restrict__ lds1,
-                                           const PolyView& v, const TileGeom& geo, uint32_t d, uint32_t c_log,
-                                           bool final_pass) {
-  const uint32_t T = 1u << (d + c_log);
-  for (uint32_t e = threadIdx.x; e < T; e += NT) {
-    uint32_t pos;
-    uint4* dst = reinterpret_cast<uint4*>(v.elem(tile_elem(geo, d, c_log, e, pos)));
-    if (final_pass) {
-      const Fr y = Fr::reduce_4p(lds_get(lds0, lds1, pos));
-      dst[0] = make_uint4(y.v[0], y.v[1], y.v[2], y.v[3]);
-      dst[1] = make_uint4(y.v[4], y.v[5], y.v[6], y.v[7]);
-    } else {
-      dst[0] = lds0[pos];
-      dst[1] = lds1[pos];
+    for (uint32_t b = threadIdx.x; b < (T >> 1); b += PASS_THREADS) {
+      const uint32_t q = b >> c_log;  // (b and threadIdx.x agree modulo C)
+      const uint32_t kk = q & (half - 1);
+      const uint32_t ka = ((q >> m) << (m + 1)) | kk;
+      const uint32_t pos = (ka << c_log) | c;
+      const Fr w = Fr::load(tw + entry(m, kk));
+      uint64_t row[2];
+      pass_rows(v, wraps, v.offset + tile_index(geo.base, geo.cstride, geo.kstride, c, ka), geo.kstride << m, row);
+      Fr29 x, y;  // from LDS in (-2N, 3N): x + t and x - t still fit 32 bits
+      if (m == 0) {
+        const Fr a = Fr::load(v.ptr + row[0]), b2 = Fr::load(v.ptr + row[1]);
+        x = Fr29::from_words<0>(a.v);
+        y = Fr29::from_words<0>(b2.v);
+      } else {
+        x = lds_get29(L, pos);
+        y = lds_get29(L, pos + (half << c_log));
+      }
+      const Fr29 t = Fr29::mul(y, Fr29::from_words<5>(w.v));
+      pass_store(v.ptr + row[0], x + t, final_pass);
+      pass_store(v.ptr + row[1], x - t, final_pass);
     }
   }
 }
 
-// One tile per workgroup of NT threads (U quads per thread per round trip):
-// load, stages, store.
-template <int NT, int U>
-__device__ __forceinline__ void dit_tile_r4(uint4* __restrict__ lds0, uint4* __restrict__ lds1, const PolyView& v,
-                                            const uint32_t* __restrict__ tw, uint32_t log_n, uint32_t s0, uint32_t d,
-                                            uint32_t c_log, uint64_t tile, bool final_pass) {
-  const uint32_t T = 1u << (d + c_log);
-  const TileGeom geo = tile_geom(s0, d, c_log, tile);
-  for (uint32_t e = threadIdx.x; e < T; e += NT) {
-    uint32_t pos;
-    const uint4* src = reinterpret_cast<const uint4*>(v.elem(tile_elem(geo, d, c_log, e, pos)));
-    lds0[pos] = src[0];
-    lds1[pos] = src[1];
-  }
-  __syncthreads();
-  pass_stages<NT, U>(lds0, lds1, tw, log_n, s0, d, c_log, geo);
-  pass_store<NT>(lds0, lds1, v, geo, d, c_log, final_pass);
-}
-
-// Passes run 512 threads per workgroup, one quad per thread per round trip:
-// with two workgroups per CU (64 KB of LDS each) that is four waves per SIMD in
-// at most 128 VGPRs, whose issue covers the waits (barriers, tile loads) that
-// two waves left exposed (2^24: 2.34 -> 2.18 ms).
-constexpr int PASS_THREADS = 512;
+// 512 threads per workgroup, a quad each: with two workgroups per CU (72 KB of
+// LDS each) that is four waves per SIMD in at most 128 VGPRs, whose issue covers
+// the waits (barriers, tile loads) that two waves left exposed.
 __global__ void __launch_bounds__(PASS_THREADS)
     dit_pass_r4(PolyView v, const uint32_t* __restrict__ tw, uint32_t log_n, uint32_t s0, uint32_t d, uint32_t c_log,
                 uint32_t final_pass) {
-  __shared__ uint4 lds0[1 << TILE_LOG];
-  __shared__ uint4 lds1[1 << TILE_LOG];
-  dit_tile_r4<PASS_THREADS, 1>(lds0, lds1, v, tw, log_n, s0, d, c_log, blockIdx.x, final_pass != 0);
-}
-
-// The earlier shape: 256 threads, two quads each per round trip (variant 3).
-__global__ void __launch_bounds__(THREADS)
-    dit_pass_r4_narrow(PolyView v, const uint32_t* __restrict__ tw, uint32_t log_n, uint32_t s0, uint32_t d,
-                       uint32_t c_log, uint32_t final_pass) {
-  __shared__ uint4 lds0[1 << TILE_LOG];
-  __shared__ uint4 lds1[1 << TILE_LOG];
-  dit_tile_r4<THREADS, 2>(lds0, lds1, v, tw, log_n, s0, d, c_log, blockIdx.x, final_pass != 0);
+  __shared__ PassLds L;
+  dit_tile_r4(L, v, tw, log_n, s0, d, c_log, blockIdx.x, final_pass != 0);
 }
 
 __global__ void __launch_bounds__(PASS_THREADS)
     dit_pass_r4_batched(const BatchInstance* __restrict__ inst, const BatchPass* __restrict__ pass,
                         const uint64_t* __restrict__ tile_prefix, uint32_t count) {
-  __shared__ uint4 lds0[1 << TILE_LOG];
-  __shared__ uint4 lds1[1 << TILE_LOG];
+  __shared__ PassLds L;
   const uint64_t b = blockIdx.x;
   if (b >= tile_prefix[count]) return;
   const uint32_t k = find_instance(tile_prefix, count, b);
   const BatchPass p = pass[k];
-  dit_tile_r4<PASS_THREADS, 1>(lds0, lds1, inst[k].v, inst[k].tw, inst[k].log_n, p.s0, p.d, p.c_log,
+  BatchInstance I = inst[k];
+  I.v.ptr = in_global(I.v.ptr, inst);
+  dit_tile_r4(L, I.v, in_global(I.tw, inst), I.log_n, p.s0, p.d, p.c_log,
                                b - tile_prefix[k], p.pad != 0);
 }
 
@@ -1091,8 +1101,8 @@ struct PlanV2 {
 static std::atomic<uint32_t> g_min_col_log[41] = {1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1,
                                                   1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1};
 // 0: persistent head + radix-4 passes; 1: plain bit reversal + radix-2 passes;
-// 2: as 0 with one tile pair per head workgroup; 3: as 0 with 256-thread
-// passes (batch plans treat 2 and 3 as 0)
+// 2: as 0 with one tile pair per head workgroup (batch plans treat it as 0);
+// 3: as 0 (it once chose 256-thread passes)
 static std::atomic<int> g_variant{0};
 
 static void plan_v2(uint32_t log_n, PlanV2* p) {
@@ -1210,12 +1220,8 @@ static hipError_t launch_ntt(PolyPtr x, const unsigned int* twiddle, unsigned in
     if ((err = hipGetLastError()) != hipSuccess || (err = mark(0)) != hipSuccess) return err;
     for (int p = 0; p < plan.np; p++) {
       const PassPlan& pp = plan.pass[p];
-      if (variant == 3)
-        hipLaunchKernelGGL(dit_pass_r4_narrow, dim3((unsigned)pp.tiles), dim3(THREADS), 0, stream, v, twiddle,
-                           (uint32_t)log_len, pp.s0, pp.d, pp.c_log, (uint32_t)(p + 1 == plan.np));
-      else
-        hipLaunchKernelGGL(dit_pass_r4, dim3((unsigned)pp.tiles), dim3(PASS_THREADS), 0, stream, v, twiddle,
-                           (uint32_t)log_len, pp.s0, pp.d, pp.c_log, (uint32_t)(p + 1 == plan.np));
+      hipLaunchKernelGGL(dit_pass_r4, dim3((unsigned)pp.tiles), dim3(PASS_THREADS), 0, stream, v, twiddle,
+                         (uint32_t)log_len, pp.s0, pp.d, pp.c_log, (uint32_t)(p + 1 == plan.np));
       if ((err = hipGetLastError()) != hipSuccess || (err = mark(1)) != hipSuccess) return err;
     }
   }
