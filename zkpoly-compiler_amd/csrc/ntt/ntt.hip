@@ -306,16 +306,48 @@ __device__ __forceinline__ void lds_put(uint4* l0, uint4* l1, uint32_t p, const 
 constexpr uint32_t HEAD_BUF = HEAD_W * HEAD_PITCH;  // one 32 x 33 tile plane
 
 // Two tile buffers per plane (x at M at offset 0, x at rev M at HEAD_BUF) and
-// the head's twiddles r[i] = w^(i * 2^(log_n - t)), i < 2^(t - 1).  The second
-// plane starts 128 bytes into the LDS bank cycle relative to the first, so the
-// two lanes that move the two halves of one element hit different banks.
+// the head's twiddles r[i] = w^(i * 2^(log_n - t)), i < 2^(t - 1), as Fr29
+// multipliers.  Between memory and the first stage, and after the last one, an
+// element is its eight words in p0 and p1; between stages it is Fr29, limbs 0-3,
+// 4-7 and 8 in p0, p1 and p2.  The second plane starts 128 bytes into the LDS
+// bank cycle relative to the first, so the two lanes that move the two halves
+// of one element hit different banks.
 struct HeadLds {
   uint4 p0[2 * HEAD_BUF];
   uint4 pad[8];
   uint4 p1[2 * HEAD_BUF];
+  int32_t p2[2 * HEAD_BUF];
   uint4 r0[HEAD_W / 2], r1[HEAD_W / 2];
+  int32_t r2[HEAD_W / 2];
 };
 static_assert((2 * HEAD_BUF * 16 + 128) % 256 == 128, "planes half a bank cycle apart");
+static_assert(2 * sizeof(HeadLds) <= 160 * 1024, "two workgroups per CU");
+
+__device__ __forceinline__ Fr29 limbs_get(const uint4* p0, const uint4* p1, const int32_t* p2, uint32_t p) {
+  const uint4 a = p0[p], b = p1[p];
+  return Fr29{{(int32_t)a.x, (int32_t)a.y, (int32_t)a.z, (int32_t)a.w, (int32_t)b.x, (int32_t)b.y, (int32_t)b.z,
+               (int32_t)b.w, p2[p]}};
+}
+__device__ __forceinline__ void limbs_put(uint4* p0, uint4* p1, int32_t* p2, uint32_t p, const Fr29& x) {
+  p0[p] = make_uint4((u32)x.l[0], (u32)x.l[1], (u32)x.l[2], (u32)x.l[3]);
+  p1[p] = make_uint4((u32)x.l[4], (u32)x.l[5], (u32)x.l[6], (u32)x.l[7]);
+  p2[p] = x.l[8];
+}
+
+// An element of a tile before a round (`packed`: the first) and after it (the last).
+__device__ __forceinline__ Fr29 head_get(const HeadLds& L, uint32_t p, bool packed) {
+  if (!packed) return limbs_get(L.p0, L.p1, L.p2, p);
+  return Fr29::from_words<0>(lds_get(L.p0, L.p1, p).v);
+}
+__device__ __forceinline__ void head_put(HeadLds& L, uint32_t p, const Fr29& x, bool packed) {
+  if (!packed) {
+    limbs_put(L.p0, L.p1, L.p2, p, x);
+    return;
+  }
+  Fr y;
+  x.reduce().to_words(y.v);
+  lds_put(L.p0, L.p1, p, y);
+}
 
 // The head moves tiles between HBM and LDS as 16-byte halves of elements:
 // half h of a tile is plane (h & 1) of element h >> 1, and consecutive lanes
@@ -363,157 +395,102 @@ __device__ __forceinline__ void head_place(HeadLds& L, uint32_t t, bool pair, ui
 }
 
 // DIT stages 0..t-1 on the placed tile(s), through the transposed index map;
-// ends with a barrier.  LAZY keeps values in [0, 4p) (Harvey butterflies, as in
-// the passes), for callers whose later passes accept such inputs; otherwise
-// every stage output is canonical.
-template <bool LAZY, int NT>
+// ends with a barrier.  Stages go two at a time on quads of rows {k0, k0+h,
+// k0+2h, k0+3h} (bits m, m+1 of k0 clear) of one column, an odd last one
+// radix-2, in Fr29 as in the passes (dit_tile_r4); the results are below
+// 1.0002 r, for a pass that always follows.
+template <int NT>
 __device__ __forceinline__ void head_stages(HeadLds& L, uint32_t t, bool pair) {
-  constexpr int U = 512 / NT;   // quads per thread per round (radix-4 stages)
-  constexpr int R2 = 1024 / NT;  // butterflies per thread per round (radix-2 stage)
   const uint32_t W = 1u << t;
   // tile 0 = y at M (in the buffer of x at Mr), tile 1 = y at Mr (buffer of x at M)
   const uint32_t y0 = pair ? HEAD_BUF : 0;
-  const uint32_t per_tile = W * (W >> 1);
-  const uint32_t total = (pair ? 2 : 1) * per_tile;
+  auto root = [&](uint32_t i) { return limbs_get(L.r0, L.r1, L.r2, i); };
   // w^0 is 1 in every table built as powers; the product by it is skipped
   // only when the table holds exactly 1, so any other table is still honoured.
-  // The skip happens at stage 0 only, whose inputs are the caller's canonical
-  // values, so the lazy bounds below hold for the unmultiplied operand too.
-  const bool unit0 = lds_get(L.r0, L.r1, 0) == Fr::one();
-  // stages two at a time: quads of rows {k0, k0+h, k0+2h, k0+3h} (bits m, m+1
-  // of k0 clear) of one column, two quads per thread
+  // The skip happens in round 0 only, on the caller's canonical values.
+  bool unit0 = true;
+  {
+    constexpr u32 one[8] = {FrParams::ONE[0], FrParams::ONE[1], FrParams::ONE[2], FrParams::ONE[3],
+                            FrParams::ONE[4], FrParams::ONE[5], FrParams::ONE[6], FrParams::ONE[7]};
+    const Fr29 w0 = root(0), w1 = Fr29::from_words<5>(one);
+#pragma unroll
+    for (int i = 0; i < 9; i++) unit0 = unit0 && w0.l[i] == w1.l[i];
+  }
   uint32_t m = 0;
   for (; m + 1 < t; m += 2) {
     const uint32_t h = 1u << m;
-    const uint32_t per_tile_q = W * (W >> 2);
-    const uint32_t totq = (pair ? 2 : 1) * per_tile_q;
-    const bool skip1 = m == 0 && unit0;
-    for (uint32_t u0 = threadIdx.x; u0 < totq; u0 += U * NT) {
-      Fr x[U][4];
-      uint32_t pos[U][4], jw[U];
-      bool live[U];
+    const uint32_t per_tile = W * (W >> 2);
+    const uint32_t total = (pair ? 2 : 1) * per_tile;
+    const bool skip = m == 0 && unit0;
+    const bool in_words = m == 0, out_words = m + 2 == t;
+#pragma unroll 1
+    for (uint32_t u = threadIdx.x; u < total; u += NT) {
+      const uint32_t tile = u >= per_tile ? 1 : 0;
+      const uint32_t r = u - tile * per_tile;
+      // consecutive lanes take consecutive LDS columns ra (the W independent
+      // transforms of a tile are interchangeable), so a row's accesses hit
+      // distinct banks
+      const uint32_t ra = r & (W - 1);
+      const uint32_t q = r >> t;
+      const uint32_t k0 = ((q >> m) << (m + 2)) | (q & (h - 1));
+      const uint32_t off = (tile ? 0 : y0) + ra;
+      const uint32_t jw = k0 & (h - 1);
+      uint32_t pos[4];
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const uint32_t uq = u0 + u * NT;
-        live[u] = uq < totq;
-        const uint32_t uu = live[u] ? uq : u0;
-        const uint32_t tile = uu >= per_tile_q ? 1 : 0;
-        const uint32_t r = uu - tile * per_tile_q;
-        // consecutive lanes take consecutive LDS columns ra (the W independent
-        // transforms of a tile are interchangeable), so a row's accesses hit
-        // distinct banks
-        const uint32_t ra = r & (W - 1);
-        const uint32_t q = r >> t;
-        const uint32_t k0 = ((q >> m) << (m + 2)) | (q & (h - 1));
-        const uint32_t off = tile ? 0 : y0;
-        jw[u] = k0 & (h - 1);
-#pragma unroll
-        for (int r4 = 0; r4 < 4; r4++) {
-          pos[u][r4] = off + rev_bits(k0 + r4 * h, t) * HEAD_PITCH + ra;
-          x[u][r4] = lds_get(L.p0, L.p1, pos[u][r4]);
+      for (int i = 0; i < 4; i++) pos[i] = off + rev_bits(k0 + i * h, t) * HEAD_PITCH;
+      Fr29 x0 = head_get(L, pos[0], in_words), x1 = head_get(L, pos[1], in_words);
+      Fr29 x2 = head_get(L, pos[2], in_words), x3 = head_get(L, pos[3], in_words);
+      const Fr29 w3 = root((jw + h) << (t - 2 - m));
+      if (skip) {
+        // w^0 = 1 in both stages: one product; x0 + x1 + x2 + x3 has limbs up to 4 2^29
+        const Fr29 a0 = x0 + x1, a1 = x0 - x1, a2 = x2 + x3;
+        const Fr29 t4 = Fr29::mul(x2 - x3, w3);
+        x0 = (a0 + a2).norm();
+        x1 = a1 + t4;
+        x2 = a0 - a2;
+        x3 = a1 - t4;
+      } else {
+        const Fr29 w1 = root(jw << (t - 1 - m));
+        const Fr29 t1 = Fr29::mul(x1, w1), t3 = Fr29::mul(x3, w1);
+        if (!in_words) {
+          x0 = x0.norm();
+          x2 = x2.norm();
         }
+        const Fr29 t2 = Fr29::mul(x2 + t3, root(jw << (t - 2 - m)));
+        const Fr29 t4 = Fr29::mul(x2 - t3, w3);
+        const Fr29 a0 = x0 + t1, a1 = x0 - t1;
+        x0 = a0 + t2;
+        x1 = a1 + t4;
+        x2 = a0 - t2;
+        x3 = a1 - t4;
       }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        Fr t1 = x[u][1], t3 = x[u][3];
-        const Fr w2 = lds_get(L.r0, L.r1, jw[u] << (t - 2 - m));
-        const Fr w3 = lds_get(L.r0, L.r1, (jw[u] + h) << (t - 2 - m));
-        if (LAZY) {
-          if (!skip1) {
-            const Fr w1 = lds_get(L.r0, L.r1, jw[u] << (t - 1 - m));
-            t1 = Fr::mul_lazy(x[u][1], w1);
-            t3 = Fr::mul_lazy(x[u][3], w1);
-          }
-          const Fr x0 = Fr::reduce_2p(x[u][0]), x2 = Fr::reduce_2p(x[u][2]);
-          const Fr a0 = Fr::add_raw(x0, t1), a1 = Fr::sub_2p(x0, t1);
-          const Fr a2 = Fr::add_raw(x2, t3), a3 = Fr::sub_2p(x2, t3);
-          // at m = 0 the second stage's first twiddle is w^0 too: a reduction instead of a product
-          Fr t2;
-          if (skip1)
-            t2 = Fr::reduce_2p(a2);
-          else
-            t2 = Fr::mul_lazy(a2, w2);
-          const Fr t4 = Fr::mul_lazy(a3, w3);
-          const Fr a0n = Fr::reduce_2p(a0), a1n = Fr::reduce_2p(a1);
-          x[u][0] = Fr::add_raw(a0n, t2);
-          x[u][2] = Fr::sub_2p(a0n, t2);
-          x[u][1] = Fr::add_raw(a1n, t4);
-          x[u][3] = Fr::sub_2p(a1n, t4);
-        } else {
-          if (!skip1) {
-            const Fr w1 = lds_get(L.r0, L.r1, jw[u] << (t - 1 - m));
-            t1 = t1 * w1;
-            t3 = t3 * w1;
-          }
-          const Fr a0 = x[u][0] + t1, a1 = x[u][0] - t1;
-          const Fr a2 = x[u][2] + t3, a3 = x[u][2] - t3;
-          Fr t2 = a2;
-          if (!skip1) t2 = a2 * w2;
-          const Fr t4 = a3 * w3;
-          x[u][0] = a0 + t2;
-          x[u][2] = a0 - t2;
-          x[u][1] = a1 + t4;
-          x[u][3] = a1 - t4;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        if (!live[u]) continue;
-#pragma unroll
-        for (int r4 = 0; r4 < 4; r4++) lds_put(L.p0, L.p1, pos[u][r4], x[u][r4]);
-      }
+      head_put(L, pos[0], x0, out_words);
+      head_put(L, pos[1], x1, out_words);
+      head_put(L, pos[2], x2, out_words);
+      head_put(L, pos[3], x3, out_words);
     }
     __syncthreads();
   }
   if (m < t) {  // odd last stage, radix-2
     const uint32_t half = 1u << m;
+    const uint32_t per_tile = W * (W >> 1);
+    const uint32_t total = (pair ? 2 : 1) * per_tile;
     const bool skip = m == 0 && unit0;
-    for (uint32_t u0 = threadIdx.x; u0 < total; u0 += R2 * NT) {
-      Fr x[R2], y[R2];
-      uint32_t pa[R2], pb[R2], wi[R2];
-      bool live[R2];
-#pragma unroll
-      for (int j = 0; j < R2; j++) {
-        const uint32_t u = u0 + j * NT;
-        live[j] = u < total;
-        const uint32_t uu = live[j] ? u : u0;
-        const uint32_t tile = uu >= per_tile ? 1 : 0;
-        const uint32_t r = uu - tile * per_tile;
-        const uint32_t ra = r & (W - 1);  // consecutive lanes, consecutive LDS columns
-        const uint32_t q = r >> t;
-        const uint32_t blo = ((q >> m) << (m + 1)) | (q & (half - 1));
-        const uint32_t off = tile ? 0 : y0;
-        pa[j] = off + rev_bits(blo, t) * HEAD_PITCH + ra;
-        pb[j] = off + rev_bits(blo + half, t) * HEAD_PITCH + ra;
-        wi[j] = (blo & (half - 1)) << (t - 1 - m);
-        x[j] = lds_get(L.p0, L.p1, pa[j]);
-        y[j] = lds_get(L.p0, L.p1, pb[j]);
-      }
-      if (!skip) {
-#pragma unroll
-        for (int j = 0; j < R2; j++) {
-          const Fr w = lds_get(L.r0, L.r1, wi[j]);
-          y[j] = LAZY ? Fr::mul_lazy(y[j], w) : y[j] * w;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < R2; j++) {
-        const Fr tt = y[j];
-        if (LAZY) {
-          const Fr xr = Fr::reduce_2p(x[j]);
-          y[j] = Fr::sub_2p(xr, tt);
-          x[j] = Fr::add_raw(xr, tt);
-        } else {
-          y[j] = x[j] - tt;
-          x[j] = x[j] + tt;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < R2; j++) {
-        if (!live[j]) continue;
-        lds_put(L.p0, L.p1, pa[j], x[j]);
-        lds_put(L.p0, L.p1, pb[j], y[j]);
-      }
+#pragma unroll 1
+    for (uint32_t u = threadIdx.x; u < total; u += NT) {
+      const uint32_t tile = u >= per_tile ? 1 : 0;
+      const uint32_t r = u - tile * per_tile;
+      const uint32_t ra = r & (W - 1);  // consecutive lanes, consecutive LDS columns
+      const uint32_t q = r >> t;
+      const uint32_t blo = ((q >> m) << (m + 1)) | (q & (half - 1));
+      const uint32_t off = (tile ? 0 : y0) + ra;
+      const uint32_t pa = off + rev_bits(blo, t) * HEAD_PITCH;
+      const uint32_t pb = off + rev_bits(blo + half, t) * HEAD_PITCH;
+      const Fr29 x = head_get(L, pa, m == 0);
+      Fr29 y = head_get(L, pb, m == 0);
+      if (!skip) y = Fr29::mul(y, root((blo & (half - 1)) << (t - 1 - m)));
+      head_put(L, pa, x + y, true);
+      head_put(L, pb, x - y, true);
     }
     __syncthreads();
   }
@@ -539,7 +516,6 @@ __device__ __forceinline__ void head_store(const HeadLds& L, const PolyView& v, 
 // One tile pair {M, rev M} per workgroup.  The caller has written L.r
 // (visible after the first barrier below).
 // (256 threads.)
-template <bool LAZY>
 __device__ __forceinline__ void head_tile(HeadLds& L, const PolyView& v, uint32_t log_n, uint32_t t, uint64_t M) {
   const uint32_t mbits = log_n - 2 * t;
   const uint64_t Mr = mbits ? (__brevll(M) >> (64 - mbits)) : 0;
@@ -553,7 +529,7 @@ __device__ __forceinline__ void head_tile(HeadLds& L, const PolyView& v, uint32_
 #pragma unroll
   for (uint32_t j = 0; j < 8; j++) head_place<THREADS>(L, t, pair, j, g[j]);
   __syncthreads();
-  head_stages<LAZY, THREADS>(L, t, pair);
+  head_stages<THREADS>(L, t, pair);
   head_store<THREADS>(L, v, t, shift_a, M, Mr, pair);
 }
 
@@ -561,7 +537,8 @@ __device__ __forceinline__ void head_tile(HeadLds& L, const PolyView& v, uint32_
 __device__ __forceinline__ void head_twiddles_from_table(HeadLds& L, const uint32_t* __restrict__ tw, uint32_t log_n,
                                                          uint32_t t) {
   if (threadIdx.x < ((1u << t) >> 1))
-    lds_put(L.r0, L.r1, threadIdx.x, Fr::load(tw + (((uint64_t)threadIdx.x << (log_n - t)) << 3)));
+    limbs_put(L.r0, L.r1, L.r2, threadIdx.x,
+              Fr29::from_words<5>(Fr::load(tw + (((uint64_t)threadIdx.x << (log_n - t)) << 3)).v));
 }
 
 // Persistent head: 2^g workgroups (g <= mbits = log_n - 2t, mbits - g even)
@@ -575,8 +552,11 @@ __device__ __forceinline__ void head_twiddles_from_table(HeadLds& L, const uint3
 // is thus taken exactly once, and each workgroup gets the same number of pairs
 // up to 2^(h-1).  The loads of the next pair are issued before the stages of
 // the current one and land in registers while they run (barriers wait only for
-// LDS), so the tile traffic overlaps the butterflies.  The stages are lazy: a
-// radix-4 pass always follows the head and takes values in [0, 4p).
+// LDS), so the tile traffic overlaps the butterflies.  A radix-4 pass always
+// follows, so the head stores values below 1.0002 r.  In 29-bit limbs its stages
+// take 590 instructions an element where 32-bit limbs took 710; at 2^24 the
+// transform went from 1 907 to 1 848 us with that, and at 2^12 (one pair per
+// workgroup, a chain of products) from 38.7 to 35.0 us.
 // Workgroup b's walk (b < 2^g), HEAD_THREADS threads; the caller has written L.r.
 // (512 threads measured no faster: the staged loads of the next pair do not fit
 // the 128 VGPRs of four waves per SIMD and spill.)
@@ -619,7 +599,7 @@ __device__ __forceinline__ void head_walk(HeadLds& L, const PolyView& v, uint32_
     __syncthreads();
     const uint64_t kn = next(k + 1);
     if (kn < K) fetch(item(kn));
-    head_stages<true, HEAD_THREADS>(L, t, pair);
+    head_stages<HEAD_THREADS>(L, t, pair);
     head_store<HEAD_THREADS>(L, v, t, shift_a, M, Mr, pair);
     if (kn >= K) break;
     __syncthreads();  // the store phase has read the tiles before they are replaced
@@ -636,7 +616,7 @@ __global__ void __launch_bounds__(HEAD_THREADS)
 
 // Workgroup bits of bitrev_head_stream for mbits = log_n - 2t: at most
 // HEAD_STREAM_G_MAX (1024 workgroups, two rounds of the two per CU that the
-// 68 KB of LDS allows on 256 CUs), with mbits - g even.
+// 75 KB of LDS allows on 256 CUs), with mbits - g even.
 constexpr uint32_t HEAD_STREAM_G_MAX = 10;
 static inline uint32_t head_stream_g(uint32_t mbits) {
   uint32_t g = mbits < HEAD_STREAM_G_MAX ? mbits : HEAD_STREAM_G_MAX;
@@ -648,7 +628,7 @@ __global__ void __launch_bounds__(THREADS)
     bitrev_head(PolyView v, const uint32_t* __restrict__ tw, uint32_t log_n, uint32_t t) {
   __shared__ HeadLds L;
   head_twiddles_from_table(L, tw, log_n, t);
-  head_tile<true>(L, v, log_n, t, blockIdx.x);
+  head_tile(L, v, log_n, t, blockIdx.x);
 }
 
 // Fused bit reversal + first head_t stages of every instance; instance k owns
@@ -696,16 +676,8 @@ struct PassLds {
   int32_t p2[1 << TILE_LOG];
 };
 
-__device__ __forceinline__ Fr29 lds_get29(const PassLds& L, uint32_t p) {
-  const uint4 a = L.p0[p], b = L.p1[p];
-  return Fr29{{(int32_t)a.x, (int32_t)a.y, (int32_t)a.z, (int32_t)a.w, (int32_t)b.x, (int32_t)b.y, (int32_t)b.z,
-               (int32_t)b.w, L.p2[p]}};
-}
-__device__ __forceinline__ void lds_put29(PassLds& L, uint32_t p, const Fr29& x) {
-  L.p0[p] = make_uint4((u32)x.l[0], (u32)x.l[1], (u32)x.l[2], (u32)x.l[3]);
-  L.p1[p] = make_uint4((u32)x.l[4], (u32)x.l[5], (u32)x.l[6], (u32)x.l[7]);
-  L.p2[p] = x.l[8];
-}
+__device__ __forceinline__ Fr29 lds_get29(const PassLds& L, uint32_t p) { return limbs_get(L.p0, L.p1, L.p2, p); }
+__device__ __forceinline__ void lds_put29(PassLds& L, uint32_t p, const Fr29& x) { limbs_put(L.p0, L.p1, L.p2, p, x); }
 
 // Word offsets of N elements of the view, `step` apart from position `at`
 // (before the wrap) on; a view that does not wrap (uniform) only adds.
@@ -928,6 +900,8 @@ __global__ void __launch_bounds__(HEAD_THREADS)
                         const uint32_t* __restrict__ omegas, uint32_t log_n, uint32_t t, uint32_t g) {
   __shared__ HeadLds L;
   build_small_roots(L.r0, L.r1, pq, pq_deg, omegas, log_n, t);
+  if (threadIdx.x < ((1u << t) >> 1))
+    limbs_put(L.r0, L.r1, L.r2, threadIdx.x, Fr29::from_words<5>(lds_get(L.r0, L.r1, threadIdx.x).v));
   head_walk(L, v, log_n, t, g, blockIdx.x);
 }
 
