@@ -1,7 +1,10 @@
 // Host driver for tests/test_fr29_cpu.py: runs Fr29 (the transforms' signed
 // 29-bit limbs) on the CPU.  Built with hipcc as host code.
 //
-// Input: "chain A B N" and N lines "W" (canonical x 2^256 mod r, 64 hex digits).
+// Input:
+// "inv A" prints the inverse of the element A (x 2^256 -> x^-1 2^256) by both of
+// inverse()'s constants, plain and up.
+// "chain A B N" and N lines "W" (canonical x 2^256 mod r, 64 hex digits).
 // Step i takes the butterfly (a, b) -> (a + b W_i, a - b W_i) with the factor b
 // as the step before left it and a normalised every second step only, as a quad
 // of a pass does, and swaps the two on odd i.  Output per step: both values
@@ -39,8 +42,18 @@ static bool in_bounds(const Fr29& a) {
 int main() {
   char sa[128], sb[128];
   int n;
-  while (scanf(" chain %127s %127s %d", sa, sb, &n) == 3) {
+  char op[16];
+  while (scanf(" %15s", op) == 1) {
     u32 w[8];
+    if (strcmp(op, "inv") == 0) {
+      if (scanf(" %127s", sa) != 1 || !read_hex(sa, w)) return 2;
+      print_reduced(Fr29Inverse::inverse(Fr29::from_words<0>(w), Fr29Inverse::INV_PLAIN));
+      printf(" ");
+      print_reduced(Fr29Inverse::inverse(Fr29::from_words<5>(w).reduce(), Fr29Inverse::INV_UP));
+      printf("\n");
+      continue;
+    }
+    if (scanf(" %127s %127s %d", sa, sb, &n) != 3) return 2;
     if (!read_hex(sa, w)) return 2;
     Fr29 a = Fr29::from_words<0>(w);
     if (!read_hex(sb, w)) return 2;

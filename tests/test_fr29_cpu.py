@@ -51,3 +51,14 @@ def test_butterfly_chains(driver, stages):
                 assert got % R == want
                 assert got < R + R // 5000  # reduce() ends below 1.0002 r
             assert ok == "1", "a limb left its bound"
+
+
+def test_inverse(driver):
+    rng = random.Random(5)
+    xs = [0, 1, 2, R - 1, R - 2, (1 << 253), (1 << 256) % R, pow(2, -1, R), pow(2, -253, R)]
+    xs += [rng.randrange(R) for _ in range(3000)]
+    r = subprocess.run([driver], input="".join(f"inv {x:064x}\n" for x in xs), capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr
+    for x, line in zip(xs, r.stdout.split("\n")):
+        want = pow(x, -1, R) * (1 << 512) % R if x else 0
+        assert [int(h, 16) % R for h in line.split()] == [want, want]

@@ -411,6 +411,38 @@ def test_permute_reuses_temp_for_a_smaller_call(libs, stream):
         assert np.array_equal(gpu2cpu(rt, rtb), want_tab)
 
 
+@pytest.mark.parametrize("k", [10, 18, 19, 22, 23])
+def test_share_edges(libs, stream, k):
+    """Evaluation, quotient and prefix products where a workgroup's share changes:
+    one share and two, runs of 4, 8, 16 and 32 elements, shares of one and two
+    rounds, with one element more than fills them."""
+    n = 1 << k
+    a = random_elements(n + 1, 140 + k)
+    x = random_elements(1, 141)[0]
+    xb, xs = dev_scalar(x)
+    rb, rs = dev_scalar(np.zeros(4, np.uint64))
+    for m in (n, n + 1):
+        ab, av = put(a[:m], rotate=m // 3)
+        op = PolyEval(libs)
+        tb, tmp = temp_buffer(op.get_buffer_size(m))
+        op.get_fn().f([tmp, rs], [av, xs, stream])
+        stream.sync()
+        assert np.array_equal(read_scalar(rb), orc.poly_eval(a[:m], x)), m
+        zb, zv = empty(m)
+        op = PolyScan(libs)
+        tb, tmp = temp_buffer(op.get_buffer_size(m))
+        op.get_fn().f([tmp, zv], [av, xs, stream])
+        stream.sync()
+        assert np.array_equal(gpu2cpu(zv, zb), orc.scan_mul(np.concatenate([x.reshape(1, 4), a[: m - 1]]))), m
+    pb, pv = put(a[:n])
+    qb, qv = empty(n)
+    op = KateDivision(libs)
+    tb, tmp = temp_buffer(op.get_buffer_size(k))
+    op.get_fn().f([tmp, qv], [pv, xs, stream])
+    stream.sync()
+    assert np.array_equal(gpu2cpu(qv, qb), orc.kate_division(a[:n], x)), k
+
+
 # ---------------------------------------------------------------- full size (2^24)
 
 

@@ -482,71 +482,6 @@ struct Fp {
     return r;
   }
 
-  // Inverse by the binary extended Euclidean algorithm, for a lone thread
-  // inverting one value (variable time: a few hundred 256-bit shifts and
-  // subtractions in place of Fermat's ~380 serial products).  The integer
-  // inverse of the Montgomery word aR is a^-1 R^-1; one product with R^3 gives
-  // a^-1 R.  Invariants: x1 * w = u and x2 * w = v (mod p), with w the word.
-  // Zero maps to zero.  Any 256-bit word is first reduced below p, so the
-  // loops always end (gcd(u, p) = 1 for 0 < u < p).
-  ZKP_HD Fp inv_binary() const {
-    const Fp p = from_raw(Params::P);
-    Fp u = *this;
-    while (!u.less_than(p)) u.sub_words(p);  // at most 5 times: 2^256 < 6p
-    if (u.is_zero()) return zero();
-    Fp v = p, x1 = zero(), x2 = zero();
-    x1.v[0] = 1;
-    while (!u.is_one_word() && !v.is_one_word()) {
-      while (!(u.v[0] & 1)) {
-        u.shr1();
-        x1.half_mod();
-      }
-      while (!(v.v[0] & 1)) {
-        v.shr1();
-        x2.half_mod();
-      }
-      if (!u.less_than(v)) {
-        u.sub_words(v);
-        x1 = x1 - x2;
-      } else {
-        v.sub_words(u);
-        x2 = x2 - x1;
-      }
-    }
-    return (u.is_one_word() ? x1 : x2) * from_raw(Params::R3);
-  }
-  ZKP_HD bool is_one_word() const {
-    u32 acc = v[0] ^ 1u;
-#pragma unroll
-    for (int i = 1; i < 8; i++) acc |= v[i];
-    return acc == 0;
-  }
-  ZKP_HD bool less_than(const Fp& o) const {
-    u32 borrow = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) (void)sbb(v[i], o.v[i], borrow);
-    return borrow != 0;
-  }
-  ZKP_HD void sub_words(const Fp& o) {
-    u32 borrow = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = sbb(v[i], o.v[i], borrow);
-  }
-  ZKP_HD void shr1() {
-#pragma unroll
-    for (int i = 0; i < 7; i++) v[i] = (v[i] >> 1) | (v[i + 1] << 31);
-    v[7] >>= 1;
-  }
-  // x / 2 mod p for x < p: (x + p) / 2 when x is odd (x + p < 2p < 2^256)
-  ZKP_HD void half_mod() {
-    if (v[0] & 1) {
-      u32 carry = 0;
-#pragma unroll
-      for (int i = 0; i < 8; i++) v[i] = adc(v[i], Params::P[i], carry);
-    }
-    shr1();
-  }
-
   // Fermat inverse x^(p-2); inverse of zero is zero.
   ZKP_HD Fp inv() const {
     u32 e[8];

@@ -172,4 +172,152 @@ struct Fr29 {
   }
 };
 
+// ---------------------------------------------------------------- inversion
+//
+// mul's two operands stand for x 2^256 and y 2^256 when the second is unpacked 5
+// bits up; a value that serves as second operand again has to keep the factor 32
+// itself.  Call a value "up" when it is 32 x 2^256 mod r: up * up is up, and
+// plain * up is plain.  Unpacked words are up below 32 r, for which mul's result
+// is below 6.1 r in magnitude, and results of mul are normalised, so chains of
+// products go on without end in either operand.
+//
+// inverse(x, c) = x^-1 c 2^-261 mod r for a normalised x in [0, 2 r); 0 where x
+// is 0 mod r.  With c = INV_PLAIN it maps x 2^256 to x^-1 2^256, with INV_UP an up value of x
+// to x^-1 2^256.
+//
+// Bernstein and Yang's division steps (Fast constant-time gcd computation and
+// modular inversion, 2019), in variable time: f = r, g = x, f odd; while g is
+// even it is halved; else with delta > 0 (f, g) becomes (g, -f), and g + w f
+// clears as many bits of g as delta allows.  29 steps at a time are taken on the
+// low words and collected in a matrix that is then applied to f and g (exactly
+// divisible by 2^29) and, mod r, to d and e with d x = f, e x = g (mod r).
+// A batch changes |d| and |e| by at most r, so limb 8 stays below 2^28 for the at
+// most 26 batches (754 steps; the paper bounds 256-bit inputs by 741).
+struct Fr29Inverse {
+  static constexpr int32_t R[9] = {0x10000001, 0x1f0fac9f, 0x0e5c2450, 0x07d090f3,
+                                  0x1585d283, 0x02db40c0, 0x00a6e141, 0x0e5c2634, 0x0030644e};
+  static constexpr int32_t INV_PLAIN[9] = {0x17e007f8, 0x1c5b7cb8, 0x0ad4a06c, 0x08aaffa3,
+                                  0x13abc077, 0x0f7013f7, 0x190d945a, 0x1b1dfff5, 0x001be8b5};
+  static constexpr int32_t INV_UP[9] = {0x1c00feee, 0x1c5573e0, 0x18197fea, 0x08b5c34c,
+                                  0x120f41ae, 0x1a97f167, 0x15f6b4bb, 0x01454f10, 0x00160937};
+
+  int32_t u, v, q, r;  // 2^29 (f', g') = [u v; q r] (f, g)
+
+  // 29 division steps on the low 32 bits of f (odd) and g
+  ZKP_HD void steps(u32 f, u32 g, int32_t& delta) {
+    u32 a = 1, b = 0, c = 0, d = 1;
+    int left = 29;
+    for (;;) {
+      const int z = __builtin_ctz(g | (1u << left));
+      g >>= z;
+      a <<= z;
+      b <<= z;
+      delta += z;
+      left -= z;
+      if (left == 0) break;
+      if (delta > 0) {
+        delta = -delta;
+        u32 t = f; f = g; g = 0u - t;
+        t = a; a = c; c = 0u - t;
+        t = b; b = d; d = 0u - t;
+      }
+      // f f (f f - 2) = (f f - 1)^2 - 1 = -1 mod 64: w f = -g mod 2^min(k, left)
+      const int k = 1 - delta < 6 ? 1 - delta : 6;
+      const u32 w = (g * f * (f * f - 2)) & ((1u << k) - 1) & ((1u << left) - 1);
+      g += w * f;
+      c += w * a;
+      d += w * b;
+    }
+    u = (int32_t)a;
+    v = (int32_t)b;
+    q = (int32_t)c;
+    r = (int32_t)d;
+  }
+
+  // (a x + b y) / 2^29: exact with mod = 0, mod r with mod = MASK
+  ZKP_HD static Fr29 row(int32_t a, const Fr29& x, int32_t b, const Fr29& y, int32_t mod) {
+    Fr29 o;
+    int64_t acc = (int64_t)a * x.l[0] + (int64_t)b * y.l[0];
+    const u32 lo = (u32)acc;
+    const int32_t m = (int32_t)(lo + (lo << 28)) & mod;
+    acc += (int64_t)m * Fr29::NEG_R[0];
+    acc >>= 29;
+#pragma unroll
+    for (int i = 1; i < 9; i++) {
+      acc += (int64_t)a * x.l[i] + (int64_t)b * y.l[i];
+      acc += (int64_t)m * Fr29::NEG_R[i];
+      o.l[i - 1] = (int32_t)((u32)acc & (u32)Fr29::MASK);
+      acc >>= 29;
+    }
+    o.l[8] = (int32_t)acc;
+    return o;
+  }
+
+  // On the device the lanes of a wave work together (all of them call, with the
+  // same x): the steps run on the scalar unit, and lanes 0..3 of every quad form f,
+  // g, d and e, each from the pair (p, q) = (f, g) or (d, e) that it keeps a copy
+  // of.  11 us at a lone wave; on one lane of the vector unit, 50.
+  ZKP_HD static Fr29 inverse(const Fr29& x, const int32_t (&c)[9]) {
+    Fr29 w;
+    int32_t delta = 1;
+    Fr29Inverse s;
+#if defined(__HIP_DEVICE_COMPILE__)
+    const u32 lane = threadIdx.x;
+    const bool second = lane & 1, mod_r = lane & 2;
+    const int32_t mod = mod_r ? Fr29::MASK : 0;
+    Fr29 p, q;
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+      p.l[i] = mod_r ? 0 : R[i];
+      q.l[i] = mod_r ? (i == 0 ? 1 : 0) : x.l[i];
+      w.l[i] = c[i];
+    }
+#pragma unroll 1
+    for (int n = 0; n < 26; n++) {
+      int32_t any = 0;
+#pragma unroll
+      for (int i = 0; i < 9; i++) any |= q.l[i];
+      if (__builtin_amdgcn_readfirstlane(any) == 0) break;
+      s.steps((u32)__builtin_amdgcn_readfirstlane(p.l[0] | p.l[1] << 29),
+              (u32)__builtin_amdgcn_readfirstlane(q.l[0] | q.l[1] << 29), delta);
+      const Fr29 o = row(second ? s.q : s.u, p, second ? s.r : s.v, q, mod);
+#pragma unroll
+      for (int i = 0; i < 9; i++) {
+        p.l[i] = __builtin_amdgcn_update_dpp(0, o.l[i], 0xa0, 0xf, 0xf, true);  // quad_perm 0, 0, 2, 2
+        q.l[i] = __builtin_amdgcn_update_dpp(0, o.l[i], 0xf5, 0xf, 0xf, true);  // quad_perm 1, 1, 3, 3
+      }
+    }
+    const int32_t top = __builtin_amdgcn_readfirstlane(p.l[8]);
+    Fr29 d;
+#pragma unroll
+    for (int i = 0; i < 9; i++) d.l[i] = __builtin_amdgcn_update_dpp(0, p.l[i], 0xaa, 0xf, 0xf, true);  // lane 2's
+#else
+    Fr29 f, g = x, d, e;
+    for (int i = 0; i < 9; i++) {
+      f.l[i] = R[i];
+      d.l[i] = 0;
+      e.l[i] = i == 0 ? 1 : 0;
+      w.l[i] = c[i];
+    }
+    for (int n = 0; n < 26; n++) {
+      int32_t any = 0;
+      for (int i = 0; i < 9; i++) any |= g.l[i];
+      if (any == 0) break;
+      s.steps((u32)f.l[0] | (u32)f.l[1] << 29, (u32)g.l[0] | (u32)g.l[1] << 29, delta);
+      const Fr29 f1 = row(s.u, f, s.v, g, 0), d1 = row(s.u, d, s.v, e, Fr29::MASK);
+      g = row(s.q, f, s.r, g, 0);
+      e = row(s.q, d, s.r, e, Fr29::MASK);
+      f = f1;
+      d = d1;
+    }
+    const int32_t top = f.l[8];
+#endif
+    // f = 1, -1, or r times one of them where x = 0 (mod r)
+    const int32_t sign = top == 0 ? 1 : top == -1 ? -1 : 0;
+#pragma unroll
+    for (int i = 0; i < 9; i++) d.l[i] *= sign;
+    return Fr29::mul(d, w);
+  }
+};
+
 }  // namespace zkp
