@@ -13,6 +13,7 @@ size), the GPU tests the results.  The reference has no fused-kernel test of
 its own (its kernels run only inside compiled programs).
 """
 import json
+import re
 
 import numpy as np
 import pytest
@@ -109,6 +110,25 @@ def test_large_graph_plan(seed, coef):
     assert "amdgpu_waves_per_eu" in src
 
 
+@pytest.mark.parametrize("budget,waves", [(16, 2), (5, 2), (16, 1), (8, 4), (16, 0)])
+def test_large_graph_buffer_holds_the_grid(budget, waves):
+    """local_buffer: the table, then 36 bytes a slot for every thread the capped grid can have."""
+    fused.set_codegen_options(Libs(), budget, waves)
+    try:
+        src = fused.codegen(Libs(), fused.random_graph(*CASES[0][:1], fused.LARGE_VERTICES), "large_buffer")
+    finally:
+        fused.set_codegen_options(Libs())
+    blocks, threads = map(int, re.search(r"kSpillThreads = (\d+)ull \* (\d+);", src).groups())
+    slots = int(re.search(r"kSpillSlots = (\d+);", src).group(1))
+    assert src.count(f"grid_capped(len, {threads}, {blocks})), dim3({threads})") == 1
+    assert src.count(f"grid_capped(total, {threads}, {blocks})), dim3({threads})") == 1
+    entries = [int(x) for x in re.findall(r"put_raw\(table \+ (\d+),", src)]
+    table = int(re.search(r"local_buffer\) \+ (\d+)\)", src).group(1))
+    assert table % 256 == 0 and max(entries) + 12 <= table // 4
+    assert max(int(x) for x in re.findall(r"spill_store\(spill, me, (\d+),", src)) < slots
+    assert int(re.search(r"return (\d+)ull; \}", src).group(1)) == table + 36 * slots * blocks * threads
+
+
 # ---------------------------------------------------------------- GPU
 
 
@@ -177,3 +197,47 @@ def test_large_graph_matches_interpreter(libs, stream, seed, coef):
             got = gpu2cpu(arr, b)
             want = want if want.ndim == 2 else np.broadcast_to(want, (n, 4))
             assert np.array_equal(got, want), o
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("coef", [False, True])
+@pytest.mark.parametrize("lens", [(1,), (511,), (513,), (131072 + 513,), (3, 600, 1)])
+def test_ranges(libs, stream, coef, lens):
+    """graph_ranges around a workgroup, past the grid, and (several lengths) as the
+    instances of one batched call, each with scalars of its own."""
+    from zkpoly_amd.batch import FusedBatch
+
+    g = json.loads(fused.graph_ranges(coef))
+    V = g["g"][0]
+    meta = fused.FusedKernelMeta("fused_arith_ranges_coef" if coef else "fused_arith_ranges", 7, len(g["outputs"]),
+                                 fused.DEMO_DIR)
+    k = fused.FusedKernel(libs, meta)
+    var, mut, bufs, want = [], [], [], []
+    for q, n in enumerate(lens):
+        polys = {g["inputs"][j]: random_elements(n, 700 + 10 * q + j) for j in range(2)}
+        polys[g["inputs"][0]][0] = 0
+        scalars = {g["inputs"][2 + j]: random_elements(1, 800 + 10 * q + j)[0] for j in range(5)}
+        get = interpret(g, polys, scalars, n)
+        for i in g["inputs"]:
+            x = polys[i] if i in polys else scalars[i].reshape(1, 4)
+            b, arr = device_array(x.shape[0])
+            cpu2gpu(x, arr, b)
+            bufs.append(b)
+            var.append(arr if i in polys else Scalar(b.addr))
+        for o in g["outputs"]:
+            op = V[o]["op"]["Output"]
+            scalar = op["typ"] == "Scalar"
+            b, arr = device_array(1 if scalar else n)
+            bufs.append(b)
+            mut.append(Scalar(b.addr) if scalar else arr)
+            want.append((arr, b, get(op["store_node"]).reshape(-1, 4)))
+    print(f"fused ranges coef={coef} lens={lens}", flush=True)
+    if len(lens) == 1:
+        arg = hip.DeviceBuffer(fused.arg_buffer_bytes(meta))
+        local = hip.DeviceBuffer(k.local_bytes)
+        k.get_fn().f([GpuBuffer(arg.addr, arg.nbytes), GpuBuffer(local.addr, k.local_bytes)] + mut, [stream] + var)
+    else:
+        FusedBatch(k, [fused._ptr_of(x) for x in var], [fused._ptr_of(x) for x in mut], list(lens)).run(stream)
+    stream.sync()
+    for arr, b, w in want:
+        assert np.array_equal(gpu2cpu(arr, b), w)

@@ -452,6 +452,95 @@ struct Emitter {
     return head + " ? " + r + " - " + l + " : " + r;  // SubBy
   }
 
+  // ---------------------------------------------------------------- 29-bit limbs
+  //
+  // A kernel with a scalar table or spill slots (`limbs`) computes in Fr29, every
+  // value "up" (32 x 2^256 mod r, fr29.hpp); a smaller one is bound by its loads
+  // and stores and stays in the words it reads and writes.  Values are reduced only
+  // where their range asks for it, and the ranges are known here: bounds of the
+  // value in multiples of r and of its limbs 0..7 in multiples of 2^29.  With them
+  // every operation decides whether an operand has to be carried (norm) or reduced
+  // first: limbs stay within 3 2^29, a product's operands within 3 2^58 (nine of
+  // those and the reduction stay below 2^63).  A graph of 800 vertices (about 210
+  // products, 18 outputs) over 2^18 elements: 620 us and 40 for the scalars, where
+  // 32-bit arithmetic took 1 120 and 62.  Bound by VALU issue (66 000 instructions an
+  // element and wave, 485 us), then by the spills and the code's own 490 KB.
+  struct Range {
+    double lo = 0, hi = 0, llo = 0, lhi = 1;
+    double value() const { return std::max(-lo, hi); }
+    double limb() const { return std::max(std::max(-llo, lhi), value() * R_WIDTH + 0.01); }
+  };
+  static constexpr double R_WIDTH = 0.005908;  // r / 2^261, and the width of r in limb 8
+  static constexpr double MAX_LIMB = 3.0, MAX_VALUE = 160.0;
+  static Range loaded() { return {0, 32, 0, 1}; }
+  static Range reduced() { return {0, 1.0002, 0, 1}; }
+  struct Val {
+    std::string name;
+    Range r;
+  };
+  bool limbs = false;
+
+  static Val norm(const Val& a) { return {a.name + ".norm()", {a.r.lo, a.r.hi, 0, 1}}; }
+  static Val reduce(const Val& a) { return {a.name + ".reduce()", reduced()}; }
+  // carried, or reduced if it already is
+  static Val smaller(const Val& a) { return a.r.llo < 0 || a.r.lhi > 1 ? norm(a) : reduce(a); }
+
+  static Val mul29(Val a, Val b) {
+    while (a.r.limb() * b.r.limb() > MAX_LIMB) {
+      Val& big = a.r.limb() >= b.r.limb() ? a : b;
+      big = smaller(big);
+    }
+    const double p[4] = {a.r.lo * b.r.lo, a.r.lo * b.r.hi, a.r.hi * b.r.lo, a.r.hi * b.r.hi};
+    const double lo = *std::min_element(p, p + 4), hi = *std::max_element(p, p + 4);
+    // a table entry comes from memory and is best left where it is, on the scalar unit
+    if (a.name.find("entry(") != std::string::npos) std::swap(a, b);
+    const bool entry = b.name.find("entry(") != std::string::npos;
+    return {"zkp::Fr29::mul(" + a.name + ", " + (entry ? b.name : "zkp::fused::factor(" + b.name + ")") + ")",
+            {std::min(lo, 0.0) * R_WIDTH - 1.001, std::max(hi, 0.0) * R_WIDTH + 0.001, 0, 1}};
+  }
+  static Val add29(Val a, Val b, bool sub) {
+    for (;;) {
+      const Range &x = a.r, &y = b.r;
+      const Range o = sub ? Range{x.lo - y.hi, x.hi - y.lo, x.llo - y.lhi, x.lhi - y.llo}
+                          : Range{x.lo + y.lo, x.hi + y.hi, x.llo + y.llo, x.lhi + y.lhi};
+      if (o.value() > MAX_VALUE) {
+        Val& big = a.r.value() >= b.r.value() ? a : b;
+        big = reduce(big);
+      } else if (o.limb() > MAX_LIMB) {
+        Val& big = a.r.limb() >= b.r.limb() ? a : b;
+        big = smaller(big);
+      } else {
+        return {"(" + a.name + (sub ? " - " : " + ") + b.name + ")", o};
+      }
+    }
+  }
+  static Val neg29(const Val& a) {
+    return {"zkp::fused::neg(" + a.name + ")", {-a.r.hi, -a.r.lo, -a.r.lhi, -a.r.llo}};
+  }
+  static Val pow29(Val a, uint64_t e) {
+    if (e == 2) return mul29(a, a);
+    if (a.r.value() > 33) a = reduce(a);
+    if (a.r.llo < 0 || a.r.lhi > 1) a = norm(a);
+    // from 33 r on squares and products stay below 7.5 r, x^1 is x and x^0 below 32 r
+    return {"zkp::fused::pow(" + a.name + ", " + std::to_string(e) + "ull)", {-33, 33, 0, 1}};
+  }
+  Val expr29(uint64_t id, const Val& l, const Val& r) const {
+    const Vertex& x = g.v[id];
+    if (x.kind == OpKind::Unr) return x.op == "Neg" ? neg29(l) : pow29(l, x.pow);
+    if (x.op == "Mul") return mul29(l, r);
+    if (x.group != Group::Sp) return add29(l, r, x.op == "Sub");
+    const Val all = x.op == "Add" ? add29(l, r, false) : x.op == "Sub" ? add29(l, r, true) : add29(r, l, true);
+    if (!g.coef) return all;
+    const Val rest = x.op == "Sub" ? neg29(r) : r;
+    return {"zkp::fused::pick((idx == 0 && is_first), " + all.name + ", " + rest.name + ")",
+            {std::min(all.r.lo, rest.r.lo), std::max(all.r.hi, rest.r.hi), std::min(all.r.llo, rest.r.llo),
+             std::max(all.r.lhi, rest.r.lhi)}};
+  }
+  const char* type() const { return limbs ? "zkp::Fr29" : "zkp::Fr"; }
+  std::map<uint64_t, Range> scalar_range;  // of the inline scalar values (limbs)
+  // 4-byte words of a table entry
+  size_t entry_words() const { return limbs ? 12 : 8; }
+
   std::string src_ptr(uint64_t id, const std::string& vars, const std::string& mut_vars) const {
     auto it = var_slot.find(id);
     if (it != var_slot.end()) return vars + "[" + std::to_string(it->second) + "]";
@@ -481,15 +570,26 @@ struct Emitter {
       }
   }
   bool scalar_table() const { return scalar_order.size() > SCALAR_REGS; }
-  size_t table_bytes() const { return scalar_table() ? align256(scalar_order.size() * 32) : 0; }
+  size_t table_bytes() const { return scalar_table() ? align256(scalar_order.size() * 4 * entry_words()) : 0; }
   static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
   // straight-line evaluation of every scalar vertex into const locals t<id>
   void emit_scalar_values(std::ostringstream& o, const std::string& vars, const std::string& mut_vars,
-                          const char* ind) const {
+                          const char* ind, const char* put = nullptr) {
     for (uint64_t id : scalar_order) {
       const Vertex& x = g.v[id];
-      if (x.kind == OpKind::Input)
+      if (limbs) {
+        Val v{"", loaded()};
+        if (x.kind == OpKind::Input)
+          v.name = "zkp::fused::scalar_in(" + src_ptr(id, vars, mut_vars) + ".ptr)";
+        else
+          v = expr29(id, {tmp(x.lhs), scalar_range.at(x.lhs)},
+                     x.kind == OpKind::Bin ? Val{tmp(x.rhs), scalar_range.at(x.rhs)} : Val{});
+        scalar_range[id] = v.r;
+        o << ind << "const zkp::Fr29 " << tmp(id) << " = " << v.name << ";\n";
+        if (put)
+          o << ind << "zkp::fused::" << put << scalar_index.at(id) * entry_words() << ", " << tmp(id) << ");\n";
+      } else if (x.kind == OpKind::Input)
         o << ind << "const zkp::Fr " << tmp(id) << " = zkp::Fr::load(" << src_ptr(id, vars, mut_vars) << ".ptr);\n";
       else
         o << ind << "const zkp::Fr " << tmp(id) << " = "
@@ -501,19 +601,26 @@ struct Emitter {
   //
   // The element loop evaluates the per-element vertices in the depth-first
   // order of the outputs, holding at most reg_budget field elements in
-  // registers (8 VGPRs each; a product needs about 40 more), so that the
+  // registers (8 or 9 VGPRs each; a product needs about 40 more), so that the
   // kernel keeps several waves per SIMD.  When a value must leave, the one used
   // furthest in the future goes (Belady): an input polynomial is simply read
   // again later, a computed value is written once to its spill slot in
-  // local_buffer (two 16-byte planes per slot, lane-contiguous, so spills are
-  // coalesced) and read back before its next use.  Outputs are stored as soon
+  // local_buffer (two 16-byte planes and one of 4 bytes per slot, lane-contiguous,
+  // so spills are coalesced) and read back before its next use.  Outputs are stored as soon
   // as their value exists, except an output that overwrites an input still to
   // be read, which waits for the end of the element.
   size_t reg_budget = 16;     // field elements kept in registers per element
   unsigned waves_per_eu = 2;  // occupancy the register allocator must keep (0: compiler's choice)
-  // grid when spilling: the workgroups of 256 threads that fit 256 CUs at the
-  // kernel's occupancy (four per CU when the compiler chooses)
-  unsigned spill_blocks() const { return 256u * (waves_per_eu ? waves_per_eu : 4u); }
+  // Threads of a workgroup.  A kernel in limbs is hundreds of KB of straight code:
+  // waves that drift apart fetch it one by one past the 64 KB instruction cache, so
+  // its workgroups hold two waves per SIMD and its waves meet at a barrier every
+  // BARRIER_EVERY products (about 16 KB): 620 us against 635 without, and 770 with
+  // one wave per SIMD and nearly no spills.
+  unsigned threads() const { return limbs && waves_per_eu != 1 ? 512u : 256u; }
+  static constexpr unsigned BARRIER_EVERY = 8;
+  // grid when spilling: the workgroups that fit 256 CUs at the kernel's occupancy
+  // (four waves per SIMD when the compiler chooses)
+  unsigned spill_blocks() const { return 256u * (waves_per_eu ? waves_per_eu : 4u) * 256u / threads(); }
   std::vector<uint64_t> elem_order;  // per-element vertices and poly outputs, in order
   size_t spill_slots = 0;
   std::string element_code;  // generated with `indent` placeholders resolved later
@@ -525,6 +632,7 @@ struct Emitter {
     std::map<uint64_t, std::vector<size_t>> uses;  // vertex -> positions of its uses
     std::map<uint64_t, std::string> reg;           // vertex -> name of its value in a register
     std::map<uint64_t, size_t> slot;               // spilled vertex -> slot
+    std::map<uint64_t, Range> range;               // of the value, as computed and as spilled (limbs)
     std::vector<size_t> free_slots;
     size_t slots = 0;
     size_t counter = 0;
@@ -568,7 +676,8 @@ struct Emitter {
           sl = slots++;
         }
         slot[victim] = sl;
-        o << ind << "zkp::fused::spill_store(spill, " << sl << ", kSpillThreads, " << reg[victim] << ");\n";
+        o << ind << "zkp::fused::spill_store(spill, me, " << sl << ", kSpillSlots, kSpillThreads, " << reg[victim]
+          << ");\n";
       }
       reg.erase(victim);
     }
@@ -586,10 +695,16 @@ struct Emitter {
       make_room(keep);
       const std::string n = fresh(id);
       const Vertex& x = e.g.v[id];
-      if (x.kind == OpKind::Input)
-        o << ind << "const zkp::Fr " << n << " = zkp::Fr::load(v" << id << ".elem(idx));\n";
-      else
-        o << ind << "const zkp::Fr " << n << " = zkp::fused::spill_load(spill, " << slot.at(id) << ", kSpillThreads);\n";
+      o << ind << "const " << e.type() << " " << n << " = ";
+      if (x.kind == OpKind::Input) {
+        if (e.limbs)
+          o << "zkp::fused::load_up(v" << id << ", idx, vars);\n";
+        else
+          o << "zkp::Fr::load(v" << id << ".elem(idx));\n";
+        range[id] = loaded();
+      } else {
+        o << "zkp::fused::spill_load(spill, me, " << slot.at(id) << ", kSpillSlots, kSpillThreads);\n";
+      }
       reg[id] = n;
       return n;
     }
@@ -608,10 +723,15 @@ struct Emitter {
   std::string operand(const Alloc& A, uint64_t id, const std::map<uint64_t, std::string>& names) const {
     (void)A;
     if (is_scalar_value(id)) {
-      if (scalar_table()) return "zkp::Fr::load(scalars + " + std::to_string(scalar_index.at(id) * 8) + ")";
+      const std::string at = std::to_string(scalar_index.at(id) * entry_words());
+      if (scalar_table()) return (limbs ? "zkp::fused::entry(scalars + " : "zkp::Fr::load(scalars + ") + at + ")";
       return tmp(id);
     }
     return names.at(id);
+  }
+  Val operand29(const Alloc& A, uint64_t id, const std::string& text) const {
+    if (!is_scalar_value(id)) return {text, A.range.at(id)};
+    return {text, scalar_table() ? reduced() : scalar_range.at(id)};
   }
 
   void plan_elements() {
@@ -626,7 +746,7 @@ struct Emitter {
   // Element code (one pass of the allocator); `ind` is the indentation.
   std::string gen_element(const char* ind_c) {
     std::ostringstream o;
-    Alloc A{*this, o, std::string(ind_c), {}, {}, {}, {}, 0, 0, 0};
+    Alloc A{*this, o, std::string(ind_c), {}, {}, {}, {}, {}, 0, 0, 0};
     // positions of uses; deferred in-place outputs use their value at the end
     const size_t END = elem_order.size();
     std::vector<uint64_t> deferred;
@@ -667,8 +787,12 @@ struct Emitter {
       std::string val;
       if (is_poly(x.store_node)) val = A.get(x.store_node, keep);
       else val = operand(A, x.store_node, {});
-      o << ind_c << val << ".store(o" << out_id << ".elem(idx));\n";
+      if (limbs)
+        o << ind_c << "zkp::fused::store_down(" << val << ", o" << out_id << ", idx, live, vars);\n";
+      else
+        o << ind_c << val << ".store(o" << out_id << ".elem(idx));\n";
     };
+    unsigned products = 0;  // since the last barrier (limbs)
     std::set<uint64_t> deferred_set(deferred.begin(), deferred.end());
     for (size_t t = 0; t < elem_order.size(); t++) {
       A.pos = t;
@@ -691,7 +815,18 @@ struct Emitter {
       for (uint64_t c : keep) A.retire(c);
       A.make_room(keep);
       const std::string n = A.fresh(id);
-      o << ind_c << "const zkp::Fr " << n << " = " << expr(id, l, r) << ";\n";
+      if (limbs) {
+        const Val v = expr29(id, operand29(A, x.lhs, l), x.kind == OpKind::Bin ? operand29(A, x.rhs, r) : Val{});
+        A.range[id] = v.r;
+        o << ind_c << "const zkp::Fr29 " << n << " = " << v.name << ";\n";
+        products += x.op == "Mul" ? 1 : x.op == "Pow" ? 3 : 0;
+        if (products >= BARRIER_EVERY) {
+          o << ind_c << "__builtin_amdgcn_s_barrier();\n";
+          products = 0;
+        }
+      } else {
+        o << ind_c << "const zkp::Fr " << n << " = " << expr(id, l, r) << ";\n";
+      }
       A.reg[id] = n;
       A.retire(id);  // never used (an output of nothing): drop at once
     }
@@ -703,7 +838,7 @@ struct Emitter {
 
   // views (and, without a scalar table, the scalar values) before the element loop
   void emit_views(std::ostringstream& o, const std::string& vars, const std::string& mut_vars, const char* ind,
-                  bool scalars_inline) const {
+                  bool scalars_inline) {
     for (uint64_t id : order) {
       const Vertex& x = g.v[id];
       if (x.kind == OpKind::Input && !x.scalar)
@@ -721,7 +856,8 @@ struct Emitter {
     for (uint64_t id : order) {
       const Vertex& x = g.v[id];
       if (x.kind != OpKind::Output || !x.scalar) continue;
-      o << ind << guard << tmp(x.store_node) << ".store(" << mut_vars << "[" << mut_slot.at(id) << "].ptr);\n";
+      const std::string val = limbs ? "zkp::fused::down(" + tmp(x.store_node) + ")" : tmp(x.store_node);
+      o << ind << guard << val << ".store(" << mut_vars << "[" << mut_slot.at(id) << "].ptr);\n";
     }
   }
 
@@ -729,60 +865,81 @@ struct Emitter {
     plan_scalars();
     plan_elements();
     const bool table = scalar_table();
+    gen_element("    ");  // the allocation: it does not depend on the arithmetic
+    const bool spills = spill_slots > 0;
+    limbs = table || spills;
+    if (limbs && !table) {  // ranges of the scalars that the element code will name
+      std::ostringstream unused;
+      emit_scalar_values(unused, "vars", "mut_vars", "");
+    }
     const std::string elem_single = gen_element("    ");
     const std::string elem_batched = gen_element("    ");  // same allocation, own names
-    const bool spills = spill_slots > 0;
     const size_t nv = var_slot.size(), nm = g.outputs.size();
     const unsigned blocks = spill_blocks();
-    const size_t local_bytes = table_bytes() + (spills ? spill_slots * 32ull * blocks * 256ull : 0);
+    const size_t local_bytes = table_bytes() + (spills ? spill_slots * 36ull * blocks * threads() : 0);
     std::ostringstream o;
     o << "// Generated fused elementwise kernel " << name << " (" << order.size() << " vertices, "
       << (g.coef ? "coefficient" : "Lagrange") << " form; " << scalar_order.size() << " scalar values"
       << (table ? " in a table" : "") << ", " << spill_slots << " spill slots).\n";
     o << "#include \"fused/fused_runtime.hpp\"\n\n";
     o << "namespace {\n";
-    if (spills) o << "constexpr uint64_t kSpillThreads = " << blocks << "ull * zkp::fused::THREADS;\n\n";
+    if (spills)
+      o << "constexpr uint64_t kSpillThreads = " << blocks << "ull * " << threads() << ";\n"
+        << "constexpr uint64_t kSpillSlots = " << spill_slots << ";\n\n";
     if (table) {
-      o << "__global__ void " << name
+      // one wave, all lanes alike; each then reduces its share of the entries
+      o << "__global__ void __launch_bounds__(64) " << name
         << "_scalars_kernel(const ConstPolyPtr* __restrict__ vars, const PolyPtr* __restrict__ mut_vars, "
            "uint32_t* __restrict__ table) {\n";
-      emit_scalar_values(o, "vars", "mut_vars", "  ");
-      for (uint64_t id : scalar_order) o << "  " << tmp(id) << ".store(table + " << scalar_index.at(id) * 8 << ");\n";
-      emit_scalar_outputs(o, "mut_vars", "  ", "");
+      emit_scalar_values(o, "vars", "mut_vars", "  ", "put_raw(table + ");
+      emit_scalar_outputs(o, "mut_vars", "  ", "if (threadIdx.x == 0) ");
+      o << "  zkp::fused::reduce_entries(table, " << scalar_order.size() << ");\n";
       o << "}\n\n";
     }
     // the occupancy the register budget was chosen for binds only kernels that spill; a small kernel keeps
     // whatever occupancy its few registers give (its loads need the waves)
-    const std::string bounds = "__launch_bounds__(zkp::fused::THREADS)" +
+    const std::string wg = std::to_string(threads());
+    const std::string bounds = "__launch_bounds__(" + wg + ")" +
         (waves_per_eu && spills ? " __attribute__((amdgpu_waves_per_eu(" + std::to_string(waves_per_eu) + ")))"
                                 : std::string());
     o << "__global__ void " << bounds << "\n    " << name
       << "_kernel(const ConstPolyPtr* __restrict__ vars, const PolyPtr* __restrict__ mut_vars, "
-         "unsigned long long len, bool is_first, uint32_t* __restrict__ local) {\n";
-    o << "  (void)local;\n";
-    if (table) o << "  const uint32_t* __restrict__ scalars = local;\n";
+         "unsigned long long len, bool is_first, const uint32_t* __restrict__ scalars, char* __restrict__ spill) {\n";
+    o << "  (void)scalars, (void)spill;\n";
     if (spills)
-      o << "  uint4* __restrict__ spill = reinterpret_cast<uint4*>(reinterpret_cast<char*>(local) + " << table_bytes()
-        << ") + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;\n";
+      o << "  const uint32_t me = blockIdx.x * blockDim.x + threadIdx.x;\n";
     emit_views(o, "vars", "mut_vars", "  ", !table);
     o << "  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;\n";
-    o << "  for (uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < len; idx += stride) {\n";
+    if (limbs) {
+      // every thread of a workgroup takes part in its barriers; those past the end repeat the last element
+      o << "  for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x; base < len; base += stride) {\n";
+      o << "    const bool live = base + threadIdx.x < len;\n";
+      o << "    const uint64_t idx = live ? base + threadIdx.x : len - 1;\n";
+    } else {
+      o << "  for (uint64_t idx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < len; idx += stride) {\n";
+    }
     o << elem_single;
-    if (!table) emit_scalar_outputs(o, "mut_vars", "    ", "if (idx == 0) ");
+    const char* first = limbs ? "if (idx == 0 && live) " : "if (idx == 0) ";
+    if (!table) emit_scalar_outputs(o, "mut_vars", "    ", first);
     o << "  }\n}\n\n";
     // batched: instance k uses vars[k * NV ..], mut_vars[k * NM ..] and elements [prefix[k], prefix[k+1]);
     // its scalars are evaluated per element
     o << "__global__ void " << bounds << "\n    " << name
       << "_batched_kernel(const ConstPolyPtr* __restrict__ vars_all, const PolyPtr* __restrict__ mut_vars_all, "
          "const unsigned long long* __restrict__ prefix, unsigned int instances, bool is_first, "
-         "uint32_t* __restrict__ local) {\n";
-    o << "  (void)local;\n";
+         "char* __restrict__ spill) {\n";
+    o << "  (void)spill;\n";
     if (spills)
-      o << "  uint4* __restrict__ spill = reinterpret_cast<uint4*>(reinterpret_cast<char*>(local) + " << table_bytes()
-        << ") + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;\n";
+      o << "  const uint32_t me = blockIdx.x * blockDim.x + threadIdx.x;\n";
     o << "  const uint64_t total = prefix[instances];\n";
     o << "  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;\n";
-    o << "  for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total; g += stride) {\n";
+    if (limbs) {
+      o << "  for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x; base < total; base += stride) {\n";
+      o << "    const bool live = base + threadIdx.x < total;\n";
+      o << "    const uint64_t g = live ? base + threadIdx.x : total - 1;\n";
+    } else {
+      o << "  for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total; g += stride) {\n";
+    }
     o << "    const unsigned int k = zkp::fused::instance_of(prefix, instances, g);\n";
     o << "    const uint64_t idx = g - prefix[k];\n";
     o << "    const ConstPolyPtr* vars = vars_all + (uint64_t)k * " << nv << ";\n";
@@ -791,14 +948,20 @@ struct Emitter {
     emit_views(o, "vars", "mut_vars", "    ", true);
     if (table) {
       // no table per instance: the element code reads scalars from one; give it a local copy
-      o << "    uint32_t scalars_buf[" << scalar_order.size() * 8 << "];\n";
-      for (uint64_t id : scalar_order) o << "    " << tmp(id) << ".store(scalars_buf + " << scalar_index.at(id) * 8 << ");\n";
+      o << "    uint32_t scalars_buf[" << scalar_order.size() * entry_words() << "];\n";
+      for (uint64_t id : scalar_order)
+        o << "    zkp::fused::put_entry(scalars_buf + " << scalar_index.at(id) * entry_words() << ", " << tmp(id) << ");\n";
       o << "    const uint32_t* scalars = scalars_buf;\n";
     }
     o << elem_batched;
-    emit_scalar_outputs(o, "mut_vars", "    ", "if (idx == 0) ");
+    emit_scalar_outputs(o, "mut_vars", "    ", first);
     o << "  }\n}\n}  // namespace\n\n";
-    const char* grid = spills ? "zkp::fused::grid_capped(len, " : "zkp::fused::grid_for(len";
+    // separate arguments, so that the table is known not to change and is read by scalar loads
+    const std::string spill =
+        spills ? "static_cast<char*>(local_buffer) + " + std::to_string(table_bytes()) : std::string("nullptr");
+    // enough workgroups to fill 256 CUs several times over, or those that the spill slots are sized for
+    const std::string cap = std::to_string(spills ? blocks : 256u * 64u * 256u / threads());
+    auto grid = [&](const char* n) { return std::string("zkp::fused::grid_capped(") + n + ", " + wg + ", " + cap + ")"; };
     o << "extern \"C\" hipError_t " << name
       << "(const ConstPolyPtr* vars, const PolyPtr* mut_vars, unsigned long long len, bool is_first, "
          "void* local_buffer, hipStream_t stream) {\n";
@@ -806,11 +969,11 @@ struct Emitter {
     o << "  if (mut_vars == nullptr" << (nv ? " || vars == nullptr" : "") << (local_bytes ? " || local_buffer == nullptr" : "")
       << ") return hipErrorInvalidValue;\n";
     if (table)
-      o << "  hipLaunchKernelGGL(" << name << "_scalars_kernel, dim3(1), dim3(1), 0, stream, vars, mut_vars, "
+      o << "  hipLaunchKernelGGL(" << name << "_scalars_kernel, dim3(1), dim3(64), 0, stream, vars, mut_vars, "
            "static_cast<uint32_t*>(local_buffer));\n";
-    o << "  hipLaunchKernelGGL(" << name << "_kernel, dim3(" << grid << (spills ? std::to_string(blocks) : "")
-      << ")), dim3(zkp::fused::THREADS), 0, stream, vars, mut_vars, len, is_first, "
-         "static_cast<uint32_t*>(local_buffer));\n";
+    o << "  hipLaunchKernelGGL(" << name << "_kernel, dim3(" << grid("len") << "), dim3(" << wg << "), 0, stream, vars, mut_vars, len, is_first, "
+         "static_cast<const uint32_t*>(local_buffer), "
+      << spill << ");\n";
     o << "  return hipGetLastError();\n}\n\n";
     o << "// instances k < n: vars[k*" << nv << " ..], mut_vars[k*" << nm
       << " ..] (device arrays), prefix[k] = sum of earlier lengths (device, n+1 entries),\n"
@@ -821,11 +984,8 @@ struct Emitter {
     o << "  if (instances == 0 || total == 0) return hipSuccess;\n";
     o << "  if (mut_vars == nullptr || prefix == nullptr" << (nv ? " || vars == nullptr" : "")
       << (spills ? " || local_buffer == nullptr" : "") << ") return hipErrorInvalidValue;\n";
-    o << "  hipLaunchKernelGGL(" << name << "_batched_kernel, dim3("
-      << (spills ? std::string("zkp::fused::grid_capped(total, ") + std::to_string(blocks) + ")"
-                 : std::string("zkp::fused::grid_for(total)"))
-      << "), dim3(zkp::fused::THREADS), 0, stream, vars, mut_vars, prefix, instances, is_first, "
-         "static_cast<uint32_t*>(local_buffer));\n";
+    o << "  hipLaunchKernelGGL(" << name << "_batched_kernel, dim3(" << grid("total") << "), dim3(" << wg << "), 0, stream, vars, mut_vars, prefix, instances, is_first, "
+      << spill << ");\n";
     o << "  return hipGetLastError();\n}\n\n";
     o << "// number of vars / mut_vars the kernel expects\n";
     o << "extern \"C\" void " << name << "_arity(unsigned int* out2) { out2[0] = " << nv << "; out2[1] = " << nm

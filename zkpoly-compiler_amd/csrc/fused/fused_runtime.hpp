@@ -5,11 +5,10 @@
 
 #include "../common/poly_ptr.hpp"
 #include "../field/bn254.hpp"
+#include "../field/fr29.hpp"
 
 namespace zkp {
 namespace fused {
-
-constexpr int THREADS = 256;
 
 // PolyPtr -> index map (iter.cuh:309-327: a rotation becomes offset = len - rotate).
 template <class P>
@@ -22,33 +21,147 @@ __device__ __forceinline__ PolyView view(const P& p) {
   return v;
 }
 
-// grid-stride launches: enough waves to fill 256 CUs several times over
-inline unsigned grid_for(uint64_t n) {
-  uint64_t g = (n + THREADS - 1) / THREADS;
-  const uint64_t cap = 256 * 64;
+// grid-stride launches: at most `cap` workgroups
+inline unsigned grid_capped(uint64_t n, unsigned threads, unsigned cap) {
+  const uint64_t g = (n + threads - 1) / threads;
   return (unsigned)(g < cap ? (g ? g : 1) : cap);
 }
 
-// grid of a kernel that keeps per-thread spill slots: at most `cap` workgroups
-inline unsigned grid_capped(uint64_t n, unsigned cap) {
-  const unsigned g = grid_for(n);
-  return g < cap ? g : cap;
+// Spill slots of generated kernels: slot s of a thread is two 16-byte planes and,
+// behind those of all slots, one of 4 bytes, each lane-contiguous over the `threads`
+// threads of the kernel's capped grid, so a wave's spill or reload is coalesced.
+// `me` is the thread's global index.  A plane's start is the same on all lanes and
+// stays on the scalar unit, hidden from the compiler, which otherwise forms every
+// plane's lane address before the loop and keeps them all in scratch.
+template <class T>
+__device__ __forceinline__ T& spill_at(char* spill, uint64_t plane_bytes, uint32_t me) {
+  asm volatile("" : "+s"(plane_bytes));
+  return *reinterpret_cast<T*>(spill + plane_bytes + me * (uint32_t)sizeof(T));
+}
+__device__ __forceinline__ void spill_store(char* spill, uint32_t me, uint64_t s, uint64_t slots, uint64_t threads, const Fr29& x) {
+  spill_at<uint4>(spill, 32 * s * threads, me) = make_uint4((u32)x.l[0], (u32)x.l[1], (u32)x.l[2], (u32)x.l[3]);
+  spill_at<uint4>(spill, (32 * s + 16) * threads, me) = make_uint4((u32)x.l[4], (u32)x.l[5], (u32)x.l[6], (u32)x.l[7]);
+  spill_at<int32_t>(spill, (32 * slots + 4 * s) * threads, me) = x.l[8];
+}
+__device__ __forceinline__ Fr29 spill_load(char* spill, uint32_t me, uint64_t s, uint64_t slots, uint64_t threads) {
+  const uint4 a = spill_at<uint4>(spill, 32 * s * threads, me), b = spill_at<uint4>(spill, (32 * s + 16) * threads, me);
+  return Fr29{{(int32_t)a.x, (int32_t)a.y, (int32_t)a.z, (int32_t)a.w, (int32_t)b.x, (int32_t)b.y, (int32_t)b.z,
+               (int32_t)b.w, spill_at<int32_t>(spill, (32 * slots + 4 * s) * threads, me)}};
 }
 
-// Spill slots of generated kernels: slot s of a thread is two 16-byte planes,
-// each plane lane-contiguous over the `threads` threads of the kernel's capped
-// grid, so a wave's spill or reload is one coalesced 1 KiB access per plane.
-// `base` is the slot area already offset by the thread's global index.
-__device__ __forceinline__ void spill_store(uint4* base, unsigned s, uint64_t threads, const Fr& x) {
-  base[(2ull * s) * threads] = make_uint4(x.v[0], x.v[1], x.v[2], x.v[3]);
-  base[(2ull * s + 1) * threads] = make_uint4(x.v[4], x.v[5], x.v[6], x.v[7]);
+// ---------------------------------------------------------------- kernels in 29-bit limbs
+//
+// Values are up: 32 x 2^256 mod r (fr29.hpp); the generator keeps their ranges.
+
+__device__ __forceinline__ Fr29 load_up(const uint32_t* p) { return Fr29::from_words<5>(Fr::load(p).v); }
+
+// Element idx of a view.  The address is taken as a distance from a kernel argument
+// (any), hidden from the compiler: a pointer read from memory is accessed as a flat
+// one, and an address that is used again is otherwise kept in registers, or in
+// scratch, from the first use to the last.
+__device__ __forceinline__ uint32_t* element(const PolyView& v, uint64_t idx, const void* anchor) {
+  int64_t d = reinterpret_cast<char*>(v.elem(idx)) - reinterpret_cast<const char*>(anchor);
+  asm volatile("" : "+v"(d));
+  return reinterpret_cast<uint32_t*>(const_cast<char*>(reinterpret_cast<const char*>(anchor)) + d);
 }
-__device__ __forceinline__ Fr spill_load(const uint4* base, unsigned s, uint64_t threads) {
-  const uint4 a = base[(2ull * s) * threads], b = base[(2ull * s + 1) * threads];
-  Fr r;
-  r.v[0] = a.x; r.v[1] = a.y; r.v[2] = a.z; r.v[3] = a.w;
-  r.v[4] = b.x; r.v[5] = b.y; r.v[6] = b.z; r.v[7] = b.w;
+__device__ __forceinline__ Fr29 load_up(const PolyView& v, uint64_t idx, const void* anchor) {
+  asm volatile("" : "+v"(idx));
+  return load_up(element(v, idx, anchor));
+}
+
+// x as a product's second operand: hides from the compiler that carried limbs are
+// not negative, or it multiplies them as unsigned by the other operand's signed
+// limbs, in four instructions for one.
+__device__ __forceinline__ Fr29 factor(Fr29 x) {
+#pragma unroll
+  for (int i = 0; i < 9; i++) asm("" : "+v"(x.l[i]));
+  return x;
+}
+
+// A scalar that every lane computes with: kept on the vector unit, the scalar unit
+// has no 64-bit multiply-add.
+__device__ __forceinline__ Fr29 scalar_in(const uint32_t* p) { return factor(load_up(p)); }
+
+__device__ __forceinline__ Fr29 neg(const Fr29& x) {
+  Fr29 r;
+#pragma unroll
+  for (int i = 0; i < 9; i++) r.l[i] = -x.l[i];
   return r;
+}
+__device__ __forceinline__ Fr29 pick(bool c, const Fr29& a, const Fr29& b) {
+  Fr29 r;
+#pragma unroll
+  for (int i = 0; i < 9; i++) r.l[i] = c ? a.l[i] : b.l[i];
+  return r;
+}
+// x^e, x normalised and within 33 r
+__device__ __forceinline__ Fr29 pow(Fr29 x, uint64_t e) {
+  if (e == 0) return Fr29::from_words<5>(Fr::one().v);
+  Fr29 r = x;
+  bool started = false;
+  for (;; e >>= 1) {
+    if (e & 1) {
+      r = started ? Fr29::mul(r, factor(x)) : x;
+      started = true;
+    }
+    if (e == 1) return r;
+    x = Fr29::mul(x, factor(x));
+  }
+}
+
+// The canonical element of an up value: (x + c r) / 32 with c = -q + k, q as in
+// reduce() and 0 <= k < 32 making the sum divisible (r = 1 mod 2^28), which is
+// below (1.0002 + 31) r / 32; then one conditional subtraction.
+__device__ __forceinline__ Fr down(const Fr29& x) {
+  const int32_t top = x.l[8] + (x.l[7] >> 29);
+  const int32_t q = (int32_t)floorf((float)top * (1.0f / 3171406.449f) - 0x1p-13f);
+  const int32_t c = ((q - x.l[0]) & 31) - q;
+  Fr29 t;
+  int64_t acc = 0;
+#pragma unroll
+  for (int i = 0; i < 9; i++) {
+    acc += (int64_t)-c * Fr29::NEG_R[i] + x.l[i];
+    t.l[i] = i < 8 ? (int32_t)((u32)acc & (u32)Fr29::MASK) : (int32_t)acc;
+    acc >>= 29;
+  }
+#pragma unroll
+  for (int i = 0; i < 9; i++)
+    t.l[i] = (int32_t)((u32)t.l[i] >> 5 | (i < 8 ? ((u32)t.l[i + 1] & 31) << 24 : 0));
+  Fr y;
+  t.to_words(y.v);
+  return Fr::reduce_once(y);
+}
+
+__device__ __forceinline__ void store_down(const Fr29& x, const PolyView& v, uint64_t idx, bool live,
+                                           const void* anchor) {
+  const Fr y = down(x);
+  asm volatile("" : "+v"(idx));
+  if (live) y.store(element(v, idx, anchor));
+}
+
+// Entry of the scalar table: nine limbs in 12 words, as computed (put_raw), then
+// below 1.0002 r.
+__device__ __forceinline__ void put_raw(uint32_t* p, const Fr29& x) {
+#pragma unroll
+  for (int i = 0; i < 9; i++) p[i] = (u32)x.l[i];
+}
+__device__ __forceinline__ void put_entry(uint32_t* p, const Fr29& x) {
+  const Fr29 y = x.reduce();
+#pragma unroll
+  for (int i = 0; i < 9; i++) p[i] = (u32)y.l[i];
+}
+__device__ __forceinline__ Fr29 entry(const uint32_t* p) {
+  Fr29 x;
+#pragma unroll
+  for (int i = 0; i < 9; i++) x.l[i] = (int32_t)p[i];
+  return x;
+}
+
+// The table's entries reduced, by one workgroup that has written them.
+__device__ __forceinline__ void reduce_entries(uint32_t* table, unsigned count) {
+  __threadfence();
+  __syncthreads();
+  for (unsigned t = threadIdx.x; t < count; t += blockDim.x) put_entry(table + 12 * t, entry(table + 12 * t));
 }
 
 // largest k < n with prefix[k] <= g (prefix has n + 1 non-decreasing entries)

@@ -245,6 +245,39 @@ def random_graph(seed: int, vertices: int = 600, poly_inputs: int = 12, scalar_i
     return g.to_json()
 
 
+def graph_ranges(coef: bool = False) -> str:
+    """Long runs of additions, subtractions and negations with no product between
+    them, products of such sums, every small power, and enough scalars for the table:
+    what the ranges of the 29-bit limb code have to follow.
+
+    vars [a, b, s0 .. s4]; mut_vars: polynomials, then two scalars.
+    """
+    g = GraphBuilder("Coef" if coef else "Lagrange")
+    a, b = g.input(), g.input()
+    s = [g.input(scalar=True) for _ in range(5)]
+    up, down = a, b
+    for k in range(12):  # up to 2^12 a, and as far below zero
+        up = g.bin("Pp", "Add", up, up)
+        down = g.neg(g.bin("Pp", "Sub", up, down)) if k % 3 else g.bin("Pp", "Sub", down, up)
+    wide = g.bin("Pp", "Mul", up, down)
+    total = s[0]
+    for k in range(30):
+        total = g.bin("Ss", ("Add", "Sub", "Add")[k % 3], total, s[k % 5] if k % 2 else total)
+    total = g.bin("Ss", "Mul", g.neg(total, scalar=True), g.bin("Ss", "Sub", s[1], total))
+    outs = [up, down, wide, g.neg(g.neg(down))]
+    for op in ("Add", "Sub", "SubBy", "Mul"):
+        outs.append(g.bin("Sp", op, total, down))
+        outs.append(g.bin("Sp", op, s[2], wide))
+    for e in (0, 1, 2, 3, 5, 64):
+        outs.append(g.pow(down, e))
+    outs.append(g.bin("Pp", "Mul", g.neg(up), g.bin("Pp", "Sub", outs[-1], g.bin("Pp", "Add", up, wide))))
+    for o in outs:
+        g.output(o)
+    g.output(total, scalar=True)
+    g.output(g.neg(s[4], scalar=True), scalar=True)
+    return g.to_json()
+
+
 def demo_kernels() -> list[tuple[str, str]]:
     return [
         (graph_ab_gamma_c_minus_z(), "fused_arith_abgcz"),
@@ -253,6 +286,8 @@ def demo_kernels() -> list[tuple[str, str]]:
         (graph_pipelined_abgcz(), "fused_arith_pipe_abgcz"),
         (graph_pipelined_mixed(), "fused_arith_pipe_mixed"),
         (graph_pipelined_coef(), "fused_arith_pipe_coef"),
+        (graph_ranges(False), "fused_arith_ranges"),
+        (graph_ranges(True), "fused_arith_ranges_coef"),
     ]
 
 
