@@ -853,7 +853,7 @@ __global__ void __launch_bounds__(PASS_THREADS)
 //   colbase(lo, m) = w^(lo * 2^(L-1-s0-m)),  small(j) = w^(j * 2^(L-d)).
 // A workgroup walks consecutive tiles, so lo grows by C from one tile to the
 // next and colbase is advanced with one product per (column, stage).
-constexpr int RTILE_LOG = 10;          // 32 KiB of tile + 16 KiB of stage twiddles
+constexpr int RTILE_LOG = 10;          // 36 KiB of tile; two workgroups per CU with the tables
 constexpr uint32_t RMAX_C_LOG = 5;     // <= 32 columns
 constexpr uint32_t RMAX_D = RTILE_LOG - 1;
 constexpr uint32_t RMAX_COLBASE = 160;  // max C * d over plans with c <= 5, c + d <= 10
@@ -905,20 +905,32 @@ __global__ void __launch_bounds__(HEAD_THREADS)
   head_walk(L, v, log_n, t, g, blockIdx.x);
 }
 
+constexpr uint32_t RTABLE = 3u << (RTILE_LOG - 3);  // twiddles of a shared round: 3 C 2^m, m <= d - 3
 struct RPassLds {
-  uint4 x0[1 << RTILE_LOG], x1[1 << RTILE_LOG];              // tile
-  uint4 w0[1 << (RTILE_LOG - 1)], w1[1 << (RTILE_LOG - 1)];  // twiddles of the current stage
-  uint4 r0[1 << (RMAX_D - 1)], r1[1 << (RMAX_D - 1)];        // small roots
-  uint4 b0[RMAX_COLBASE], b1[RMAX_COLBASE];                  // colbase of the current tile, [c * d + m]
-  uint4 z0[RMAX_COLBASE], z1[RMAX_COLBASE];                  // colbase at lo_block 0
+  uint4 x0[1 << RTILE_LOG], x1[1 << RTILE_LOG];  // tile: limbs 0-3, 4-7 and 8, as all tables but z
+  int32_t x2[1 << RTILE_LOG];
+  uint4 w0[RTABLE], w1[RTABLE];  // twiddles of the current round
+  int32_t w2[RTABLE];
+  uint4 r0[1 << (RMAX_D - 1)], r1[1 << (RMAX_D - 1)];  // small roots
+  int32_t r2[1 << (RMAX_D - 1)];
+  uint4 b0[RMAX_COLBASE], b1[RMAX_COLBASE];  // colbase of the current tile, [c * d + m]
+  int32_t b2[RMAX_COLBASE];
+  uint4 z0[RMAX_COLBASE], z1[RMAX_COLBASE];  // colbase at lo_block 0 (words)
 };
+static_assert(2 * sizeof(RPassLds) <= 160 * 1024, "two workgroups per CU");
 
 // Stages [s0, s0 + d) over tiles [blockIdx.x * per_block, ...) of 2^d rows x
-// 2^c_log columns, tile geometry as dit_tile.
-// 512 threads (one butterfly each per stage at the 1024-element tile); lazy
-// butterflies, values in [0, 4p) between stages and passes, canonical stores
-// in the transform's last pass (final_pass).
-constexpr int RPASS_THREADS = 512;
+// 2^c_log columns, tile geometry and quads as dit_tile_r4, in Fr29: memory to
+// registers in the first round, LDS between rounds, memory from the last.
+// Multipliers carry their factor 32 (fr29.hpp), so colbase * small is one product
+// and a multiplier again.  A round whose quads share twiddles forms each once in a
+// table; in the last one no two quads share any, and a thread forms its own.
+// Bound by products: two stages cost a quad four for the butterflies and up to three
+// for the twiddles.  At 2^21 radix-2 stages in 32-bit limbs, each with a table and
+// two barriers, took 173 + 186 us for the two
+// passes, these 124 + 135.
+constexpr int RPASS_THREADS = 256;
+static_assert(4 * RPASS_THREADS >= 1 << RTILE_LOG, "a quad per thread");
 __global__ void __launch_bounds__(RPASS_THREADS)
     rdit_pass(PolyView v, const uint32_t* __restrict__ pq, uint32_t pq_deg, const uint32_t* __restrict__ omegas,
               uint32_t log_n, uint32_t s0, uint32_t d, uint32_t c_log, uint64_t tiles, uint32_t per_block,
@@ -931,6 +943,8 @@ __global__ void __launch_bounds__(RPASS_THREADS)
   if (first >= tiles) return;
   const uint64_t last = first + per_block < tiles ? first + per_block : tiles;
   const uint64_t lo_blocks = s0 ? ((1ull << s0) >> c_log) : 1;
+  const bool wraps = v.offset + v.len > v.whole_len;
+  auto up = [](const Fr& x) { return Fr29::from_words<5>(x.v); };
 
   if (s0) {
     const uint64_t lob = first % lo_blocks;
@@ -938,92 +952,108 @@ __global__ void __launch_bounds__(RPASS_THREADS)
       const uint32_t c = e / d, m = e - c * d;
       const uint32_t sh = log_n - 1 - s0 - m;
       lds_put(S.z0, S.z1, e, pow_ladder(omegas, c, sh));
-      lds_put(S.b0, S.b1, e, pow_ladder(omegas, lob * C + c, sh));
+      limbs_put(S.b0, S.b1, S.b2, e, up(pow_ladder(omegas, lob * C + c, sh)));
     }
   }
   build_small_roots(S.r0, S.r1, pq, pq_deg, omegas, log_n, d);  // ends with a barrier
+  for (uint32_t j = threadIdx.x; j < (R >> 1); j += RPASS_THREADS)
+    limbs_put(S.r0, S.r1, S.r2, j, up(lds_get(S.r0, S.r1, j)));
 
+  // w^((lo + kp 2^s0) 2^(log_n - 1 - s0 - m)) of column c
+  auto twiddle = [&](uint32_t m, uint32_t c, uint32_t kp) -> Fr29 {
+    const Fr29 r = limbs_get(S.r0, S.r1, S.r2, kp << (d - 1 - m));
+    return s0 ? Fr29::mul(r, limbs_get(S.b0, S.b1, S.b2, c * d + m)) : r;
+  };
   for (uint64_t tile = first; tile < last; tile++) {
-    uint64_t base, cstride, kstride;
-    if (s0 == 0) {
-      base = (tile << c_log) << d;
-      cstride = R;
-      kstride = 1;
-    } else {
-      const uint64_t hi = tile / lo_blocks;
-      const uint64_t lo_block = tile % lo_blocks;
-      base = lo_block * C + (hi << (s0 + d));
-      cstride = 1;
-      kstride = 1ull << s0;
-      if (tile != first) {  // lo grows by C, or wraps to 0 with the next hi
-        const bool wrap = lo_block == 0;
-        for (uint32_t e = threadIdx.x; e < C * d; e += RPASS_THREADS) {
-          const uint32_t m = e % d;
-          const Fr nb = wrap ? lds_get(S.z0, S.z1, e)
-                             : lds_get(S.b0, S.b1, e) * Fr::load(omegas + (c_log + log_n - 1 - s0 - m) * 8);
-          lds_put(S.b0, S.b1, e, nb);
+    const TileGeom geo = tile_geom(s0, d, c_log, tile);
+    if (s0 && tile != first) {  // lo grows by C, or wraps to 0 with the next hi
+      const bool wrap = tile % lo_blocks == 0;
+      for (uint32_t e = threadIdx.x; e < C * d; e += RPASS_THREADS) {
+        const uint32_t m = e % d;
+        const Fr29 nb = wrap ? up(lds_get(S.z0, S.z1, e))
+                             : Fr29::mul(limbs_get(S.b0, S.b1, S.b2, e),
+                                         up(Fr::load(omegas + (c_log + log_n - 1 - s0 - m) * 8)));
+        limbs_put(S.b0, S.b1, S.b2, e, nb);
+      }
+    }
+    __syncthreads();
+    uint32_t m = 0;
+    for (; m + 1 < d; m += 2) {
+      const uint32_t h = 1u << m;
+      const bool from_memory = m == 0, to_memory = m + 2 == d;
+      if (!to_memory) {
+        for (uint32_t e = threadIdx.x; e < 3 * (C << m); e += RPASS_THREADS) {
+          const bool second = e >= (C << m);  // of stage m + 1
+          const uint32_t i = second ? e - (C << m) : e;
+          const uint32_t mm = second ? m + 1 : m;
+          limbs_put(S.w0, S.w1, S.w2, e, twiddle(mm, i >> mm, i & ((1u << mm) - 1)));
+        }
+        __syncthreads();
+      }
+      if (threadIdx.x < (T >> 2)) {
+        const uint32_t c = threadIdx.x & (C - 1), qr = threadIdx.x >> c_log;
+        const uint32_t kk = qr & (h - 1);
+        const uint32_t k0 = ((qr >> m) << (m + 2)) | kk;
+        const uint32_t pos = (k0 << c_log) | c;
+        uint64_t row[4];
+        if (from_memory || to_memory)
+          pass_rows(v, wraps, v.offset + tile_index(geo.base, geo.cstride, geo.kstride, c, k0), geo.kstride << m, row);
+        Fr29 x0, x1, x2, x3;
+        if (from_memory) {
+          const Fr y0 = Fr::load(v.ptr + row[0]), y1 = Fr::load(v.ptr + row[1]);
+          const Fr y2 = Fr::load(v.ptr + row[2]), y3 = Fr::load(v.ptr + row[3]);
+          x0 = Fr29::from_words<0>(y0.v);
+          x1 = Fr29::from_words<0>(y1.v);
+          x2 = Fr29::from_words<0>(y2.v);
+          x3 = Fr29::from_words<0>(y3.v);
+        } else {
+          x0 = limbs_get(S.x0, S.x1, S.x2, pos).norm();
+          x1 = limbs_get(S.x0, S.x1, S.x2, pos + (h << c_log));
+          x2 = limbs_get(S.x0, S.x1, S.x2, pos + (2 * h << c_log)).norm();
+          x3 = limbs_get(S.x0, S.x1, S.x2, pos + (3 * h << c_log));
+        }
+        const uint32_t at1 = c * h + kk, at2 = C * h + c * 2 * h + kk;
+        const Fr29 w1 = to_memory ? twiddle(m, c, kk) : limbs_get(S.w0, S.w1, S.w2, at1);
+        const Fr29 t1 = Fr29::mul(x1, w1), t3 = Fr29::mul(x3, w1);
+        const Fr29 w2 = to_memory ? twiddle(m + 1, c, kk) : limbs_get(S.w0, S.w1, S.w2, at2);
+        const Fr29 t2 = Fr29::mul(x2 + t3, w2);
+        const Fr29 w3 = to_memory ? twiddle(m + 1, c, kk + h) : limbs_get(S.w0, S.w1, S.w2, at2 + h);
+        const Fr29 t4 = Fr29::mul(x2 - t3, w3);
+        const Fr29 a0 = x0 + t1, a1 = x0 - t1;
+        if (to_memory) {
+          pass_store(v.ptr + row[0], a0 + t2, final_pass);
+          pass_store(v.ptr + row[1], a1 + t4, final_pass);
+          pass_store(v.ptr + row[2], a0 - t2, final_pass);
+          pass_store(v.ptr + row[3], a1 - t4, final_pass);
+        } else {
+          limbs_put(S.x0, S.x1, S.x2, pos, a0 + t2);
+          limbs_put(S.x0, S.x1, S.x2, pos + (h << c_log), a1 + t4);
+          limbs_put(S.x0, S.x1, S.x2, pos + (2 * h << c_log), a0 - t2);
+          limbs_put(S.x0, S.x1, S.x2, pos + (3 * h << c_log), a1 - t4);
         }
       }
-    }
-    for (uint32_t e = threadIdx.x; e < T; e += RPASS_THREADS) {
-      uint32_t c, k;
-      if (cstride == 1) {
-        c = e & (C - 1);
-        k = e >> c_log;
-      } else {
-        k = e & (R - 1);
-        c = e >> d;
-      }
-      const uint4* src = reinterpret_cast<const uint4*>(v.elem(tile_index(base, cstride, kstride, c, k)));
-      const uint32_t pos = (k << c_log) | c;
-      S.x0[pos] = src[0];
-      S.x1[pos] = src[1];
-    }
-    __syncthreads();
-    for (uint32_t m = 0; m < d; m++) {
-      const uint32_t h = 1u << m;
-      for (uint32_t e = threadIdx.x; e < (C << m); e += RPASS_THREADS) {
-        const uint32_t c = e >> m, kp = e & (h - 1);
-        Fr w = lds_get(S.r0, S.r1, kp << (d - 1 - m));
-        if (s0) w = lds_get(S.b0, S.b1, c * d + m) * w;
-        lds_put(S.w0, S.w1, e, w);
-      }
       __syncthreads();
+    }
+    if (m < d) {  // odd last stage, radix-2
       for (uint32_t b = threadIdx.x; b < (T >> 1); b += RPASS_THREADS) {
-        const uint32_t c = b & (C - 1);
-        const uint32_t q = b >> c_log;
-        const uint32_t ka = ((q >> m) << (m + 1)) | (q & (h - 1));
-        const uint32_t pa = (ka << c_log) | c;
-        const uint32_t pb = ((ka + h) << c_log) | c;
-        const Fr w = lds_get(S.w0, S.w1, (c << m) | (ka & (h - 1)));
-        const Fr x = Fr::reduce_2p(lds_get(S.x0, S.x1, pa));
-        const Fr t = Fr::mul_lazy(lds_get(S.x0, S.x1, pb), w);
-        lds_put(S.x0, S.x1, pa, Fr::add_raw(x, t));
-        lds_put(S.x0, S.x1, pb, Fr::sub_2p(x, t));
+        const uint32_t c = b & (C - 1), ka = b >> c_log;  // rows ka and ka + 2^m
+        uint64_t row[2];
+        pass_rows(v, wraps, v.offset + tile_index(geo.base, geo.cstride, geo.kstride, c, ka), geo.kstride << m, row);
+        Fr29 x, y;
+        if (m == 0) {
+          const Fr xw = Fr::load(v.ptr + row[0]), yw = Fr::load(v.ptr + row[1]);
+          x = Fr29::from_words<0>(xw.v);
+          y = Fr29::from_words<0>(yw.v);
+        } else {
+          x = limbs_get(S.x0, S.x1, S.x2, b);
+          y = limbs_get(S.x0, S.x1, S.x2, b + (T >> 1));
+        }
+        const Fr29 t = Fr29::mul(y, twiddle(m, c, ka));
+        pass_store(v.ptr + row[0], x + t, final_pass);
+        pass_store(v.ptr + row[1], x - t, final_pass);
       }
-      __syncthreads();
+      __syncthreads();  // the colbase and the tile are written again
     }
-    for (uint32_t e = threadIdx.x; e < T; e += RPASS_THREADS) {
-      uint32_t c, k;
-      if (cstride == 1) {
-        c = e & (C - 1);
-        k = e >> c_log;
-      } else {
-        k = e & (R - 1);
-        c = e >> d;
-      }
-      uint4* dst = reinterpret_cast<uint4*>(v.elem(tile_index(base, cstride, kstride, c, k)));
-      const uint32_t pos = (k << c_log) | c;
-      if (final_pass) {
-        const Fr y = Fr::reduce_4p(lds_get(S.x0, S.x1, pos));
-        dst[0] = make_uint4(y.v[0], y.v[1], y.v[2], y.v[3]);
-        dst[1] = make_uint4(y.v[4], y.v[5], y.v[6], y.v[7]);
-      } else {
-        dst[0] = S.x0[pos];
-        dst[1] = S.x1[pos];
-      }
-    }
-    __syncthreads();
   }
 }
 
