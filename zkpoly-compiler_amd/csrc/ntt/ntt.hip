@@ -516,21 +516,22 @@ __device__ __forceinline__ void head_store(const HeadLds& L, const PolyView& v, 
 // One tile pair {M, rev M} per workgroup.  The caller has written L.r
 // (visible after the first barrier below).
 // (256 threads.)
+template <int NT>
 __device__ __forceinline__ void head_tile(HeadLds& L, const PolyView& v, uint32_t log_n, uint32_t t, uint64_t M) {
   const uint32_t mbits = log_n - 2 * t;
   const uint64_t Mr = mbits ? (__brevll(M) >> (64 - mbits)) : 0;
   if (M > Mr) return;  // the pair is handled by block Mr (uniform per block)
   const bool pair = M != Mr;
   const uint32_t shift_a = log_n - t;
-  static_assert(2 * HEAD_W * HEAD_W == 8 * THREADS, "eight staged loads per thread");
-  HeadStaged g[8];
+  constexpr uint32_t loads = 2 * HEAD_W * HEAD_W / NT;
+  HeadStaged g[loads];
 #pragma unroll
-  for (uint32_t j = 0; j < 8; j++) g[j] = head_fetch<THREADS>(v, t, shift_a, M, Mr, j);
+  for (uint32_t j = 0; j < loads; j++) g[j] = head_fetch<NT>(v, t, shift_a, M, Mr, j);
 #pragma unroll
-  for (uint32_t j = 0; j < 8; j++) head_place<THREADS>(L, t, pair, j, g[j]);
+  for (uint32_t j = 0; j < loads; j++) head_place<NT>(L, t, pair, j, g[j]);
   __syncthreads();
-  head_stages<THREADS>(L, t, pair);
-  head_store<THREADS>(L, v, t, shift_a, M, Mr, pair);
+  head_stages<NT>(L, t, pair);
+  head_store<NT>(L, v, t, shift_a, M, Mr, pair);
 }
 
 // L.r[i] = tw[i << (log_n - t)] for i < 2^(t - 1)
@@ -624,11 +625,17 @@ static inline uint32_t head_stream_g(uint32_t mbits) {
   return g;
 }
 
-__global__ void __launch_bounds__(THREADS)
+// One tile pair per workgroup: a quad per thread and round.  Up to HEAD_PAIR_MAX
+// tile bits there is at most a workgroup per CU and nothing to load ahead; a pair's
+// chain of rounds then runs on twice the waves (2^12: 13.6 us, the walk 17).  From
+// two workgroups per CU on the walk is faster (2^20: 48 us, this 53).
+constexpr uint32_t HEAD_PAIR_MAX = 8;
+constexpr int HEAD_PAIR_THREADS = 512;
+__global__ void __launch_bounds__(HEAD_PAIR_THREADS)
     bitrev_head(PolyView v, const uint32_t* __restrict__ tw, uint32_t log_n, uint32_t t) {
   __shared__ HeadLds L;
   head_twiddles_from_table(L, tw, log_n, t);
-  head_tile(L, v, log_n, t, blockIdx.x);
+  head_tile<HEAD_PAIR_THREADS>(L, v, log_n, t, blockIdx.x);
 }
 
 // Fused bit reversal + first head_t stages of every instance; instance k owns
@@ -1158,6 +1165,19 @@ static void plan_recompute(uint32_t log_n, PlanV2* p) {
   }
 }
 
+// A transform on its own whose tiles are fewer than CUs takes narrower ones, down to
+// runs of four elements (a 128-byte line): a tile's chain of rounds is as long, with
+// fewer of its waves on each SIMD.
+static void spread_tiles(PlanV2* p) {
+  for (int k = 0; k < p->np; k++) {
+    PassPlan& q = p->pass[k];
+    while (q.tiles < 256 && q.c_log > 2) {
+      q.c_log--;
+      q.tiles <<= 1;
+    }
+  }
+}
+
 static inline unsigned grid_for(uint64_t work, unsigned threads, unsigned cap) {
   uint64_t g = (work + threads - 1) / threads;
   if (g > cap) g = cap;
@@ -1208,13 +1228,14 @@ static hipError_t launch_ntt(PolyPtr x, const unsigned int* twiddle, unsigned in
   } else {
     PlanV2 plan;
     plan_v2(log_len, &plan);
+    spread_tiles(&plan);
     if (plan.head_t == 0) {
       hipLaunchKernelGGL(bitrev_kernel, dim3(grid_for(v.len, THREADS, 65536)), dim3(THREADS), 0, stream, v,
                          (uint32_t)log_len);
     } else {
-      if (variant == 2) {
-        hipLaunchKernelGGL(bitrev_head, dim3((unsigned)(1ull << (log_len - 2 * plan.head_t))), dim3(THREADS), 0,
-                           stream, v, twiddle, (uint32_t)log_len, plan.head_t);
+      if (variant == 2 || log_len - 2 * plan.head_t <= HEAD_PAIR_MAX) {
+        hipLaunchKernelGGL(bitrev_head, dim3((unsigned)(1ull << (log_len - 2 * plan.head_t))),
+                           dim3(HEAD_PAIR_THREADS), 0, stream, v, twiddle, (uint32_t)log_len, plan.head_t);
       } else {
         const uint32_t g = head_stream_g((uint32_t)log_len - 2 * plan.head_t);
         hipLaunchKernelGGL(bitrev_head_stream, dim3(1u << g), dim3(HEAD_THREADS), 0, stream, v, twiddle,
