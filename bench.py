@@ -928,17 +928,17 @@ def main():
             "launches": len(dit),
         },
         "int_mul": {
-            "note": "v_mad_u64_u32 rate over the whole step: 136 per Montgomery product, n/2 products per "
-                    "stage; they are about half of the product's VALU instructions, so the binding rate is "
-                    "the VALU issue in valu_issue",
+            "note": "32 x 32-bit multiply-add rate over the whole step: 136 per Montgomery product, n/2 products "
+                    "per stage (in 29-bit limbs a product issues 162); the binding rate is the VALU issue in "
+                    "valu_issue",
             "achieved_mads_per_s": float(f"{int_rate:.4e}"),
             "peak_mads_per_s": INT_MUL_PEAK,
             "frac": round(int_rate / INT_MUL_PEAK, 4),
         },
         "valu_issue": valu_issue(ms_step, dit_avg_ms) if k == 24 else None,
         "bitrev_head_avg_ms": round(sum(per_kind[0]) / max(1, len(per_kind[0])), 5),
-        "valu_rocprof": valu_from_profiles(["dit_pass_r4", "bitrev_head_stream", "k_accumulate0", "k_close_runs",
-                                            "k_reduce_level", "k_reduce_tail", "k_seg_scatter"]),
+        "valu_rocprof": valu_from_profiles(["dit_pass_r4", "bitrev_head_stream", "k_accumulate<false>", "k_close_runs<false>",
+                                            "k_reduce_level", "k_reduce_tail_quad", "k_seg_scatter"]),
     }
     if not args.quick:
         # GPU legs first: in this process, after the 16-thread CPU NTT baseline of
