@@ -41,8 +41,6 @@ struct FrParams {
                                  0x7879462eu, 0x666ea36fu, 0x9a07df2fu, 0x0e0a77c1u};
   static constexpr u32 R2[8] = {0xae216da7u, 0x1bb8e645u, 0xe35c59e3u, 0x53fe3ab1u,
                                 0x53bb8085u, 0x8c49833du, 0x7f4e44a5u, 0x0216d0b1u};
-  static constexpr u32 R3[8] = {0xb4bf0040u, 0x5e94d8e1u, 0x1cfbb6b8u, 0x2a489cbeu,
-                                0xa19fcfedu, 0x893cc664u, 0x7fcc657cu, 0x0cf8594bu};  // 2^768 mod r
 };
 
 struct FqParams {
@@ -54,8 +52,6 @@ struct FqParams {
                                  0x7879462cu, 0x666ea36fu, 0x9a07df2fu, 0x0e0a77c1u};
   static constexpr u32 R2[8] = {0x538afa89u, 0xf32cfc5bu, 0xd44501fbu, 0xb5e71911u,
                                 0x0a417ff6u, 0x47ab1effu, 0xcab8351fu, 0x06d89f71u};
-  static constexpr u32 R3[8] = {0xda1530dfu, 0xb1cd6dafu, 0xa7283db6u, 0x62f210e6u,
-                                0x0ada0afbu, 0xef7f0b0cu, 0x2d592544u, 0x20fd6e90u};  // 2^768 mod q
 };
 
 template <class Params>
@@ -160,61 +156,6 @@ struct Fp {
 
   ZKP_HD Fp dbl() const { return *this + *this; }
 
-  // ---- lazy forms for butterflies: values kept in [0, 4p) (4p < 2^256) ----
-  // limb i of 2p
-  static constexpr u32 p2_limb(int i) { return (Params::P[i] << 1) | (i ? Params::P[i - 1] >> 31 : 0u); }
-
-  // x - 2p if x >= 2p, for x < 4p: result in [0, 2p).
-  ZKP_HD static Fp reduce_2p(const Fp& x) {
-    Fp d;
-    u32 borrow = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) d.v[i] = sbb(x.v[i], p2_limb(i), borrow);
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < 8; i++) r.v[i] = borrow ? x.v[i] : d.v[i];
-    return r;
-  }
-  // [0, 4p) -> canonical.
-  ZKP_HD static Fp reduce_4p(const Fp& x) { return reduce_once(reduce_2p(x)); }
-  // a + b without reduction (the caller keeps the sum below 2^256).
-  ZKP_HD static Fp add_raw(const Fp& a, const Fp& b) {
-    Fp s;
-    u32 c = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) s.v[i] = adc(a.v[i], b.v[i], c);
-    return s;
-  }
-  // a + 2p - b for a, b < 2p: result in (0, 4p).
-  ZKP_HD static Fp sub_2p(const Fp& a, const Fp& b) {
-    Fp d;
-    u32 c = 0, borrow = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) d.v[i] = adc(a.v[i], sbb(p2_limb(i), b.v[i], borrow), c);  // 2p - b >= 0
-    return d;
-  }
-  // Montgomery product without the final subtraction: for a < 4p and b < p
-  // the result a*b*R^-1 (mod p) lies in [0, 2p).
-  ZKP_HD static Fp mul_lazy(const Fp& a, const Fp& b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    return mul_ps_raw(a, b);
-#else
-    return mul_cios64_raw(a, b);
-#endif
-  }
-  // Two independent lazy products (device: interleaved chains).
-  ZKP_HD static void mul_lazy2(const Fp& a0, const Fp& b0, const Fp& a1, const Fp& b1, Fp& r0, Fp& r1) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const Fp a[2] = {a0, a1}, b[2] = {b0, b1};
-    Fp r[2];
-    mul_ps_raw_n<2>(a, b, r);
-    r0 = r[0];
-    r1 = r[1];
-#else
-    r0 = mul_cios64_raw(a0, b0);
-    r1 = mul_cios64_raw(a1, b1);
-#endif
-  }
   // N independent canonical products r[n] = a[n] * b[n].
   template <int N>
   ZKP_HD static void muln(const Fp (&a)[N], const Fp (&b)[N], Fp (&r)[N]) {
@@ -226,28 +167,6 @@ struct Fp {
     for (int n = 0; n < N; n++) r[n] = a[n] * b[n];
 #endif
   }
-  // Two / three independent canonical products.
-  ZKP_HD static void mul2(const Fp& a0, const Fp& b0, const Fp& a1, const Fp& b1, Fp& r0, Fp& r1) {
-    mul_lazy2(a0, b0, a1, b1, r0, r1);
-    r0 = reduce_once(r0);
-    r1 = reduce_once(r1);
-  }
-  ZKP_HD static void mul3(const Fp& a0, const Fp& b0, const Fp& a1, const Fp& b1, const Fp& a2, const Fp& b2, Fp& r0,
-                          Fp& r1, Fp& r2) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const Fp a[3] = {a0, a1, a2}, b[3] = {b0, b1, b2};
-    Fp r[3];
-    mul_ps_raw_n<3>(a, b, r);
-    r0 = reduce_once(r[0]);
-    r1 = reduce_once(r[1]);
-    r2 = reduce_once(r[2]);
-#else
-    r0 = a0 * b0;
-    r1 = a1 * b1;
-    r2 = a2 * b2;
-#endif
-  }
-
   // Montgomery product a*b*R^-1 mod p.
   //
   // Device: product scanning (column-wise) with interleaved reduction.  Each
