@@ -91,6 +91,46 @@ def test_variants_and_tunings(libs, stream, variant, min_col):
             set_tuning(libs, k, DEFAULT_MIN_COL_LOG)
 
 
+@pytest.mark.parametrize("min_col,ks,batch", [
+    (10, (19, 20), (11, 12, 13)), (9, (19, 20), (11, 12, 13)), (8, (20,), (12, 13)), (7, (19,), (12, 13))])
+def test_shallow_passes(libs, stream, min_col, ks, batch):
+    """Tunings that leave passes of one to four stages over up to 1 024 columns,
+    alone from the sizes on whose tiles stay that wide, and batched, where tiles
+    are not narrowed."""
+    from zkpoly_amd.batch import NttBatch
+    from zkpoly_amd.runtime import PolyPtr
+
+    try:
+        for k in ks:
+            set_tuning(libs, k, min_col)
+            n = 1 << k
+            data = random_elements(n, 310 + k)
+            w = random_elements(1, 910 + k)[0]
+            got, _ = gpu_ntt(libs, stream, data, w, rotate=n // 3)
+            assert np.array_equal(got, orc.best_fft(data, w, k, THREADS)), (min_col, k)
+        polys, tables, bufs, want = [], [], [], []
+        for k in batch:
+            set_tuning(libs, k, min_col)
+            n = 1 << k
+            data = random_elements(n, 330 + k)
+            w = random_elements(1, 930 + k)[0]
+            buf, x = device_array(n)
+            tbuf, tw = device_array(n // 2)
+            cpu2gpu(data, x, buf)
+            cpu2gpu(orc.twiddles(n // 2, w), tw, tbuf)
+            polys.append(PolyPtr(buf.addr, n, 0, 0, n))
+            tables.append(tbuf.addr)
+            bufs.append((x, buf, tbuf))
+            want.append(orc.best_fft(data, w, k, THREADS))
+        NttBatch(libs, polys, tables, list(batch)).run(stream)
+        stream.sync()
+        for k, (x, buf, _), expect in zip(batch, bufs, want):
+            assert np.array_equal(gpu2cpu(x, buf), expect), (min_col, k, "batched")
+    finally:
+        for k in ks + batch:
+            set_tuning(libs, k, DEFAULT_MIN_COL_LOG)
+
+
 @pytest.mark.parametrize("k", [21, 23])
 def test_head_variants_at_large_sizes(libs, stream, k):
     """From 2^21 on a head workgroup walks several tile pairs (loads of the next

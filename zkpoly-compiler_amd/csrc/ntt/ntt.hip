@@ -739,12 +739,14 @@ __device__ __forceinline__ void dit_tile_r4(PassLds& L, const PolyView& v, const
   const uint32_t c = threadIdx.x & (C - 1);
   const uint32_t qr = threadIdx.x >> c_log;
   const bool live = threadIdx.x < (T >> 2);
-  // this thread's column modulo 2^s0, the part of a twiddle's exponent that no row adds to
-  const uint64_t lo = (geo.base & ((1ull << s0) - 1)) + (s0 ? c : 0);
-  // words before the table entry of stage s0 + m for rows that are kk modulo 2^m
-  auto entry = [&](uint32_t m, uint32_t kk) -> uint64_t {
+  // a column modulo 2^s0, the part of a twiddle's exponent that no row adds to
+  auto column = [&](uint32_t c) -> uint64_t { return (geo.base & ((1ull << s0) - 1)) + (s0 ? c : 0); };
+  // words before the table entry of stage s0 + m for column lo and rows that are kk modulo 2^m
+  auto entry_of = [&](uint64_t lo, uint32_t m, uint32_t kk) -> uint64_t {
     return (lo + ((uint64_t)kk << s0)) << (log_n - 1 - (s0 + m)) << 3;
   };
+  const uint64_t lo = column(c);
+  auto entry = [&](uint32_t m, uint32_t kk) -> uint64_t { return entry_of(lo, m, kk); };
   uint32_t m = 0;
   Fr w1;
   if (d > 1 && live) w1 = Fr::load(tw + entry(0, 0));
@@ -798,11 +800,13 @@ __device__ __forceinline__ void dit_tile_r4(PassLds& L, const PolyView& v, const
   if (m < d) {  // odd last stage, radix-2
     const uint32_t half = 1u << m;
     for (uint32_t b = threadIdx.x; b < (T >> 1); b += PASS_THREADS) {
-      const uint32_t q = b >> c_log;  // (b and threadIdx.x agree modulo C)
+      // b's own column: a pass of this stage alone may have 1 024 of them, more than threads
+      const uint32_t c = b & (C - 1);
+      const uint32_t q = b >> c_log;
       const uint32_t kk = q & (half - 1);
       const uint32_t ka = ((q >> m) << (m + 1)) | kk;
       const uint32_t pos = (ka << c_log) | c;
-      const Fr w = Fr::load(tw + entry(m, kk));
+      const Fr w = Fr::load(tw + entry_of(column(c), m, kk));
       uint64_t row[2];
       pass_rows(v, wraps, v.offset + tile_index(geo.base, geo.cstride, geo.kstride, c, ka), geo.kstride << m, row);
       Fr29 x, y;  // from LDS in (-2N, 3N): x + t and x - t still fit 32 bits
