@@ -47,6 +47,10 @@ hipError_t zkp_msm_precompute_host(unsigned int window, unsigned int target_wind
 /* Device workspace bytes for zkp_msm_device (0 if the configuration is invalid). */
 unsigned long long zkp_msm_workspace_size(unsigned long long len, unsigned int window, unsigned int target_windows);
 
+/* The smallest workspace that zkp_msm_device and zkp_msm_device_enqueue accept (0 if the configuration is
+ * invalid): no larger than a longer call's. Below zkp_msm_workspace_size, small MSMs take longer. */
+unsigned long long zkp_msm_workspace_least(unsigned long long len, unsigned int window, unsigned int target_windows);
+
 /* MSM over device-resident point tables (n_precompute tables of len affine
  * points, table-major) and device scalars; synchronizes `stream` and writes
  * the affine result to host h_result[16]. */

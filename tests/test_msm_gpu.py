@@ -21,6 +21,7 @@ from zkpoly_amd.msm import (
     MsmConfig,
     msm_device,
     mul_generator,
+    workspace_least,
     workspace_size,
 )
 from zkpoly_amd.runtime import GpuBuffer, Point, PointArray, ScalarArray
@@ -451,3 +452,22 @@ def test_runs_over_chunk_edges(libs, stream, n, window, heavy):
                 ss[i] = mont_limbs(1 << (window - 2))
     got = run_device(libs, stream, gpu_bases(libs, stream, ks), ss, window)
     assert list(got) == list(closed_form(ks, ss))
+
+
+@pytest.mark.parametrize("n,longer,window", [(512, 512, 5), (953, 1024, 6), (1024, 1024, 6), (2048, 2048, 8), (2400, 2500, 17)])
+def test_least_workspace(libs, stream, n, longer, window):
+    """Small MSMs with a long run in the smallest workspace, their own and a longer
+    call's: chunks are as long as its room for pieces asks."""
+    target = -(-254 // window)
+    ks, ss = random_elements(n, 61), random_elements(n, 62)
+    ss[: n // 3] = mont_limbs(5)
+    pb = gpu_bases(libs, stream, ks)
+    sb = hip.DeviceBuffer(n * 32)
+    sb.upload(ss)
+    want = list(closed_form(ks, ss))
+    for size in (workspace_least(libs, n, window, target), workspace_least(libs, longer, window, target),
+                 workspace_size(libs, n, window, target)):
+        assert list(msm_device(libs, pb.addr, sb.addr, n, window, target, hip.DeviceBuffer(size), stream)) == want
+    with pytest.raises(hip.HipError):
+        msm_device(libs, pb.addr, sb.addr, n, window, target, hip.DeviceBuffer(workspace_least(libs, n, window, target) - 1),
+                   stream)

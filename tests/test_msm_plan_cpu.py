@@ -7,13 +7,14 @@
 * plan_msm keeps every choice within the memory limit as the library's own
   sizing call counts it, trades parts / batch_per_run / precomputation for
   memory as the limit tightens, and gives up only when nothing fits.
+* A call's workspace is no larger than it was, nor than a longer call's.
 """
 import json
 import os
 
 import pytest
 
-from zkpoly_amd.msm import MSM, MsmConfig
+from zkpoly_amd.msm import MSM, MsmConfig, workspace_least, workspace_size
 from zkpoly_amd.msm_plan import Choice, model_time_us, plan_msm, reference_choice
 from zkpoly_amd.runtime import Libs
 
@@ -80,3 +81,34 @@ def test_model_counts_resident_points_across_runs():
     four = MsmConfig(window_size=16, target_window=16, batch_per_run=4)
     scalars_copy_us = (1 << 20) * 32 / (55.0 * 1e3)
     assert model_time_us(one, 1 << 20, 4) - model_time_us(four, 1 << 20, 4) == pytest.approx(3 * scalars_copy_us)
+
+
+# (points, window, target windows, bytes): workspaces that programs were told to keep before
+KEPT_WORKSPACES = [
+    (1, 8, 32, 581120), (256, 8, 32, 794624), (512, 5, 51, 835584), (953, 6, 43, 1334528), (1024, 6, 43, 1413376),
+    (2048, 8, 32, 2332160), (4096, 8, 32, 4089344), (4096, 8, 8, 3610112), (5000, 12, 11, 10302720),
+    (1 << 14, 10, 26, 15796224), (1 << 16, 12, 22, 53083392), (65537, 13, 10, 48094464), (1 << 16, 21, 13, 4486785792),
+    (1 << 18, 14, 19, 171980032), (1 << 18, 16, 4, 144057344), (1 << 19, 18, 15, 835734272), (1 << 20, 12, 22, 456903168),
+    (1 << 20, 16, 16, 511852032), (1 << 22, 16, 16, 1396862464)]
+
+
+@pytest.mark.parametrize("n,window,target,kept", KEPT_WORKSPACES)
+def test_kept_workspace_still_does(n, window, target, kept):
+    assert workspace_least(Libs(), n, window, target) <= kept
+
+
+@pytest.mark.parametrize("window,target", [(6, 43), (8, 32), (12, 11), (13, 20), (16, 16), (21, 13)])
+def test_workspace_does_for_a_shorter_call(window, target):
+    libs = Libs()
+    lens = sorted({1, 2, 3, 7, 13, 30, 100, 300, 762, 763, 953, 1280, 1281, 2048, 2400, 2475, 2476, 18604, 18605, 30000,
+                   50000, 100000, 104858, 131073, 139265, 262144, 262145, 300000, 1 << 19, 524289, 1 << 20, 1100000})
+    for query in (workspace_least, workspace_size):
+        sizes = [query(libs, n, window, target) for n in lens]
+        assert sizes == sorted(sizes)
+
+
+@pytest.mark.parametrize("window,target,kept", [(8, 32, 4250112), (13, 20, 49658112), (16, 16, 307735296)])
+def test_kept_host_buffer_still_does(window, target, kept):
+    """The drop-in call's buffer (its size does not come with the call): 5000 points, two batches a run."""
+    cfg = MsmConfig(window, target, batch_per_run=2, parts=2, stage_scalars=2, stage_points=2)
+    assert MSM(Libs(), cfg).get_buffer_size(5000)[0] <= kept

@@ -856,8 +856,13 @@ __global__ void __launch_bounds__(THREADS)
 // a workgroup join their segments in LDS as a tree, k_long_tiles leaves one
 // segment per workgroup and k_long_join joins those.  So a run of any length
 // costs (its pieces / 64 / LONG_TILES) + about 30 additions in sequence.
+// Up to LONG_TILES workgroups, one chunk a quad where that takes fewer.
 constexpr uint32_t LONG_QUADS = THREADS / 4;
 constexpr uint32_t LONG_TILES = 512;
+static inline uint32_t long_tiles_for(uint32_t chunks) {
+  const uint32_t t = (chunks + LONG_QUADS - 1) / LONG_QUADS;
+  return t < LONG_TILES ? t : LONG_TILES;
+}
 
 enum : uint32_t { SEG_EMPTY = 0, SEG_ONE = 1, SEG_SEVERAL = 2 };  // runs in a segment: none, one, more
 
@@ -956,7 +961,7 @@ __global__ void __launch_bounds__(THREADS)
   const uint32_t N = counts[0];
   const uint32_t nchunks = chunks_of(N, ch);
   const uint32_t quad = threadIdx.x >> 2, q = threadIdx.x & 3;
-  const uint32_t per = (nchunks + LONG_TILES * LONG_QUADS - 1) / (LONG_TILES * LONG_QUADS);
+  const uint32_t per = (nchunks + gridDim.x * LONG_QUADS - 1) / (gridDim.x * LONG_QUADS);
   const uint32_t lo = (blockIdx.x * LONG_QUADS + quad) * per;
   const uint32_t hi = lo + per < nchunks ? lo + per : nchunks;
   SegmentWalk w;
@@ -1016,15 +1021,15 @@ __global__ void __launch_bounds__(THREADS)
 // The tiles' segments joined (one workgroup); the last runs are closed.
 __global__ void __launch_bounds__(THREADS)
     k_long_join(const uint32_t* __restrict__ counts, const uint32_t* __restrict__ seg_meta,
-                const u32* __restrict__ seg_pts, u32* buckets) {
+                const u32* __restrict__ seg_pts, uint32_t tiles, u32* buckets) {
   if (counts[1] == 0) return;
   __shared__ SegmentLds S;
   const uint32_t quad = threadIdx.x >> 2, q = threadIdx.x & 3;
   SegmentWalk w;
-  const uint32_t per = 2 * LONG_TILES / LONG_QUADS;
+  constexpr uint32_t per = 2 * LONG_TILES / LONG_QUADS;  // a constant: the meta loads go out together
   for (uint32_t v = quad * per; v < (quad + 1) * per; v++) {
     const uint32_t b = v >> 1;
-    if (seg_meta[3 * b] > (v & 1))
+    if (b < tiles && seg_meta[3 * b] > (v & 1))
       w.piece(S, quad, q, buckets, seg_meta[3 * b + 1 + (v & 1)], Quad29::load(seg_pts + (size_t)v * 32, q));
   }
   w.finish(S, quad, q);
@@ -1286,8 +1291,12 @@ __global__ void __launch_bounds__(THREADS)
 static inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Device workspace for one MSM of `len` points (per table) and config cfg.
+// The pieces of cut runs live in the accumulation only, the sort's temporaries
+// (matrix, keys_tmp, vals_tmp, slices) before it and the reduction's levels (red)
+// after it, all on one stream, so the pieces lie over the other two.
 struct Layout {
-  size_t hist, block_sums, cursor, keys0, vals0, counts, pieces, seg_meta, seg_pts, buckets, red[4], sums, total;
+  size_t hist, block_sums, cursor, keys0, vals0, counts, pieces, seg_meta, seg_pts, buckets, red[4], sums;
+  size_t least, total;  // smallest workspace that does, and the one to ask for
   size_t matrix, keys_tmp, vals_tmp, slices;  // partition sort (when `part`)
   uint32_t max_slices;
   bool part;
@@ -1327,7 +1336,21 @@ static bool make_sort_plan(const Config& cfg, uint64_t len, SortPlan* sp) {
   return sp->tiles > 0;
 }
 
-static bool make_layout(const Config& cfg, uint64_t len, Layout* L, uint32_t sets = 1) {
+// Room for pieces beyond the sort's and the reduction's.  The least workspace of a
+// length may not grow from one version to the next (a saved plan's buffer has to
+// do), nor be smaller than a shorter length's: the first accumulation kept 10.3
+// bytes an entry for itself, and the first one with pieces, which lay apart, no
+// less than 24 MB from 2.4 M entries on.  Chunks of sixteen entries take 16 bytes
+// of pieces an entry and fit there.  The shorter ones of small MSMs, down to four
+// entries (65 bytes an entry, at most 10 240 chunks), do not where the reduction has
+// no levels, so the size asked for has room for them, and a smaller buffer gets
+// longer chunks: 2^10 points, window 8, 250 us, and 281 us in the least workspace.
+constexpr uint64_t PIECE_BYTES_PER_ENTRY = 10, PIECE_BYTES_MAX = 24000000;
+constexpr uint64_t SHORT_CHUNK_BYTES_PER_ENTRY = 68, SHORT_CHUNK_BYTES_MAX = 2750000;
+
+// The layout in `room` bytes of workspace, at least L->least, at most L->total:
+// chunks are as long as room for their pieces asks.
+static bool make_layout(const Config& cfg, uint64_t len, Layout* L, uint32_t sets, uint64_t room) {
   memset(L, 0, sizeof(*L));
   if (sets == 0) return false;
   L->sets = sets;
@@ -1343,8 +1366,6 @@ static bool make_layout(const Config& cfg, uint64_t len, Layout* L, uint32_t set
   }
   L->n_entries_max = len * cfg.actual_windows;
   if (len * cfg.n_precompute >= 0x80000000ull || L->n_entries_max >= 0xffffffffull) return false;
-  L->share = share_for(L->n_entries_max);
-  L->chunks_max = (uint32_t)((L->n_entries_max + L->share.ch - 1) / L->share.ch);
   // reduction level sizes (halving down to RED_TAIL items per window)
   uint32_t M = cfg.buckets;
   int rl = 0;
@@ -1362,6 +1383,13 @@ static bool make_layout(const Config& cfg, uint64_t len, Layout* L, uint32_t set
   L->hist = off; off = align256(off + ((size_t)L->H + 1) * 4);
   L->cursor = off; off = align256(off + ((size_t)L->H + 1) * 4);
   L->block_sums = off; off = align256(off + (size_t)(L->nb_scan > L->nb_matrix ? L->nb_scan : L->nb_matrix) * 4);
+  L->counts = off; off = align256(off + 2 * 4);
+  L->keys0 = off; off = align256(off + L->n_entries_max * 4);
+  L->vals0 = off; off = align256(off + L->n_entries_max * 4);
+  L->bucket_bytes = align256((size_t)L->H * 128);
+  L->buckets = off; off += L->bucket_bytes * sets;
+  L->sums = off; off = align256(off + (size_t)cfg.n_windows * 128);
+  const size_t shared = off;
   if (L->part) {
     L->matrix = off; off = align256(off + (size_t)L->matrix_n * 4);
     L->keys_tmp = off; off = align256(off + L->n_entries_max * 4);
@@ -1369,21 +1397,26 @@ static bool make_layout(const Config& cfg, uint64_t len, Layout* L, uint32_t set
     L->slices = off; off = align256(off + ((size_t)L->sp.nc + 1) * 4);
     L->max_slices = (uint32_t)((L->n_entries_max + SEG_SLICE - 1) / SEG_SLICE) + L->sp.nc;
   }
-  L->counts = off; off = align256(off + 2 * 4);
-  L->keys0 = off; off = align256(off + L->n_entries_max * 4);
-  L->vals0 = off; off = align256(off + L->n_entries_max * 4);
-  L->pieces = off; off = align256(off + (size_t)L->chunks_max * 2 * 128);
-  L->seg_meta = off; off = align256(off + (size_t)LONG_TILES * 3 * 4);
-  L->seg_pts = off; off = align256(off + (size_t)LONG_TILES * 2 * 128);
-  L->bucket_bytes = align256((size_t)L->H * 128);
-  L->buckets = off; off += L->bucket_bytes * sets;
   // reduction ping-pong: X and Y for even / odd levels
   L->red[0] = off; off = align256(off + (size_t)cfg.n_windows * red_max0 * 128);
   L->red[1] = off; off = align256(off + (size_t)cfg.n_windows * red_max0 * 128);
   L->red[2] = off; off = align256(off + (size_t)cfg.n_windows * (red_max1 ? red_max1 : 1) * 128);
   L->red[3] = off; off = align256(off + (size_t)cfg.n_windows * (red_max1 ? red_max1 : 1) * 128);
-  L->sums = off; off = align256(off + (size_t)cfg.n_windows * 128);
-  L->total = off;
+  const uint64_t least = PIECE_BYTES_PER_ENTRY * L->n_entries_max, full = SHORT_CHUNK_BYTES_PER_ENTRY * L->n_entries_max;
+  L->least = align256(off + (least < PIECE_BYTES_MAX ? least : PIECE_BYTES_MAX));
+  L->total = align256(off + (full < SHORT_CHUNK_BYTES_MAX ? full : SHORT_CHUNK_BYTES_MAX));
+  if (L->total < L->least) L->total = L->least;
+  if (room < L->least) return false;
+  // chunks as share_for wants them, longer where their pieces would not fit
+  L->share = share_for(L->n_entries_max);
+  for (;; L->share.ch += 4) {
+    L->chunks_max = (uint32_t)((L->n_entries_max + L->share.ch - 1) / L->share.ch);
+    const uint32_t tiles = L->chunks_max > RUN_MAX + 1 ? long_tiles_for(L->chunks_max) : 0;
+    L->pieces = shared;
+    L->seg_meta = align256(L->pieces + (L->chunks_max > 1 ? (size_t)L->chunks_max * 2 * 128 : 0));
+    L->seg_pts = align256(L->seg_meta + (size_t)tiles * 3 * 4);
+    if (L->seg_pts + (size_t)tiles * 2 * 128 <= (room < L->total ? room : L->total)) break;
+  }
   return true;
 }
 
@@ -1561,9 +1594,10 @@ static hipError_t accumulate_sorted(const Layout& L, char* ws, uint32_t set, con
     ZKP_CHECK(hipGetLastError());
   }
   if (L.chunks_max > RUN_MAX + 1) {
-    hipLaunchKernelGGL(k_long_tiles, dim3(LONG_TILES), dim3(THREADS), 0, stream, keys0, pieces, counts, ch, buckets,
+    const uint32_t tiles = long_tiles_for(L.chunks_max);
+    hipLaunchKernelGGL(k_long_tiles, dim3(tiles), dim3(THREADS), 0, stream, keys0, pieces, counts, ch, buckets,
                        seg_meta, seg_pts);
-    hipLaunchKernelGGL(k_long_join, dim3(1), dim3(THREADS), 0, stream, counts, seg_meta, seg_pts, buckets);
+    hipLaunchKernelGGL(k_long_join, dim3(1), dim3(THREADS), 0, stream, counts, seg_meta, seg_pts, tiles, buckets);
     ZKP_CHECK(hipGetLastError());
   }
   pt.mark("runs");
@@ -1690,7 +1724,7 @@ struct HostPlan {
   size_t sc_bytes;        // one scalar stage: part_len Fr elements
   Layout L;
 
-  size_t total() const { return stage_points * pts_bytes + stage_scalars * sc_bytes + L.total; }
+  size_t total() const { return stage_points * pts_bytes + stage_scalars * sc_bytes + L.least; }
 };
 
 static bool make_host_plan(const Config& cfg, uint64_t card_len, uint32_t parts, uint32_t batch_per_run,
@@ -1703,7 +1737,10 @@ static bool make_host_plan(const Config& cfg, uint64_t card_len, uint32_t parts,
   P->batch_per_run = batch_per_run;
   const bool several = P->part_len < card_len;
   P->scratch_set = several ? batch_per_run : UINT32_MAX;
-  if (!make_layout(cfg, P->part_len ? P->part_len : 1, &P->L, batch_per_run + (several ? 1 : 0))) return false;
+  // (the buffer's size does not come with the call, so the plan is for the least)
+  if (!make_layout(cfg, P->part_len ? P->part_len : 1, &P->L, batch_per_run + (several ? 1 : 0), UINT64_MAX) ||
+      !make_layout(cfg, P->part_len ? P->part_len : 1, &P->L, batch_per_run + (several ? 1 : 0), P->L.least))
+    return false;
   P->pts_bytes = align256((size_t)P->part_len * cfg.n_precompute * 64);
   P->sc_bytes = align256((size_t)P->part_len * 32);
   return true;
@@ -2038,8 +2075,19 @@ unsigned long long zkp_msm_workspace_size(unsigned long long len, unsigned int w
   Config cfg;
   if (!make_config(window, target_windows, &cfg)) return 0;
   Layout L;
-  if (!make_layout(cfg, len ? len : 1, &L)) return 0;
+  if (!make_layout(cfg, len ? len : 1, &L, 1, UINT64_MAX)) return 0;
   return L.total;
+}
+
+// The smallest workspace that zkp_msm_device accepts (0 if the configuration is
+// invalid): no larger than an earlier version's size or a longer call's.  Below
+// zkp_msm_workspace_size, small MSMs accumulate in longer chains.
+unsigned long long zkp_msm_workspace_least(unsigned long long len, unsigned int window, unsigned int target_windows) {
+  Config cfg;
+  if (!make_config(window, target_windows, &cfg)) return 0;
+  Layout L;
+  if (!make_layout(cfg, len ? len : 1, &L, 1, UINT64_MAX)) return 0;
+  return L.least;
 }
 
 // MSM with points (n_precompute tables of len affine points, table-major) and
@@ -2051,8 +2099,8 @@ hipError_t zkp_msm_device(const unsigned int* d_points, const unsigned int* d_sc
   Config cfg;
   if (!make_config(window, target_windows, &cfg)) return hipErrorInvalidValue;
   Layout L;
-  if (!make_layout(cfg, len ? len : 1, &L)) return hipErrorInvalidValue;
-  if (d_workspace == nullptr || workspace_bytes < L.total || h_result == nullptr) return hipErrorInvalidValue;
+  if (!make_layout(cfg, len ? len : 1, &L, 1, workspace_bytes)) return hipErrorInvalidValue;
+  if (d_workspace == nullptr || h_result == nullptr) return hipErrorInvalidValue;
   if (len > 0 && (d_points == nullptr || d_scalars == nullptr)) return hipErrorInvalidValue;
   G1XYZZ r;
   ZKP_CHECK(msm_device(cfg, d_points, d_scalars, len, reinterpret_cast<char*>(d_workspace), L, stream, &r,
@@ -2077,8 +2125,8 @@ hipError_t zkp_msm_device_enqueue(const unsigned int* d_points, const unsigned i
   Config cfg;
   if (!make_config(window, target_windows, &cfg)) return hipErrorInvalidValue;
   Layout L;
-  if (!make_layout(cfg, len ? len : 1, &L)) return hipErrorInvalidValue;
-  if (d_workspace == nullptr || workspace_bytes < L.total) return hipErrorInvalidValue;
+  if (!make_layout(cfg, len ? len : 1, &L, 1, workspace_bytes)) return hipErrorInvalidValue;
+  if (d_workspace == nullptr) return hipErrorInvalidValue;
   if (len > 0 && (d_points == nullptr || d_scalars == nullptr)) return hipErrorInvalidValue;
   char* ws = reinterpret_cast<char*>(d_workspace);
   PhaseTimer pt{false, stream, {}, {}};

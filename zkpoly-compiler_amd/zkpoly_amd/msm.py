@@ -81,6 +81,8 @@ def core_lib(libs: Libs) -> ctypes.CDLL:
         P = ctypes.c_void_p
         lib.zkp_msm_workspace_size.argtypes = [ctypes.c_ulonglong, ctypes.c_uint, ctypes.c_uint]
         lib.zkp_msm_workspace_size.restype = ctypes.c_ulonglong
+        lib.zkp_msm_workspace_least.argtypes = [ctypes.c_ulonglong, ctypes.c_uint, ctypes.c_uint]
+        lib.zkp_msm_workspace_least.restype = ctypes.c_ulonglong
         lib.zkp_msm_device.argtypes = [P, P, ctypes.c_ulonglong, ctypes.c_uint, ctypes.c_uint, P, ctypes.c_ulonglong,
                                        P, P, ctypes.c_int]
         lib.zkp_msm_device.restype = ctypes.c_int
@@ -161,6 +163,14 @@ class MSMPrecompute:
 
 def workspace_size(libs: Libs, length: int, window: int, target: int) -> int:
     n = core_lib(libs).zkp_msm_workspace_size(length, window, target)
+    if n == 0:
+        raise ValueError(f"invalid MSM configuration window={window} target={target} len={length}")
+    return int(n)
+
+
+def workspace_least(libs: Libs, length: int, window: int, target: int) -> int:
+    """The smallest workspace msm_device accepts; below workspace_size small MSMs take longer."""
+    n = core_lib(libs).zkp_msm_workspace_least(length, window, target)
     if n == 0:
         raise ValueError(f"invalid MSM configuration window={window} target={target} len={length}")
     return int(n)
