@@ -14,6 +14,7 @@ its own (its kernels run only inside compiled programs).
 """
 import json
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -129,6 +130,22 @@ def test_large_graph_buffer_holds_the_grid(budget, waves):
     assert int(re.search(r"return (\d+)ull; \}", src).group(1)) == table + 36 * slots * blocks * threads
 
 
+def test_running_sum_needs_no_scratch(tmp_path):
+    """The compiler must not put a sum off until it is stored and keep its terms."""
+    from zkpoly_amd import build
+
+    path = tmp_path / "tree.hip"
+    path.write_text(fused.codegen(Libs(), fused.graph_product_tree(), "tree"))
+    out = subprocess.run([build.hipcc(), *build.HIP_FLAGS, f"-I{build.CSRC}", "--cuda-device-only", "-S", str(path), "-o",
+                          str(tmp_path / "tree.s")], capture_output=True, text=True)
+    assert out.returncode == 0, out.stderr
+    text = (tmp_path / "tree.s").read_text()
+    scratch = {m.group(1): int(m.group(2)) for m in
+               re.finditer(r"\.amdhsa_kernel (\S+).*?private_segment_fixed_size (\d+)", text, re.S)}
+    (single,) = [v for k, v in scratch.items() if "tree_kernel" in k]
+    assert single == 0, scratch
+
+
 # ---------------------------------------------------------------- GPU
 
 
@@ -235,6 +252,58 @@ def test_ranges(libs, stream, coef, lens):
     if len(lens) == 1:
         arg = hip.DeviceBuffer(fused.arg_buffer_bytes(meta))
         local = hip.DeviceBuffer(k.local_bytes)
+        k.get_fn().f([GpuBuffer(arg.addr, arg.nbytes), GpuBuffer(local.addr, k.local_bytes)] + mut, [stream] + var)
+    else:
+        FusedBatch(k, [fused._ptr_of(x) for x in var], [fused._ptr_of(x) for x in mut], list(lens)).run(stream)
+    stream.sync()
+    for arr, b, w in want:
+        assert np.array_equal(gpu2cpu(arr, b), w)
+
+
+DEMO_FORMS = {"product_tree": fused.graph_product_tree()}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", DEMO_FORMS)
+@pytest.mark.parametrize("lens", [(1,), (257,), (511,), (131072 + 513,), (3, 600, 1)])
+def test_forms(libs, stream, name, lens):
+    """Kernels in limbs with spills and no table: around a workgroup, past the spill
+    slots' grid, and batched."""
+    from zkpoly_amd.batch import FusedBatch
+
+    g = json.loads(DEMO_FORMS[name])
+    V = g["g"][0]
+    meta = fused.FusedKernelMeta("fused_arith_" + name, len(g["inputs"]), len(g["outputs"]), fused.DEMO_DIR)
+    k = fused.FusedKernel(libs, meta)
+    var, mut, bufs, want = [], [], [], []
+    for q, n in enumerate(lens):
+        polys, scalars = {}, {}
+        for j, i in enumerate(g["inputs"]):
+            if V[i]["op"]["Input"]["typ"] == "Scalar":
+                scalars[i] = random_elements(1, 900 + 40 * q + j)[0]
+            else:
+                polys[i] = random_elements(n, 900 + 40 * q + j)
+                polys[i][n // 2] = 0
+        get = interpret(g, polys, scalars, n)
+        for j, i in enumerate(g["inputs"]):
+            x = polys[i] if i in polys else scalars[i].reshape(1, 4)
+            b, arr = device_array(x.shape[0])
+            if i in polys and n > 8:
+                arr.rotate(j % 7)
+            cpu2gpu(x, arr, b)
+            bufs.append(b)
+            var.append(arr if i in polys else Scalar(b.addr))
+        for o in g["outputs"]:
+            op = V[o]["op"]["Output"]
+            scalar = op["typ"] == "Scalar"
+            b, arr = device_array(1 if scalar else n)
+            bufs.append(b)
+            mut.append(Scalar(b.addr) if scalar else arr)
+            want.append((arr, b, get(op["store_node"]).reshape(-1, 4)))
+    print(f"fused form {name} lens={lens}", flush=True)
+    local = hip.DeviceBuffer(max(16, k.local_bytes))
+    if len(lens) == 1:
+        arg = hip.DeviceBuffer(fused.arg_buffer_bytes(meta))
         k.get_fn().f([GpuBuffer(arg.addr, arg.nbytes), GpuBuffer(local.addr, k.local_bytes)] + mut, [stream] + var)
     else:
         FusedBatch(k, [fused._ptr_of(x) for x in var], [fused._ptr_of(x) for x in mut], list(lens)).run(stream)

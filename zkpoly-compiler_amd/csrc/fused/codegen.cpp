@@ -743,6 +743,18 @@ struct Emitter {
     }
   }
 
+  // A sum or negation at position t that is not used before some product has been
+  // formed.  (Sums used at once fuse into v_add3.)
+  bool outlasts_product(const Alloc& A, uint64_t id, size_t t) const {
+    if (g.v[id].op == "Mul" || g.v[id].op == "Pow") return false;
+    const size_t use = std::min(A.next_use(id), elem_order.size());
+    for (size_t k = t + 1; k < use; k++) {
+      const Vertex& x = g.v[elem_order[k]];
+      if (x.kind != OpKind::Output && (x.op == "Mul" || x.op == "Pow")) return true;
+    }
+    return false;
+  }
+
   // Element code (one pass of the allocator); `ind` is the indentation.
   std::string gen_element(const char* ind_c) {
     std::ostringstream o;
@@ -818,7 +830,8 @@ struct Emitter {
       if (limbs) {
         const Val v = expr29(id, operand29(A, x.lhs, l), x.kind == OpKind::Bin ? operand29(A, x.rhs, r) : Val{});
         A.range[id] = v.r;
-        o << ind_c << "const zkp::Fr29 " << n << " = " << v.name << ";\n";
+        o << ind_c << "const zkp::Fr29 " << n << " = "
+          << (outlasts_product(A, id, t) ? "zkp::fused::pinned(" + v.name + ")" : v.name) << ";\n";
         products += x.op == "Mul" ? 1 : x.op == "Pow" ? 3 : 0;
         if (products >= BARRIER_EVERY) {
           o << ind_c << "__builtin_amdgcn_s_barrier();\n";

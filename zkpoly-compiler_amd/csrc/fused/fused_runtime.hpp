@@ -78,6 +78,17 @@ __device__ __forceinline__ Fr29 factor(Fr29 x) {
   return x;
 }
 
+// A computed value, formed where the source forms it.  Left alone the compiler puts
+// sums off until they are used and holds their operands instead: a kernel of 24
+// columns, 71 products and a running sum kept 1 380 bytes of scratch and took 395 us
+// over 2^18 elements, with this none and 176 (in words 222).
+__device__ __forceinline__ Fr29 pinned(Fr29 x) {
+  asm volatile(""
+               : "+v"(x.l[0]), "+v"(x.l[1]), "+v"(x.l[2]), "+v"(x.l[3]), "+v"(x.l[4]), "+v"(x.l[5]), "+v"(x.l[6]),
+                 "+v"(x.l[7]), "+v"(x.l[8]));
+  return x;
+}
+
 // A scalar that every lane computes with: kept on the vector unit, the scalar unit
 // has no 64-bit multiply-add.
 __device__ __forceinline__ Fr29 scalar_in(const uint32_t* p) { return factor(load_up(p)); }

@@ -278,6 +278,26 @@ def graph_ranges(coef: bool = False) -> str:
     return g.to_json()
 
 
+def graph_product_tree() -> str:
+    """24 columns: a running sum of products of products, which stays live across
+    them, and the product of the first ones, more values than stay in registers.
+
+    vars: the columns; mut_vars [sum, product].
+    """
+    g = GraphBuilder("Lagrange")
+    p = [g.input() for _ in range(24)]
+    pairs = [g.bin("Pp", "Mul", p[i], p[(i + 7) % 24]) for i in range(24)]
+    total = product = None
+    for i in range(24):
+        m = g.bin("Pp", "Mul", pairs[i], pairs[23 - i])
+        total = m if total is None else g.bin("Pp", "Add", total, m)
+    for x in pairs:
+        product = x if product is None else g.bin("Pp", "Mul", product, x)
+    g.output(total)
+    g.output(product)
+    return g.to_json()
+
+
 def demo_kernels() -> list[tuple[str, str]]:
     return [
         (graph_ab_gamma_c_minus_z(), "fused_arith_abgcz"),
@@ -288,6 +308,7 @@ def demo_kernels() -> list[tuple[str, str]]:
         (graph_pipelined_coef(), "fused_arith_pipe_coef"),
         (graph_ranges(False), "fused_arith_ranges"),
         (graph_ranges(True), "fused_arith_ranges_coef"),
+        (graph_product_tree(), "fused_arith_product_tree"),
     ]
 
 
