@@ -130,6 +130,28 @@ def test_large_graph_buffer_holds_the_grid(budget, waves):
     assert int(re.search(r"return (\d+)ull; \}", src).group(1)) == table + 36 * slots * blocks * threads
 
 
+@pytest.mark.parametrize("graph,limbs,big", [
+    (fused.graph_product_tree(), True, True),       # products, values spill
+    (fused.graph_ranges(), True, False),            # products, everything stays in registers
+], ids=["product_tree", "ranges"])
+def test_form_of_kernel(graph, limbs, big):
+    """Workgroups of 512 that meet at barriers, and table entries reduced by a pass of
+    their own, only where limbs also spill."""
+    src = fused.codegen(Libs(), graph, "form")
+    assert ("Fr29" in src) == limbs
+    assert ("s_barrier" in src) == big
+    assert ("__launch_bounds__(512)" in src) == big and ("__launch_bounds__(256)" in src) != big
+    if not big:
+        assert "reduce_entries" not in src
+    slots = re.search(r"kSpillSlots = (\d+);", src)
+    if slots:
+        blocks, threads = map(int, re.search(r"kSpillThreads = (\d+)ull \* (\d+);", src).groups())
+        assert max(int(x) for x in re.findall(r"spill_store\(spill, me, (\d+),", src)) < int(slots.group(1))
+        table = int(re.search(r"local_buffer\) \+ (\d+)", src).group(1))
+        assert int(re.search(r"return (\d+)ull; \}", src).group(1)) == (
+            table + (36 if limbs else 32) * int(slots.group(1)) * blocks * threads)
+
+
 def test_running_sum_needs_no_scratch(tmp_path):
     """The compiler must not put a sum off until it is stored and keep its terms."""
     from zkpoly_amd import build

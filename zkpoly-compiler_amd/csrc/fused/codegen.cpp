@@ -536,7 +536,13 @@ struct Emitter {
             {std::min(all.r.lo, rest.r.lo), std::max(all.r.hi, rest.r.hi), std::min(all.r.llo, rest.r.llo),
              std::max(all.r.lhi, rest.r.lhi)}};
   }
+  // as a table entry: carried limbs, and a range like an unpacked element's
+  static Val table_form(const Val& a) {
+    if (a.r.value() > 33) return reduce(a);
+    return a.r.llo < 0 || a.r.lhi > 1 ? norm(a) : a;
+  }
   const char* type() const { return limbs ? "zkp::Fr29" : "zkp::Fr"; }
+  bool reduced_entries = false;            // the element code's table is reduced below 1.0002 r
   std::map<uint64_t, Range> scalar_range;  // of the inline scalar values (limbs)
   // 4-byte words of a table entry
   size_t entry_words() const { return limbs ? 12 : 8; }
@@ -575,7 +581,7 @@ struct Emitter {
 
   // straight-line evaluation of every scalar vertex into const locals t<id>
   void emit_scalar_values(std::ostringstream& o, const std::string& vars, const std::string& mut_vars,
-                          const char* ind, const char* put = nullptr) {
+                          const char* ind, const char* table = nullptr) {
     for (uint64_t id : scalar_order) {
       const Vertex& x = g.v[id];
       if (limbs) {
@@ -585,16 +591,25 @@ struct Emitter {
         else
           v = expr29(id, {tmp(x.lhs), scalar_range.at(x.lhs)},
                      x.kind == OpKind::Bin ? Val{tmp(x.rhs), scalar_range.at(x.rhs)} : Val{});
+        if (scalar_table()) v = table_form(v);
         scalar_range[id] = v.r;
         o << ind << "const zkp::Fr29 " << tmp(id) << " = " << v.name << ";\n";
-        if (put)
-          o << ind << "zkp::fused::" << put << scalar_index.at(id) * entry_words() << ", " << tmp(id) << ");\n";
-      } else if (x.kind == OpKind::Input)
+      } else if (x.kind == OpKind::Input) {
         o << ind << "const zkp::Fr " << tmp(id) << " = zkp::Fr::load(" << src_ptr(id, vars, mut_vars) << ".ptr);\n";
-      else
+      } else {
         o << ind << "const zkp::Fr " << tmp(id) << " = "
           << expr(id, tmp(x.lhs), x.kind == OpKind::Bin ? tmp(x.rhs) : "") << ";\n";
+      }
+      if (table) emit_entry(o, ind, table, id);
     }
+  }
+  // t<id> into its place of a table
+  void emit_entry(std::ostringstream& o, const char* ind, const char* table, uint64_t id) const {
+    const std::string at = std::string(table) + " + " + std::to_string(scalar_index.at(id) * entry_words());
+    if (limbs)
+      o << ind << "zkp::fused::put_raw(" << at << ", " << tmp(id) << ");\n";
+    else
+      o << ind << tmp(id) << ".store(" << at << ");\n";
   }
 
   // ---------------------------------------------------------------- per-element schedule and registers
@@ -611,12 +626,15 @@ struct Emitter {
   // be read, which waits for the end of the element.
   size_t reg_budget = 16;     // field elements kept in registers per element
   unsigned waves_per_eu = 2;  // occupancy the register allocator must keep (0: compiler's choice)
-  // Threads of a workgroup.  A kernel in limbs is hundreds of KB of straight code:
-  // waves that drift apart fetch it one by one past the 64 KB instruction cache, so
-  // its workgroups hold two waves per SIMD and its waves meet at a barrier every
-  // BARRIER_EVERY products (about 16 KB): 620 us against 635 without, and 770 with
-  // one wave per SIMD and nearly no spills.
-  unsigned threads() const { return limbs && waves_per_eu != 1 ? 512u : 256u; }
+  // Threads of a workgroup.  A kernel in limbs that spills is hundreds of KB of
+  // straight code: waves that drift apart fetch it one by one past the 64 KB
+  // instruction cache, so its workgroups hold two waves per SIMD and its waves meet at
+  // a barrier every BARRIER_EVERY products (about 16 KB): 620 us against 635 without,
+  // and 770 with one wave per SIMD and nearly no spills.  One that keeps everything in
+  // registers is bound by the latency of a chain and keeps small workgroups (160
+  // vertices over 2^10 and 2^18 elements: 27 and 67 us, big ones 37 and 73).
+  bool big() const { return limbs && spill_slots > 0; }
+  unsigned threads() const { return big() && waves_per_eu != 1 ? 512u : 256u; }
   static constexpr unsigned BARRIER_EVERY = 8;
   // grid when spilling: the workgroups that fit 256 CUs at the kernel's occupancy
   // (four waves per SIMD when the compiler chooses)
@@ -731,7 +749,8 @@ struct Emitter {
   }
   Val operand29(const Alloc& A, uint64_t id, const std::string& text) const {
     if (!is_scalar_value(id)) return {text, A.range.at(id)};
-    return {text, scalar_table() ? reduced() : scalar_range.at(id)};
+    if (reduced_entries) return {text, reduced()};
+    return {text, scalar_range.at(id)};
   }
 
   void plan_elements() {
@@ -833,7 +852,7 @@ struct Emitter {
         o << ind_c << "const zkp::Fr29 " << n << " = "
           << (outlasts_product(A, id, t) ? "zkp::fused::pinned(" + v.name + ")" : v.name) << ";\n";
         products += x.op == "Mul" ? 1 : x.op == "Pow" ? 3 : 0;
-        if (products >= BARRIER_EVERY) {
+        if (big() && products >= BARRIER_EVERY) {
           o << ind_c << "__builtin_amdgcn_s_barrier();\n";
           products = 0;
         }
@@ -881,11 +900,13 @@ struct Emitter {
     gen_element("    ");  // the allocation: it does not depend on the arithmetic
     const bool spills = spill_slots > 0;
     limbs = table || spills;
-    if (limbs && !table) {  // ranges of the scalars that the element code will name
+    if (limbs) {  // ranges of the scalars that the element code will name
       std::ostringstream unused;
       emit_scalar_values(unused, "vars", "mut_vars", "");
     }
+    reduced_entries = table && big();
     const std::string elem_single = gen_element("    ");
+    reduced_entries = false;
     const std::string elem_batched = gen_element("    ");  // same allocation, own names
     const size_t nv = var_slot.size(), nm = g.outputs.size();
     const unsigned blocks = spill_blocks();
@@ -900,13 +921,13 @@ struct Emitter {
       o << "constexpr uint64_t kSpillThreads = " << blocks << "ull * " << threads() << ";\n"
         << "constexpr uint64_t kSpillSlots = " << spill_slots << ";\n\n";
     if (table) {
-      // one wave, all lanes alike; each then reduces its share of the entries
+      // one wave, all lanes alike
       o << "__global__ void __launch_bounds__(64) " << name
         << "_scalars_kernel(const ConstPolyPtr* __restrict__ vars, const PolyPtr* __restrict__ mut_vars, "
            "uint32_t* __restrict__ table) {\n";
-      emit_scalar_values(o, "vars", "mut_vars", "  ", "put_raw(table + ");
+      emit_scalar_values(o, "vars", "mut_vars", "  ", "table");
       emit_scalar_outputs(o, "mut_vars", "  ", "if (threadIdx.x == 0) ");
-      o << "  zkp::fused::reduce_entries(table, " << scalar_order.size() << ");\n";
+      if (big()) o << "  zkp::fused::reduce_entries(table, " << scalar_order.size() << ");\n";
       o << "}\n\n";
     }
     // the occupancy the register budget was chosen for binds only kernels that spill; a small kernel keeps
@@ -962,8 +983,7 @@ struct Emitter {
     if (table) {
       // no table per instance: the element code reads scalars from one; give it a local copy
       o << "    uint32_t scalars_buf[" << scalar_order.size() * entry_words() << "];\n";
-      for (uint64_t id : scalar_order)
-        o << "    zkp::fused::put_entry(scalars_buf + " << scalar_index.at(id) * entry_words() << ", " << tmp(id) << ");\n";
+      for (uint64_t id : scalar_order) emit_entry(o, "    ", "scalars_buf", id);
       o << "    const uint32_t* scalars = scalars_buf;\n";
     }
     o << elem_batched;

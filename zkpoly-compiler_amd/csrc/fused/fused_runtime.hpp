@@ -150,16 +150,10 @@ __device__ __forceinline__ void store_down(const Fr29& x, const PolyView& v, uin
   if (live) y.store(element(v, idx, anchor));
 }
 
-// Entry of the scalar table: nine limbs in 12 words, as computed (put_raw), then
-// below 1.0002 r.
+// Entry of the scalar table: nine limbs in 12 words, as computed (put_raw).
 __device__ __forceinline__ void put_raw(uint32_t* p, const Fr29& x) {
 #pragma unroll
   for (int i = 0; i < 9; i++) p[i] = (u32)x.l[i];
-}
-__device__ __forceinline__ void put_entry(uint32_t* p, const Fr29& x) {
-  const Fr29 y = x.reduce();
-#pragma unroll
-  for (int i = 0; i < 9; i++) p[i] = (u32)y.l[i];
 }
 __device__ __forceinline__ Fr29 entry(const uint32_t* p) {
   Fr29 x;
@@ -168,11 +162,11 @@ __device__ __forceinline__ Fr29 entry(const uint32_t* p) {
   return x;
 }
 
-// The table's entries reduced, by one workgroup that has written them.
+// The table's entries below 1.0002 r, by one workgroup that has written them.
 __device__ __forceinline__ void reduce_entries(uint32_t* table, unsigned count) {
   __threadfence();
   __syncthreads();
-  for (unsigned t = threadIdx.x; t < count; t += blockDim.x) put_entry(table + 12 * t, entry(table + 12 * t));
+  for (unsigned t = threadIdx.x; t < count; t += blockDim.x) put_raw(table + 12 * t, entry(table + 12 * t).reduce());
 }
 
 // largest k < n with prefix[k] <= g (prefix has n + 1 non-decreasing entries)
