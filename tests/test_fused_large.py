@@ -133,10 +133,13 @@ def test_large_graph_buffer_holds_the_grid(budget, waves):
 @pytest.mark.parametrize("graph,limbs,big", [
     (fused.graph_product_tree(), True, True),       # products, values spill
     (fused.graph_ranges(), True, False),            # products, everything stays in registers
-], ids=["product_tree", "ranges"])
+    (fused.graph_scaled_columns(), False, False),   # a product a column
+    (fused.graph_column_sums(), False, False),      # sums, some spill
+], ids=["product_tree", "ranges", "scaled_columns", "column_sums"])
 def test_form_of_kernel(graph, limbs, big):
-    """Workgroups of 512 that meet at barriers, and table entries reduced by a pass of
-    their own, only where limbs also spill."""
+    """29-bit limbs where products outweigh the columns' conversion; workgroups of 512
+    that meet at barriers, and table entries reduced by a pass of their own, only where
+    limbs also spill."""
     src = fused.codegen(Libs(), graph, "form")
     assert ("Fr29" in src) == limbs
     assert ("s_barrier" in src) == big
@@ -282,15 +285,16 @@ def test_ranges(libs, stream, coef, lens):
         assert np.array_equal(gpu2cpu(arr, b), w)
 
 
-DEMO_FORMS = {"product_tree": fused.graph_product_tree()}
+DEMO_FORMS = {"product_tree": fused.graph_product_tree(), "scaled_columns": fused.graph_scaled_columns(False),
+              "scaled_columns_coef": fused.graph_scaled_columns(True), "column_sums": fused.graph_column_sums()}
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", DEMO_FORMS)
 @pytest.mark.parametrize("lens", [(1,), (257,), (511,), (131072 + 513,), (3, 600, 1)])
 def test_forms(libs, stream, name, lens):
-    """Kernels in limbs with spills and no table: around a workgroup, past the spill
-    slots' grid, and batched."""
+    """Kernels in limbs with spills and no table, in words with a table, and in words
+    with spills: around a workgroup, past the spill slots' grid, and batched."""
     from zkpoly_amd.batch import FusedBatch
 
     g = json.loads(DEMO_FORMS[name])

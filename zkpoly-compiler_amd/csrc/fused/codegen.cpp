@@ -17,8 +17,9 @@
 // common/src/arith.rs:411-452).  Scalars are 1-element views.  Semantics per
 // operation follow kernel_gen.rs:457-566, including the coefficient-form rule
 // for scalar-polynomial add/sub (only element 0 of the first chunk sees the
-// scalar).  Register allocation is left to the compiler: the straight-line body
-// needs no explicit spill buffer, so local_buffer is accepted and unused.
+// scalar).  local_buffer holds the table of the graph's scalar values and the spill
+// slots of the per-element values that the generator does not keep in registers;
+// <name>_local_buffer_bytes gives its size, 0 for small graphs.
 //
 // Each library also exports <name>_batched, which runs the same expression over
 // several independent instances of different lengths in one launch.
@@ -544,8 +545,9 @@ struct Emitter {
   const char* type() const { return limbs ? "zkp::Fr29" : "zkp::Fr"; }
   bool reduced_entries = false;            // the element code's table is reduced below 1.0002 r
   std::map<uint64_t, Range> scalar_range;  // of the inline scalar values (limbs)
-  // 4-byte words of a table entry
+  // 4-byte words of a table entry, bytes of a spill slot
   size_t entry_words() const { return limbs ? 12 : 8; }
+  uint64_t slot_bytes() const { return limbs ? 36 : 32; }
 
   std::string src_ptr(uint64_t id, const std::string& vars, const std::string& mut_vars) const {
     auto it = var_slot.find(id);
@@ -721,7 +723,7 @@ struct Emitter {
           o << "zkp::Fr::load(v" << id << ".elem(idx));\n";
         range[id] = loaded();
       } else {
-        o << "zkp::fused::spill_load(spill, me, " << slot.at(id) << ", kSpillSlots, kSpillThreads);\n";
+        o << "zkp::fused::spill_load<" << e.type() << ">(spill, me, " << slot.at(id) << ", kSpillSlots, kSpillThreads);\n";
       }
       reg[id] = n;
       return n;
@@ -760,6 +762,36 @@ struct Emitter {
       if ((x.kind == OpKind::Bin || x.kind == OpKind::Unr) && is_poly(id)) elem_order.push_back(id);
       if (x.kind == OpKind::Output && !x.scalar) elem_order.push_back(id);
     }
+  }
+
+  // Whether an element's products and sums gain more in limbs than unpacking the
+  // columns read and packing those written costs, in SIMD cycles per wave: a product
+  // 910 against 1 190, a sum about 60 with the carrying that sums ask for against 90,
+  // 46 to unpack, about 330 to reduce and pack.  Measured over 2^18 elements, limbs
+  // against words: one column plus five scalars 6.7 and 6.4 us, eight columns scaled
+  // 32.2 and 32.0, eight outputs s p + q 39.1 and 38.1; eight outputs s p + t q 49.4
+  // and 52.3, five scaled columns added up 15.4 and 17.6.  16 instances of 2^12 in one
+  // call: 64 sums of 24 columns 46 and 24 us, eight columns scaled 14.7 and 13.7, eight
+  // outputs s p + t q 21.0 and 22.5.
+  bool limbs_pay() const {
+    double gain = 0;
+    std::set<uint64_t> read;
+    for (uint64_t id : elem_order) {
+      const Vertex& x = g.v[id];
+      if (x.kind == OpKind::Output) {
+        gain -= 330;
+        continue;
+      }
+      gain += x.op == "Mul" ? 280 : x.op == "Pow" ? 280 * pow_products(x.pow) : 30;
+      for (uint64_t c : {x.lhs, x.kind == OpKind::Bin ? x.rhs : x.lhs})
+        if (g.v[c].kind == OpKind::Input && is_poly(c)) read.insert(c);
+    }
+    return gain > 46.0 * read.size();
+  }
+  static int pow_products(uint64_t e) {  // of square and multiply
+    int n = 0;
+    for (; e > 1; e >>= 1) n += 1 + (int)(e & 1);
+    return n;
   }
 
   // A sum or negation at position t that is not used before some product has been
@@ -899,7 +931,7 @@ struct Emitter {
     const bool table = scalar_table();
     gen_element("    ");  // the allocation: it does not depend on the arithmetic
     const bool spills = spill_slots > 0;
-    limbs = table || spills;
+    limbs = (table || spills) && limbs_pay();
     if (limbs) {  // ranges of the scalars that the element code will name
       std::ostringstream unused;
       emit_scalar_values(unused, "vars", "mut_vars", "");
@@ -910,7 +942,7 @@ struct Emitter {
     const std::string elem_batched = gen_element("    ");  // same allocation, own names
     const size_t nv = var_slot.size(), nm = g.outputs.size();
     const unsigned blocks = spill_blocks();
-    const size_t local_bytes = table_bytes() + (spills ? spill_slots * 36ull * blocks * threads() : 0);
+    const size_t local_bytes = table_bytes() + (spills ? spill_slots * slot_bytes() * blocks * threads() : 0);
     std::ostringstream o;
     o << "// Generated fused elementwise kernel " << name << " (" << order.size() << " vertices, "
       << (g.coef ? "coefficient" : "Lagrange") << " form; " << scalar_order.size() << " scalar values"

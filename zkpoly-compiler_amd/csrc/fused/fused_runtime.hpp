@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../common/poly_ptr.hpp"
 #include "../field/bn254.hpp"
 #include "../field/fr29.hpp"
@@ -27,9 +29,10 @@ inline unsigned grid_capped(uint64_t n, unsigned threads, unsigned cap) {
   return (unsigned)(g < cap ? (g ? g : 1) : cap);
 }
 
-// Spill slots of generated kernels: slot s of a thread is two 16-byte planes and,
-// behind those of all slots, one of 4 bytes, each lane-contiguous over the `threads`
-// threads of the kernel's capped grid, so a wave's spill or reload is coalesced.
+// Spill slots of generated kernels: slot s of a thread is two 16-byte planes and, in
+// limbs, behind those of all slots, one of 4 bytes, each lane-contiguous over the
+// `threads` threads of the kernel's capped grid, so a wave's spill or reload is
+// coalesced.
 // `me` is the thread's global index.  A plane's start is the same on all lanes and
 // stays on the scalar unit, hidden from the compiler, which otherwise forms every
 // plane's lane address before the loop and keeps them all in scratch.
@@ -43,10 +46,23 @@ __device__ __forceinline__ void spill_store(char* spill, uint32_t me, uint64_t s
   spill_at<uint4>(spill, (32 * s + 16) * threads, me) = make_uint4((u32)x.l[4], (u32)x.l[5], (u32)x.l[6], (u32)x.l[7]);
   spill_at<int32_t>(spill, (32 * slots + 4 * s) * threads, me) = x.l[8];
 }
-__device__ __forceinline__ Fr29 spill_load(char* spill, uint32_t me, uint64_t s, uint64_t slots, uint64_t threads) {
-  const uint4 a = spill_at<uint4>(spill, 32 * s * threads, me), b = spill_at<uint4>(spill, (32 * s + 16) * threads, me);
-  return Fr29{{(int32_t)a.x, (int32_t)a.y, (int32_t)a.z, (int32_t)a.w, (int32_t)b.x, (int32_t)b.y, (int32_t)b.z,
-               (int32_t)b.w, spill_at<int32_t>(spill, (32 * slots + 4 * s) * threads, me)}};
+// In words the planes' addresses are left to the compiler.
+__device__ __forceinline__ void spill_store(char* spill, uint32_t me, uint64_t s, uint64_t, uint64_t threads, const Fr& x) {
+  uint4* p = reinterpret_cast<uint4*>(spill) + me;
+  p[2 * s * threads] = make_uint4(x.v[0], x.v[1], x.v[2], x.v[3]);
+  p[(2 * s + 1) * threads] = make_uint4(x.v[4], x.v[5], x.v[6], x.v[7]);
+}
+template <class T>
+__device__ __forceinline__ T spill_load(char* spill, uint32_t me, uint64_t s, uint64_t slots, uint64_t threads) {
+  if constexpr (std::is_same<T, Fr>::value) {
+    const uint4* p = reinterpret_cast<const uint4*>(spill) + me;
+    const uint4 a = p[2 * s * threads], b = p[(2 * s + 1) * threads];
+    return Fr{{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
+  } else {
+    const uint4 a = spill_at<uint4>(spill, 32 * s * threads, me), b = spill_at<uint4>(spill, (32 * s + 16) * threads, me);
+    return Fr29{{(int32_t)a.x, (int32_t)a.y, (int32_t)a.z, (int32_t)a.w, (int32_t)b.x, (int32_t)b.y, (int32_t)b.z,
+                 (int32_t)b.w, spill_at<int32_t>(spill, (32 * slots + 4 * s) * threads, me)}};
+  }
 }
 
 // ---------------------------------------------------------------- kernels in 29-bit limbs

@@ -271,6 +271,10 @@ def graph_ranges(coef: bool = False) -> str:
     for e in (0, 1, 2, 3, 5, 64):
         outs.append(g.pow(down, e))
     outs.append(g.bin("Pp", "Mul", g.neg(up), g.bin("Pp", "Sub", outs[-1], g.bin("Pp", "Add", up, wide))))
+    chain = down
+    for k in range(16):  # products of sums of products
+        chain = g.bin("Pp", "Mul", g.bin("Pp", "Sub", chain, wide) if k % 2 else chain, g.bin("Sp", "SubBy", s[k % 5], chain))
+    outs.append(chain)
     for o in outs:
         g.output(o)
     g.output(total, scalar=True)
@@ -298,6 +302,30 @@ def graph_product_tree() -> str:
     return g.to_json()
 
 
+def graph_scaled_columns(coef: bool = False) -> str:
+    """Few products to many columns: vars [p0 .. p5, s0 .. s5]; mut_vars s_j p_j and, for
+    odd j, s_j p_j + s_0, then the scalar s_0 s_1 - s_2."""
+    g = GraphBuilder("Coef" if coef else "Lagrange")
+    p = [g.input() for _ in range(6)]
+    s = [g.input(scalar=True) for _ in range(6)]
+    for j in range(6):
+        x = g.bin("Sp", "Mul", s[j], p[j])
+        g.output(g.bin("Sp", "Add", s[0], x) if j % 2 else x)
+    g.output(g.bin("Ss", "Sub", g.bin("Ss", "Mul", s[0], s[1]), s[2]), scalar=True)
+    return g.to_json()
+
+
+def graph_column_sums() -> str:
+    """Sums only, more than stay in registers: vars: 24 columns; mut_vars: 8 outputs."""
+    g = GraphBuilder("Lagrange")
+    p = [g.input() for _ in range(24)]
+    s = [g.bin("Pp", "Add", p[i], p[(i + 1) % 24]) for i in range(24)]
+    t = [g.bin("Pp", "Sub", s[i], s[(i + 11) % 24]) for i in range(24)]
+    for j in range(8):
+        g.output(g.bin("Pp", "Add", g.bin("Pp", "Add", t[j], t[(j + 9) % 24]), t[(j + 16) % 24]))
+    return g.to_json()
+
+
 def demo_kernels() -> list[tuple[str, str]]:
     return [
         (graph_ab_gamma_c_minus_z(), "fused_arith_abgcz"),
@@ -309,6 +337,9 @@ def demo_kernels() -> list[tuple[str, str]]:
         (graph_ranges(False), "fused_arith_ranges"),
         (graph_ranges(True), "fused_arith_ranges_coef"),
         (graph_product_tree(), "fused_arith_product_tree"),
+        (graph_scaled_columns(False), "fused_arith_scaled_columns"),
+        (graph_scaled_columns(True), "fused_arith_scaled_columns_coef"),
+        (graph_column_sums(), "fused_arith_column_sums"),
     ]
 
 
