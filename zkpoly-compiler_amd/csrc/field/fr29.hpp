@@ -185,12 +185,14 @@ struct Fr29 {
 // is 0 mod r.  With c = INV_PLAIN it maps x 2^256 to x^-1 2^256, with INV_UP an up value of x
 // to x^-1 2^256.
 //
-// Bernstein and Yang's division steps (Fast constant-time gcd computation and
-// modular inversion, 2019), in variable time: f = r, g = x, f odd; while g is
-// even it is halved; else with delta > 0 (f, g) becomes (g, -f), and g + w f
-// clears as many bits of g as delta allows.  29 steps at a time are taken on the
-// low words and collected in a matrix that is then applied to f and g (exactly
-// divisible by 2^29) and, mod r, to d and e with d x = f, e x = g (mod r).
+// By the division steps of Bernstein and Yang (Fast constant-time gcd computation
+// and modular inversion, 2019, definition 8.1), with f = r, g = x and delta = 1: f is
+// odd, and a step takes
+//   (delta, f, g) to (1 - delta, g, (g - f) / 2) if delta > 0 and g is odd,
+//                    (1 + delta, f, (g + (g mod 2) f) / 2) otherwise.
+// 29 steps at a time are taken on the low words and collected in a matrix that is
+// then applied to f and g (exactly divisible by 2^29) and, mod r, to d and e with
+// d x = f, e x = g (mod r).
 // A batch changes |d| and |e| by at most r, so limb 8 stays below 2^28 for the at
 // most 26 batches (754 steps; the paper bounds 256-bit inputs by 741).
 struct Fr29Inverse {
@@ -203,35 +205,50 @@ struct Fr29Inverse {
 
   int32_t u, v, q, r;  // 2^29 (f', g') = [u v; q r] (f, g)
 
-  // 29 division steps on the low 32 bits of f (odd) and g
+  // 29 division steps on the low 32 bits of f (odd) and g: after k of them 32 - k
+  // bits of g are still right.  The matrix is kept times 2^k, so that steps which
+  // shift g down shift f's row up.  Steps that do the same are taken together:
+  //  * those that find g even halve it and count;
+  //  * with g odd and delta > 0 f and g change places: written as (f, g) = (g, -f)
+  //    with delta = -delta, what is left of that step is one of the third kind;
+  //  * with delta <= 0 the next 1 - delta steps keep f, and k of them take g to
+  //    (g + w f) / 2^k, the w < 2^k that makes the sum divisible.  The square of an
+  //    odd number is 1 mod 8, so w = -g f mod 2^k up to k = 3.
+  // The shift by k is left to the next round, which finds those zeros.  (Gathering
+  // variable-time steps so is public practice, in libsecp256k1 with up to six of the
+  // last kind; most rounds exchange, and few have more than three of them.)
   ZKP_HD void steps(u32 f, u32 g, int32_t& delta) {
-    u32 a = 1, b = 0, c = 0, d = 1;
-    int left = 29;
-    for (;;) {
-      const int z = __builtin_ctz(g | (1u << left));
-      g >>= z;
-      a <<= z;
-      b <<= z;
-      delta += z;
-      left -= z;
+    u32 fu = 1, fv = 0, gu = 0, gv = 1;  // 2^k f' = fu f + fv g, 2^k g' = gu f + gv g
+    for (u32 left = 29;;) {
+      const u32 zeros = (u32)__builtin_ffs((int)g) - 1;  // all ones for g = 0
+      const u32 k = zeros < left ? zeros : left;
+      g >>= k;
+      fu <<= k;
+      fv <<= k;
+      delta += (int32_t)k;
+      left -= k;
       if (left == 0) break;
       if (delta > 0) {
+        const u32 f0 = f, u0 = fu, v0 = fv;
+        f = g;
+        fu = gu;
+        fv = gv;
+        g = 0u - f0;
+        gu = 0u - u0;
+        gv = 0u - v0;
         delta = -delta;
-        u32 t = f; f = g; g = 0u - t;
-        t = a; a = c; c = 0u - t;
-        t = b; b = d; d = 0u - t;
       }
-      // f f (f f - 2) = (f f - 1)^2 - 1 = -1 mod 64: w f = -g mod 2^min(k, left)
-      const int k = 1 - delta < 6 ? 1 - delta : 6;
-      const u32 w = (g * f * (f * f - 2)) & ((1u << k) - 1) & ((1u << left) - 1);
+      // k = min(3, 1 - delta, left), as a mask; delta <= 0 here
+      const u32 mask = (delta < -1 ? 7u : delta < 0 ? 3u : 1u) & ~(~0u << left);
+      const u32 w = (0u - g * f) & mask;
       g += w * f;
-      c += w * a;
-      d += w * b;
+      gu += w * fu;
+      gv += w * fv;
     }
-    u = (int32_t)a;
-    v = (int32_t)b;
-    q = (int32_t)c;
-    r = (int32_t)d;
+    u = (int32_t)fu;
+    v = (int32_t)fv;
+    q = (int32_t)gu;
+    r = (int32_t)gv;
   }
 
   // (a x + b y) / 2^29: exact with mod = 0, mod r with mod = MASK
@@ -256,7 +273,7 @@ struct Fr29Inverse {
   // On the device the lanes of a wave work together (all of them call, with the
   // same x): the steps run on the scalar unit, and lanes 0..3 of every quad form f,
   // g, d and e, each from the pair (p, q) = (f, g) or (d, e) that it keeps a copy
-  // of.  12 us as a launch of one wave.  (With all of it on one lane of the vector
+  // of.  13 us as a launch of one wave.  (With all of it on one lane of the vector
   // unit the batched inversion took 119 us where it took 92 with this.)
   ZKP_HD static Fr29 inverse(const Fr29& x, const int32_t (&c)[9]) {
     Fr29 w;
