@@ -434,9 +434,9 @@ def test_all_scalars_equal(libs, stream, value):
     (5000, 13, [2500, 2500]),
 ])
 def test_runs_over_chunk_edges(libs, stream, n, window, heavy):
-    """Small scalars 1, 2, ... with the given multiplicities (the rest uniform):
-    bucket v of window 0 is a run of exactly that many sorted entries, plus what
-    the uniform scalars add to it."""
+    """Small scalars 1, 2, ... with the given multiplicities, the rest uniform but for
+    window 0's digits of that size: bucket v of window 0 is a run of exactly that many
+    sorted entries, and begins where the smaller ones end."""
     ks = random_elements(n, 91)
     ss = random_elements(n, 92)
     at = 0
@@ -445,11 +445,17 @@ def test_runs_over_chunk_edges(libs, stream, n, window, heavy):
         at += count
     perm = np.random.Generator(np.random.PCG64(93)).permutation(n)
     ss = np.ascontiguousarray(ss[perm])
-    if at < n:  # the runs' lengths stay exact: the uniform scalars keep out of window 0's small buckets
-        small = [i for i, x in enumerate(array_to_ints(ss)) if 0 < from_mont(x) % (1 << window) <= len(heavy) + 1]
-        for i in small:
-            if from_mont(array_to_ints(ss[i:i + 1])[0]) > len(heavy):
-                ss[i] = mont_limbs(1 << (window - 2))
+    values = [from_mont(x) for x in array_to_ints(ss)]
+
+    def bucket(x):  # |digit| of window 0
+        return min(x % (1 << window), -x % (1 << window))
+
+    for i, x in enumerate(values):
+        if x > len(heavy) and 0 < bucket(x) <= len(heavy) + 1:
+            values[i] = 1 << (window - 2)
+            ss[i] = mont_limbs(values[i])
+    sizes = np.bincount([bucket(x) for x in values], minlength=len(heavy) + 2)
+    assert list(sizes[1:len(heavy) + 2]) == heavy + [0]
     got = run_device(libs, stream, gpu_bases(libs, stream, ks), ss, window)
     assert list(got) == list(closed_form(ks, ss))
 
