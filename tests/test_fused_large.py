@@ -6,7 +6,7 @@ the oracle's field operations.
 
 The generated kernels hold at most a fixed number of field elements in
 registers per element and spill the rest to local_buffer, and keep the
-graph's many scalar values in a table that a one-thread prologue fills, so
+graph's many scalar values in a table that a one-wave prologue fills, so
 these graphs run with several waves per SIMD and no compiler scratch; the
 CPU tests check the generator's plan for them (spill slots, table, buffer
 size), the GPU tests the results.  The reference has no fused-kernel test of

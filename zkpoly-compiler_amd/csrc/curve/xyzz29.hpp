@@ -75,19 +75,6 @@ struct G1X29 {
     zz.store(p + 16);
     zzz.store(p + 24);
   }
-  // The four coordinates as canonical x 2^256: G1XYZZ's layout and form.
-  __device__ __forceinline__ void store_mont256(u32* p) const {
-    const Fq29* c[4] = {&x, &y, &zz, &zzz};
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      u32 w[8];
-      c[k]->to_mont256(w);
-      uint4* q = reinterpret_cast<uint4*>(p + 8 * k);
-      q[0] = make_uint4(w[0], w[1], w[2], w[3]);
-      q[1] = make_uint4(w[4], w[5], w[6], w[7]);
-    }
-  }
-
   // dbl-2008-s-1
   ZKP_HD G1X29 dbl() const {
     if (is_identity()) return *this;

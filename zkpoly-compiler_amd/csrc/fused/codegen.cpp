@@ -562,7 +562,7 @@ struct Emitter {
   // element loop and held in registers.  Many of them (a compiler's fused
   // graph carries dozens) would stay live across the loop and crowd out the
   // per-element values, so above SCALAR_REGS the single-instance entry point
-  // computes them once in a one-thread prologue kernel into a table at the
+  // computes them once in a one-wave prologue kernel into a table at the
   // head of local_buffer, which the element loop reads at each use (uniform
   // addresses: scalar loads); scalar outputs are stored by that prologue,
   // after every scalar input has been read.

@@ -728,8 +728,8 @@ __device__ __forceinline__ uint32_t chunks_of(uint32_t entries, uint32_t ch) {
 // Nothing else is written: which slots hold a piece follows from the keys at
 // the chunk edges.
 // 109 VGPRs let four waves share a SIMD, which covers the dependent loads of an
-// entry (key, point index, point): 2^20 points at window 16 take 1.32 ms, 83 %
-// of the VALU's issue; 1.43 ms with the doubling inlined a second time (three waves).
+// entry (key, point index, point): 2^20 points at window 16 take 1.27 ms, 88 %
+// VALUBusy; with the doubling inlined a second time (three waves) it was 8 % more.
 template <bool QUAD>
 __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3)))
     k_accumulate(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,

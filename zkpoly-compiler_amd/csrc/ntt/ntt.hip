@@ -515,7 +515,6 @@ __device__ __forceinline__ void head_store(const HeadLds& L, const PolyView& v, 
 
 // One tile pair {M, rev M} per workgroup.  The caller has written L.r
 // (visible after the first barrier below).
-// (256 threads.)
 template <int NT>
 __device__ __forceinline__ void head_tile(HeadLds& L, const PolyView& v, uint32_t log_n, uint32_t t, uint64_t M) {
   const uint32_t mbits = log_n - 2 * t;
@@ -657,7 +656,7 @@ __global__ void __launch_bounds__(HEAD_THREADS)
 // ---------------------------------------------------------------- radix-4 pass
 //
 // Same tile geometry as dit_tile (2^d rows x 2^c_log columns); the stages run
-// two at a time (pass_stages).
+// two at a time (dit_tile_r4).
 __device__ __forceinline__ uint64_t tile_index(uint64_t base, uint64_t cstride, uint64_t kstride, uint32_t c,
                                                uint32_t k) {
   return base + c * cstride + (uint64_t)k * kstride;
@@ -1321,9 +1320,10 @@ int zkp_ntt_set_variant(int variant) {
   return zkp::ntt::g_variant.exchange(variant);
 }
 
-// Tuning of transforms of 2^log_n (variant 0): every pass reads runs of at
-// least 2^min_col_log adjacent elements, so a smaller value means fewer,
-// deeper passes.  Returns 0, or -1 when out of range.  No counterpart in the
+// Tuning of transforms of 2^log_n (variant 0): passes are planned for runs of at
+// least 2^min_col_log adjacent elements, so a smaller value means fewer, deeper
+// passes.  (A transform on its own with fewer tiles than CUs then takes narrower
+// ones, down to runs of four.)  Returns 0, or -1 when out of range.  No counterpart in the
 // reference ABI (autotuner hook).
 int zkp_ntt_set_tuning(unsigned int log_n, unsigned int min_col_log) {
   if (log_n > 40 || min_col_log > (unsigned)zkp::ntt::TILE_LOG - 1) return -1;

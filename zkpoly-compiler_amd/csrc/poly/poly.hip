@@ -263,9 +263,9 @@ __device__ __forceinline__ Fr29 horner_waves(const WaveLds& L, Fr29 s, const Fr2
 }
 
 // total[b] = the fold of share b, of `rounds` (a power of two) times TH * PER
-// positions; *power = x^len.  With keep_last the last share's total, which nobody
-// reads, leaves its place to *power.  With res (a single share) the fold is the
-// result and goes there.
+// positions; *power = x^len.  Without last_total the last share's total, which
+// nobody reads, is not written and its place may be *power's.  With res (a single
+// share) the fold is the result and goes there.
 template <int PER>
 __global__ void __launch_bounds__(TH)
     k_horner_fold(PolyView v, const uint32_t* x, uint64_t n, uint64_t npad, uint32_t rounds,
@@ -387,11 +387,11 @@ __global__ void __launch_bounds__(TH)
 // its own: one launch, and no tile waits for another.  One of the four waves inverts
 // the tile's product while the others form, per thread, the product of all other
 // threads' elements; which one goes by the tile, so that tiles on one CU use
-// different SIMDs.  (A fifth wave for it left one workgroup to a CU: two of five
-// waves do not fit three to a SIMD.)  2^20 elements: 68 us, bound by products (three an
-// element, 15 a thread, and the inversion with every wave of the chip waiting for
-// it), where a fold, one workgroup with one inversion on one lane and a rescan took
-// 26 + 127 + 75.
+// different SIMDs.  The tables of 55 KB leave two workgroups to a CU, two waves to a
+// SIMD.  (A fifth wave for the inversion measured 92 to 119 us: one workgroup to a CU.)
+// 2^20 elements: 60 us, bound by products (three an element, 15 a thread, and the
+// inversion with every wave of the chip waiting for it), where a fold, one workgroup
+// with one inversion on one lane and a rescan took 216.
 constexpr int INV_PER = 8;
 constexpr int INV_TILE = TH * INV_PER;
 
@@ -419,7 +419,7 @@ struct InvertLds {
   }
 };
 
-__global__ void __launch_bounds__(TH, 3) k_invert(PolyView v, uint64_t n) {
+__global__ void __launch_bounds__(TH) k_invert(PolyView v, uint64_t n) {
   __shared__ InvertLds L;
   const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const uint64_t k0 = (uint64_t)blockIdx.x * INV_TILE + (uint64_t)threadIdx.x * INV_PER;
@@ -455,7 +455,7 @@ __global__ void __launch_bounds__(TH, 3) k_invert(PolyView v, uint64_t n) {
   for (uint32_t l = 1; l < 6; l++) others = Fr29::mul(others, L.get(l, threadIdx.x ^ (1u << l)));
   for (uint32_t w = 1; w < TH / 64; w++) others = Fr29::mul(others, L.wave.get((wave + w) % (TH / 64)));
   __syncthreads();
-  // read again, an element ahead: 64 registers less than held from the first time
+  // read again, an element ahead, instead of held in 64 registers from the first time
   Fr x = element(INV_PER - 1);
   Fr29 inv = Fr29::mul(L.wave.get(TH / 64), others);  // of the thread's own product
   each<INV_PER>([&](auto i) {
@@ -540,7 +540,8 @@ static void launch_horner_fold(const Shares& s, const PolyView& v, const uint32_
 static size_t invert_part_bytes(uint64_t n) { return align256(tiles_of(n ? n : 1) * sizeof(Fr)); }
 
 // What batched_invert asks its caller for: three products a tile and one element.
-// Its kernel keeps them in LDS now; the size stays what callers' plans hold.
+// Its kernel keeps them in LDS and reads none of it; the size stays what callers' plans
+// and the runtime's checks hold.
 static size_t invert_temp_bytes(uint64_t n) { return 3 * invert_part_bytes(n) + align256(sizeof(Fr)); }
 
 static hipError_t invert_launch(const PolyView& v, hipStream_t stream) {
@@ -553,7 +554,8 @@ static hipError_t invert_launch(const PolyView& v, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// The longest polynomial zkp_batched_invert_noalloc takes.
+// The longest polynomial zkp_batched_invert_noalloc takes: what its interface has
+// always refused stays refused, though no scratch array sets the limit any more.
 #define ZKP_INVERT_NOALLOC_MAX_LEN (1ull << 26)
 
 extern "C" {
